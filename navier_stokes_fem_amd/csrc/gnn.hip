@@ -211,29 +211,64 @@ __global__ __launch_bounds__(kRB) void k_loss(int n, const double *__restrict__ 
     block_partial<1>(v, part);
 }
 
-// dh3 = dy w4 (FP32), dz3 = bf16(dh3 [z3 > 0]); partials of h3 dy and dy
+// dh3 = dy w4 (FP32), dz3 = bf16(dh3 [z3 > 0]); partials of h3 dy and dy.
+// Bound by the loads of h3 and z3: 8 lanes a node, 4 features each (8-byte
+// and 16-byte loads), a block striding over the nodes and summing its
+// partials in registers, so that the lanes are added once a block.  One
+// thread a node (2-byte loads and 33 sums over the wave per 64 nodes) took
+// 34 us on the 65,656 nodes of the 512 x 128 channel; this takes 5.9.
 __global__ __launch_bounds__(kRB) void k_readout_bwd(int n, const uint16_t *__restrict__ h3,
                                                      const float *__restrict__ dy,
                                                      const float *__restrict__ prm,
                                                      const float *__restrict__ z3,
                                                      uint16_t *__restrict__ dz3,
                                                      double *__restrict__ part) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double v[H + 1];
+    constexpr int CH = H / 4, NW = kRB / 64;
+    __shared__ double red[NW][H + 1];
+    const int c = threadIdx.x % CH;
+    double w4[4], v[4] = {0.0, 0.0, 0.0, 0.0}, vd = 0.0;
 #pragma unroll
-    for (int k = 0; k <= H; ++k) v[k] = 0.0;
-    if (i < n) {
+    for (int f = 0; f < 4; ++f) w4[f] = (double)prm[OFF_W4 + 4 * c + f];
+    constexpr int NB = kRB / CH;  // nodes a block takes at a time
+    for (int64_t i = blockIdx.x * (int64_t)NB + threadIdx.x / CH; i < n;
+         i += (int64_t)gridDim.x * NB) {
         const float d = dy[i];
+        const uint2 h = *reinterpret_cast<const uint2 *>(h3 + i * H + 4 * c);
+        const float4 z = *reinterpret_cast<const float4 *>(z3 + i * H + 4 * c);
+        const uint32_t hb[4] = {h.x, h.x >> 16, h.y, h.y >> 16};
+        const float zz[4] = {z.x, z.y, z.z, z.w};
+        uint16_t r[4];
 #pragma unroll
-        for (int f = 0; f < H; ++f) {
-            const size_t e = (size_t)i * H + f;
-            v[f] = (double)bf2f(h3[e]) * (double)d;
-            const float dh = (float)((double)d * (double)prm[OFF_W4 + f]);
-            dz3[e] = z3[e] > 0.f ? f2bf(dh) : (uint16_t)0;
+        for (int f = 0; f < 4; ++f) {
+            v[f] += (double)bf2f(hb[f]) * (double)d;
+            const float dh = (float)((double)d * w4[f]);
+            r[f] = zz[f] > 0.f ? f2bf(dh) : (uint16_t)0;
         }
-        v[H] = (double)d;
+        vd += (double)d;
+        uint2 o;
+        o.x = (uint32_t)r[0] | ((uint32_t)r[1] << 16);
+        o.y = (uint32_t)r[2] | ((uint32_t)r[3] << 16);
+        *reinterpret_cast<uint2 *>(dz3 + i * H + 4 * c) = o;
     }
-    block_partial<H + 1>(v, part);
+    // lanes CH apart hold the same features
+#pragma unroll
+    for (int o = CH; o < 64; o *= 2) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) v[f] += __shfl_xor(v[f], o, 64);
+        vd += __shfl_xor(vd, o, 64);
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane < CH) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) red[wave][4 * c + f] = v[f];
+        if (lane == 0) red[wave][H] = vd;
+    }
+    __syncthreads();
+    if (threadIdx.x <= H) {
+        double t = 0.0;
+        for (int w = 0; w < NW; ++w) t += red[w][threadIdx.x];
+        part[(size_t)blockIdx.x * (H + 1) + threadIdx.x] = t;
+    }
 }
 
 // Partials of dW = X^T dz ([KP][H]) and dc = sum dz ([H]) per block:
@@ -377,30 +412,60 @@ __global__ void k_agg_bwd(int n, const int32_t *__restrict__ rs, const int32_t *
     *reinterpret_cast<uint2 *>(dzp + (size_t)i * H + 4 * c) = o;
 }
 
-// out[k] (+)= sum_b part[b][k], blocks in order (FP64), k < count
-__global__ void k_reduce(int nb, int count, const double *__restrict__ part, float *__restrict__ out,
-                         double *__restrict__ out64) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= count) return;
+// Sums of per-block partials part[b][e], b < nb, e < count (FP64): a block
+// takes kRedCols columns e, kRedSegs threads a column, each adding one
+// contiguous run of b in order; the runs are then added in order, so the sum
+// has one fixed order for a given nb.  The reads of a run are independent of
+// each other and kRedCols consecutive doubles (a 128-byte line) wide; one
+// thread a column, with its chain of nb dependent adds behind nb far-apart
+// loads, took 60-65 us for the 256 x 2,080 partials of a layer and 39 us
+// for 257 x 33, this 3.4 us each.
+constexpr int kRedCols = 16;
+constexpr int kRedSegs = kRB / kRedCols;
+
+__device__ __forceinline__ double sum_partials(int nb, int count, int e,
+                                               const double *__restrict__ part) {
+    __shared__ double seg[kRedSegs][kRedCols];
+    const int c = threadIdx.x % kRedCols, g = threadIdx.x / kRedCols;
+    const int lo = (int)((int64_t)nb * g / kRedSegs), hi = (int)((int64_t)nb * (g + 1) / kRedSegs);
     double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += part[(size_t)b * count + k];
-    if (out) out[k] = (float)s;
-    if (out64) out64[k] = s;
+    if (e < count) {
+#pragma unroll 8
+        for (int b = lo; b < hi; ++b) s += part[(size_t)b * count + e];
+    }
+    seg[g][c] = s;
+    __syncthreads();
+    s = 0.0;
+    if (g == 0) {
+#pragma unroll
+        for (int k = 0; k < kRedSegs; ++k) s += seg[k][c];
+    }
+    return s;  // whole in the threads with g == 0
+}
+
+// out[e] = sum_b part[b][e] in FP32 and / or FP64
+__global__ __launch_bounds__(kRB) void k_reduce(int nb, int count, const double *__restrict__ part,
+                                                float *__restrict__ out,
+                                                double *__restrict__ out64) {
+    const int e = blockIdx.x * kRedCols + threadIdx.x % kRedCols;
+    const double s = sum_partials(nb, count, e, part);
+    if (threadIdx.x >= kRedCols || e >= count) return;
+    if (out) out[e] = (float)s;
+    if (out64) out64[e] = s;
 }
 
 // grads of one dense layer from its partial buffer [nb][KP*H + H]:
 // rows < kin of dW, then dc
-__global__ void k_reduce_layer(int nb, int kp, int kin, const double *__restrict__ part,
-                               float *__restrict__ gW, float *__restrict__ gc) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kRB) void k_reduce_layer(int nb, int kp, int kin,
+                                                      const double *__restrict__ part,
+                                                      float *__restrict__ gW,
+                                                      float *__restrict__ gc) {
+    const int e = blockIdx.x * kRedCols + threadIdx.x % kRedCols;
     const int count = kp * H + H;
-    if (e >= count) return;
-    const bool is_w = e < kp * H;
-    if (is_w && e / H >= kin) return;
-    double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += part[(size_t)b * count + e];
-    if (is_w) gW[e] = (float)s;
-    else gc[e - kp * H] = (float)s;
+    const double s = sum_partials(nb, count, e, part);
+    if (threadIdx.x >= kRedCols || e >= count) return;
+    if (e >= kp * H) gc[e - kp * H] = (float)s;
+    else if (e / H < kin) gW[e] = (float)s;
 }
 
 // Gradient-norm clipping, one block: |g| against a running average of the
@@ -495,6 +560,11 @@ void gnn_pack(GnnNet &g) {
     NSFEM_HIP(hipGetLastError());
 }
 
+// Blocks of k_readout_bwd: 32 nodes each at a time, two blocks a CU at most.
+int readout_blocks(int n) { return std::min(512, gnn::blocks_for(n, gnn::kRB * 4 / gnn::H)); }
+
+int reduce_blocks(int count) { return gnn::blocks_for(count, gnn::kRedCols); }
+
 void gnn_reserve(GnnNet &g, int n) {
     if (n <= g.cap) return;
     using namespace gnn;
@@ -513,7 +583,8 @@ void gnn_reserve(GnnNet &g, int n) {
     const size_t nb = (size_t)blocks_for(n);
     const size_t groups = ((size_t)n + 15) / 16;
     const size_t nbw = std::max<size_t>(1, std::min<size_t>(256, (groups + 3) / 4));
-    g.part.resize(std::max(nb * (H + 1), nbw * (K2 * H + H)));
+    const size_t nbr = (size_t)readout_blocks(n);
+    g.part.resize(std::max(std::max(nb, nbr * (H + 1)), nbw * (K2 * H + H)));
     g.cap = n;
 }
 
@@ -564,15 +635,17 @@ void gnn_backward(GnnNet &g, GnnGraph &gr, const double *b, const double *p) {
     const int nb = blocks_for(n);
     launch_dot_accumulate(d, n, p, p, g.scal.ptr + 1);
     k_loss<<<nb, kRB, 0, d.stream>>>(n, g.phat.ptr, p, g.scal.ptr, g.dy.ptr, g.part.ptr);
-    k_reduce<<<1, 64, 0, d.stream>>>(nb, 1, g.part.ptr, nullptr, g.scal.ptr + 2);
-    k_readout_bwd<<<nb, kRB, 0, d.stream>>>(n, g.h3.ptr, g.dy.ptr, g.params.ptr, g.z3.ptr, g.dz.ptr,
-                                            g.part.ptr);
-    k_reduce<<<1, 64, 0, d.stream>>>(nb, H + 1, g.part.ptr, g.grads.ptr + OFF_W4, nullptr);
+    k_reduce<<<1, kRB, 0, d.stream>>>(nb, 1, g.part.ptr, nullptr, g.scal.ptr + 2);
+    const int nbr = readout_blocks(n);
+    k_readout_bwd<<<nbr, kRB, 0, d.stream>>>(n, g.h3.ptr, g.dy.ptr, g.params.ptr, g.z3.ptr,
+                                             g.dz.ptr, g.part.ptr);
+    k_reduce<<<reduce_blocks(H + 1), kRB, 0, d.stream>>>(nbr, H + 1, g.part.ptr,
+                                                         g.grads.ptr + OFF_W4, nullptr);
     const int nbw = bwd_w_blocks(n);
     const int nbt = blocks_for(((int64_t)n + 15) / 16 * 64);
     // layer 3
     k_dense_bwd_w<K2><<<nbw, kRB, 0, d.stream>>>(n, g.X3.ptr, g.dz.ptr, g.part.ptr);
-    k_reduce_layer<<<blocks_for(K2 * H + H), kRB, 0, d.stream>>>(
+    k_reduce_layer<<<reduce_blocks(K2 * H + H), kRB, 0, d.stream>>>(
         nbw, K2, K2, g.part.ptr, g.grads.ptr + OFF_W3, g.grads.ptr + OFF_C3);
     k_dense_bwd_x<K2><<<nbt, kRB, 0, d.stream>>>(n, g.dz.ptr, g.wr3.ptr, g.dX.ptr);
     k_agg_bwd<<<blocks_for((int64_t)n * (H / 4)), kRB, 0, d.stream>>>(n, gr.rs.ptr, gr.col.ptr,
@@ -580,7 +653,7 @@ void gnn_backward(GnnNet &g, GnnGraph &gr, const double *b, const double *p) {
                                                                       g.dz.ptr);
     // layer 2
     k_dense_bwd_w<K2><<<nbw, kRB, 0, d.stream>>>(n, g.X2.ptr, g.dz.ptr, g.part.ptr);
-    k_reduce_layer<<<blocks_for(K2 * H + H), kRB, 0, d.stream>>>(
+    k_reduce_layer<<<reduce_blocks(K2 * H + H), kRB, 0, d.stream>>>(
         nbw, K2, K2, g.part.ptr, g.grads.ptr + OFF_W2, g.grads.ptr + OFF_C2);
     k_dense_bwd_x<K2><<<nbt, kRB, 0, d.stream>>>(n, g.dz.ptr, g.wr2.ptr, g.dX.ptr);
     k_agg_bwd<<<blocks_for((int64_t)n * (H / 4)), kRB, 0, d.stream>>>(n, gr.rs.ptr, gr.col.ptr,
@@ -588,7 +661,7 @@ void gnn_backward(GnnNet &g, GnnGraph &gr, const double *b, const double *p) {
                                                                       g.dz.ptr);
     // layer 1 (8 real input rows of the 16-row padded operand)
     k_dense_bwd_w<K1><<<nbw, kRB, 0, d.stream>>>(n, g.X1.ptr, g.dz.ptr, g.part.ptr);
-    k_reduce_layer<<<blocks_for(K1 * H + H), kRB, 0, d.stream>>>(
+    k_reduce_layer<<<reduce_blocks(K1 * H + H), kRB, 0, d.stream>>>(
         nbw, K1, 8, g.part.ptr, g.grads.ptr + OFF_W1, g.grads.ptr + OFF_C1);
     NSFEM_HIP(hipGetLastError());
 }

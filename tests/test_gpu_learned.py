@@ -85,6 +85,33 @@ def test_gradients_match_oracle(gpu, kind):
     pg.close()
 
 
+@pytest.mark.parametrize("n", [1, 4, 15, 16, 130])
+def test_gradient_sums_at_their_edges(gpu, n):
+    """Node counts at the edges of the gradient sums: 4 nodes (fewer partials
+    than runs, most of a block idle), 25, 256 and 289 around one block, and
+    17,161, more than one round of the readout's blocks.  Same bounds as the
+    oracle comparison above."""
+    from navier_stokes_fem_amd import learned as L, mesh
+    from oracle import gnn
+
+    og, pg, b, p, bb, pb = _setup(gpu, mesh.cavity(n), seed=n)
+    params = gnn.init_params(9)
+    rng = np.random.default_rng(10)
+    for k in params:
+        params[k] = (params[k] + 0.05 * rng.standard_normal(params[k].shape)).astype(np.float32)
+    net = L.WarmStartNet(gpu)
+    net.set_params(L.WarmStartNet.flatten(params))
+    loss, flat = net.gradients(pg, bb, pb)
+    want_loss, want, _ = gnn.loss_and_grad(params, og, b, p, bf16_mode=True)
+    assert loss == pytest.approx(want_loss, rel=5e-3)
+    got = L.WarmStartNet.unflatten(flat)
+    for name, _ in L.WarmStartNet.LAYOUT:
+        e = np.linalg.norm(got[name] - want[name]) / (np.linalg.norm(want[name]) + 1e-30)
+        assert e < 1e-2, (name, e)
+    net.close()
+    pg.close()
+
+
 def test_adam_step_clips_outlier_gradients(gpu):
     """Two Adam steps against the update restated on the host: an ordinary
     pair (its norm starts the running average, no clipping), then the same
