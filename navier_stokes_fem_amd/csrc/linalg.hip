@@ -201,21 +201,14 @@ void set_group_loads(Matrix &m) {
 void build_tiles(Matrix &m, const std::vector<int32_t> &rs) {
     std::vector<int32_t> t = cut_rows(rs, m.rows, kTileRows, kSpmvTileNnz);
     m.n_tiles = (int)t.size() - 1;
-    m.host_tiles = t;
-    m.tiles.resize(t.size());
-    NSFEM_HIP(hipMemcpy(m.tiles.ptr, t.data(), t.size() * sizeof(int32_t),
-                        hipMemcpyHostToDevice));
     m.host_rs = rs;
-    {
-        std::vector<int4> meta((size_t)std::max(m.n_tiles, 1));
-        for (int i = 0; i < m.n_tiles; ++i)
-            meta[i] = make_int4(t[i], t[i + 1], rs[t[i]], rs[t[i + 1]] - rs[t[i]]);
-        DeviceArray<int4> dmeta;
-        dmeta.resize(meta.size());
-        NSFEM_HIP(hipMemcpy(dmeta.ptr, meta.data(), meta.size() * sizeof(int4),
-                            hipMemcpyHostToDevice));
-        m.bcol_ok = col_delta(m, m.n_tiles, dmeta.ptr, m.bcol);
-    }
+    std::vector<int4> meta((size_t)std::max(m.n_tiles, 1));
+    for (int i = 0; i < m.n_tiles; ++i)
+        meta[i] = make_int4(t[i], t[i + 1], rs[t[i]], rs[t[i + 1]] - rs[t[i]]);
+    m.tiles.resize(meta.size());
+    NSFEM_HIP(hipMemcpy(m.tiles.ptr, meta.data(), meta.size() * sizeof(int4),
+                        hipMemcpyHostToDevice));
+    m.bcol_ok = col_delta(m, m.n_tiles, m.tiles.ptr, m.bcol);
     build_wave_tiles(m, kWaveRows, kStageNnz);
 }
 
@@ -375,7 +368,7 @@ namespace {
 // suffers on smooth vectors).
 template <int MODE, typename IT, typename T, typename S = T>
 __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_t nnz,
-                                                 const int32_t *__restrict__ tiles,
+                                                 const int4 *__restrict__ tiles,
                                                  const int32_t *__restrict__ rs,
                                                  const int32_t *__restrict__ col,
                                                  const int16_t *__restrict__ bcol,
@@ -390,9 +383,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
     const int t = xcd_swizzle(blockIdx.x, gridDim.x);
     if (t >= n_tiles) return;
     const int tid = threadIdx.x;
-    const int r0 = tiles[t], r1 = tiles[t + 1];
-    const int k0 = rs[r0];
-    const int nz = rs[r1] - k0;
+    const int4 tile = tiles[t];
+    const int r0 = tile.x, r1 = tile.y, k0 = tile.z, nz = tile.w;
     if (nz <= kSpmvTileNnz) {
         // groups of 4 nonzeros from ka = k0 rounded down to a multiple of 4;
         // entries of the neighbouring tiles in the first and last group are
@@ -445,6 +437,20 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
                 }
             }
         }
+        // the row's own words, needed only after the barrier: asked for here,
+        // behind the streams
+        const int row = r0 + tid;
+        int ra = ka, rb = ka;
+        S lrow = S(0), drow = S(0), xrow = S(0);
+        if (row < r1) {
+            ra = rs[row];
+            rb = rs[row + 1];
+            if (MODE != 0) lrow = lhs[row];
+            if (MODE == 3) {
+                drow = dinv[row];
+                xrow = (S)x[row];
+            }
+        }
         // columns transposed through the wave's own slice of prod (256
         // products; the 256 columns take 1 KB of it), so that each gather
         // instruction covers 64 consecutive nonzeros
@@ -489,17 +495,15 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
             }
         }
         __syncthreads();
-        const int row = r0 + tid;
         if (row < r1) {
-            const int a = rs[row] - ka, b = rs[row + 1] - ka;
             S s = S(0);
-            for (int k = a; k < b; ++k) s += prod[k];
+            for (int k = ra - ka; k < rb - ka; ++k) s += prod[k];
             if (MODE == 0) y[row] = s;
-            if (MODE == 1) y[row] = lhs[row] - s;
-            if (MODE == 2) y[row] = s - lhs[row];
+            if (MODE == 1) y[row] = lrow - s;
+            if (MODE == 2) y[row] = s - lrow;
             if (MODE == 3) {
-                const S r = lhs[row] - s;
-                y[row] = __builtin_fma(omega * dinv[row], r, (S)x[row]);
+                const S r = lrow - s;
+                y[row] = __builtin_fma(omega * drow, r, xrow);
             }
         }
     } else {  // one row longer than a tile

@@ -116,9 +116,8 @@ struct Matrix {
     DeviceArray<int32_t> row_start, col;
     DeviceArray<double> val;
     DeviceArray<float> val32;  // FP32 copy for the refined solver (lazy)
-    DeviceArray<int32_t> tiles;  // [n_tiles + 1] first row of each tile
+    DeviceArray<int4> tiles;  // [n_tiles] {first row, end row, first nnz, nnz}
     int n_tiles = 0;
-    std::vector<int32_t> host_tiles;
     DeviceArray<int32_t> wtiles;  // [n_wtiles + 1] first row of each wave tile
     DeviceArray<int4> wmeta;      // [n_wtiles] {first row, end row, first nnz, nnz}
     int n_wtiles = 0;
