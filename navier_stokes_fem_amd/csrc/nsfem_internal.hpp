@@ -260,6 +260,9 @@ void launch_spmv(Device &d, Matrix &m, const double *x, const double *lhs, doubl
                  int mode);
 // the same in FP32 from the FP32 copy of the values (ensure_val32 first)
 void launch_spmv(Device &d, Matrix &m, const float *x, const float *lhs, float *y, int mode);
+// y = A x with a dense row-major n x n matrix (double, float)
+template <typename T>
+void launch_dense(Device &d, int n, const T *a, const T *x, T *y);
 void launch_axpy(Device &d, int n, double a, const double *x, double *y);
 void launch_axpby(Device &d, int n, double a, double b, const double *x,
                   const double *y, double *out);

@@ -95,14 +95,16 @@ struct LevelVectors<float> {
 // for a deepest level of at most kMgDenseMax nodes, its dense inverse.
 struct MgLevels {
     std::vector<std::unique_ptr<MgLevel>> lv;
-    Matrix deep_inv;  // as CSR
+    DeviceArray<double> deep_inv;   // row-major
+    DeviceArray<float> deep_inv32;  // the FP32 cycle's (built on first use)
     bool deep_ok = false;
     std::vector<int32_t> deep_rs, deep_col;
     std::vector<double> deep_val;
     bool fp32_ok = false;  // the levels' FP32 vectors and values are built
     void release() {
         lv.clear();
-        matrix_release(deep_inv);
+        deep_inv.release();
+        deep_inv32.release();
         deep_ok = false;
         fp32_ok = false;
         deep_rs.clear();
@@ -110,6 +112,17 @@ struct MgLevels {
         deep_val.clear();
     }
 };
+
+template <typename T>
+const T *deep_inverse(const MgLevels &m);
+template <>
+const double *deep_inverse<double>(const MgLevels &m) {
+    return m.deep_inv.ptr;
+}
+template <>
+const float *deep_inverse<float>(const MgLevels &m) {
+    return m.deep_inv32.ptr;
+}
 
 struct Simulation {
     Device *dev = nullptr;
@@ -761,7 +774,7 @@ void mg_cycle(Device &d, Matrix &A, int n, const T *dinv, T *r, MgLevels &m, siz
               const T *b, T *x, bool zero = true, int sweeps = kMgSweeps,
               double omega = kMgOmega) {
     if (l == m.lv.size() && m.deep_ok) {
-        launch_spmv(d, m.deep_inv, b, nullptr, x, 0);
+        launch_dense(d, n, deep_inverse<T>(m), b, x);
         return;
     }
     if (l == m.lv.size() || (zero && sweeps == 0)) launch_fill(d, n, 0.0, x);
@@ -817,7 +830,10 @@ void ensure_fp32_levels(Device &d, MgLevels &m) {
         launch_convert(d, l.n, l.dinv.ptr, l.dinv32.ptr);
         for (DeviceArray<float> *a : {&l.b32, &l.x32, &l.r32}) a->resize((size_t)l.n);
     }
-    if (m.deep_ok) ensure_val32(d, m.deep_inv);
+    if (m.deep_ok) {
+        m.deep_inv32.resize(m.deep_inv.count);
+        launch_convert(d, (int)m.deep_inv.count, m.deep_inv.ptr, m.deep_inv32.ptr);
+    }
     m.fp32_ok = true;
 }
 
@@ -1329,17 +1345,15 @@ namespace {
 // The dense inverse of m's deepest level when it has at most kMgDenseMax
 // nodes and is positive definite (else the deepest level keeps CG).
 void dense_inverse(Device &d, MgLevels &m) {
-    matrix_release(m.deep_inv);
+    m.deep_inv.release();
+    m.deep_inv32.release();
     m.deep_ok = false;
     const int n = m.lv.back()->n;
     if (n > kMgDenseMax) return;
     std::vector<double> inv;
     if (!spd_inverse(n, m.deep_rs.data(), m.deep_col.data(), m.deep_val.data(), inv)) return;
-    std::vector<int32_t> rs((size_t)n + 1), col((size_t)n * n);
-    for (int r = 0; r <= n; ++r) rs[r] = r * n;
-    for (int r = 0; r < n; ++r)
-        for (int c = 0; c < n; ++c) col[(size_t)r * n + c] = c;
-    upload_csr(d, m.deep_inv, n, n, (int64_t)n * n, rs.data(), col.data(), inv.data());
+    m.deep_inv.resize((size_t)n * n);
+    NSFEM_HIP(hipMemcpy(m.deep_inv.ptr, inv.data(), m.deep_inv.bytes(), hipMemcpyHostToDevice));
     m.deep_ok = true;
 }
 
