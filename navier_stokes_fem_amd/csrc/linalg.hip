@@ -358,6 +358,13 @@ namespace {
 // MODE 2: y = A x - lhs.  MODE 3: y = x + omega dinv (lhs - A x), a damped
 // Jacobi sweep into another vector (y aliases neither x nor lhs; the same
 // roundings as the residual product followed by k_jacobi).
+// MODE 4: y += A x (the roundings of the product followed by k_add).
+// MODE 5: y = A x and y2 = omega dinv y, the Jacobi sweep from zero that
+// follows a restriction (k_jacobi0's roundings).
+// DOT: partial[tile] = the tile's rows' sum of y times x (MODE 0) or times
+// rdot (MODE 3) in FP64, one wave after the other: a CG's (p, A p) and
+// (r, z) without another pass over the vectors or another launch (a launch
+// costs 3.3 us however little it does).
 // IT = int16_t reads the columns as 16-bit offsets from the tile's first row
 // (bcol, square matrices whose offsets fit): 2 bytes less per nonzero.
 // T = double: the FP64 values; T = float: the FP32 copy (val32) with FP32
@@ -366,7 +373,16 @@ namespace {
 // values and x (each FP32 x FP32 product exact in FP64, summed in FP64: the
 // product of a CG's FP32 direction, free of the cancellation an FP32 sum
 // suffers on smooth vectors).
-template <int MODE, typename IT, typename T, typename S = T>
+template <typename S>
+struct SpmvTail {
+    const S *dinv = nullptr;
+    S omega = S(0);
+    S *y2 = nullptr;
+    const double *rdot = nullptr;
+    double *partial = nullptr;
+};
+
+template <int MODE, typename IT, typename T, typename S = T, bool DOT = false>
 __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_t nnz,
                                                  const int4 *__restrict__ tiles,
                                                  const int32_t *__restrict__ rs,
@@ -374,12 +390,13 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
                                                  const int16_t *__restrict__ bcol,
                                                  const T *__restrict__ val,
                                                  const T *__restrict__ x,
-                                                 const S *lhs, S *y,
-                                                 const S *__restrict__ dinv, S omega) {
+                                                 const S *lhs, S *y, const SpmvTail<S> tail) {
     constexpr bool F64 = std::is_same<T, double>::value;
     constexpr bool S64 = std::is_same<S, double>::value;
     __shared__ __align__(16) S prod[kTileNnz];
     __shared__ S red[kWaves];
+    __shared__ double dred[DOT ? kWaves : 1];
+    double dsum[1] = {0.0};
     const int t = xcd_swizzle(blockIdx.x, gridDim.x);
     if (t >= n_tiles) return;
     const int tid = threadIdx.x;
@@ -442,14 +459,15 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
         const int row = r0 + tid;
         int ra = ka, rb = ka;
         S lrow = S(0), drow = S(0), xrow = S(0);
+        double dotrow = 0.0;
         if (row < r1) {
             ra = rs[row];
             rb = rs[row + 1];
-            if (MODE != 0) lrow = lhs[row];
-            if (MODE == 3) {
-                drow = dinv[row];
-                xrow = (S)x[row];
-            }
+            if (MODE >= 1 && MODE <= 3) lrow = lhs[row];
+            if (MODE == 4) lrow = y[row];
+            if (MODE == 3 || MODE == 5) drow = tail.dinv[row];
+            if (MODE == 3 || (DOT && MODE == 0)) xrow = (S)x[row];
+            if (DOT && MODE == 3) dotrow = tail.rdot[row];
         }
         // columns transposed through the wave's own slice of prod (256
         // products; the 256 columns take 1 KB of it), so that each gather
@@ -503,8 +521,19 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
             if (MODE == 2) y[row] = s - lrow;
             if (MODE == 3) {
                 const S r = lrow - s;
-                y[row] = __builtin_fma(omega * drow, r, xrow);
+                s = __builtin_fma(tail.omega * drow, r, xrow);
+                y[row] = s;
             }
+            if (MODE == 4) y[row] = s + lrow;
+            if (MODE == 5) {
+                y[row] = s;
+                tail.y2[row] = (tail.omega * drow) * s;
+            }
+            if (DOT) dsum[0] = (double)s * (MODE == 0 ? (double)xrow : dotrow);
+        }
+        if (DOT) {
+            block_sum<1, kBlock>(dsum, dred);
+            if (tid == 0) tail.partial[t] = dsum[0];
         }
     } else {  // one row longer than a tile
         S s = S(0);
@@ -520,8 +549,15 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n_tiles, int n_rows, int64_
             if (MODE == 2) y[r0] = tot - lhs[r0];
             if (MODE == 3) {
                 const S r = lhs[r0] - tot;
-                y[r0] = __builtin_fma(omega * dinv[r0], r, (S)x[r0]);
+                tot = __builtin_fma(tail.omega * tail.dinv[r0], r, (S)x[r0]);
+                y[r0] = tot;
             }
+            if (MODE == 4) y[r0] = tot + y[r0];
+            if (MODE == 5) {
+                y[r0] = tot;
+                tail.y2[r0] = (tail.omega * tail.dinv[r0]) * tot;
+            }
+            if (DOT) tail.partial[t] = (double)tot * (MODE == 0 ? (double)x[r0] : tail.rdot[r0]);
         }
     }
 }
@@ -593,7 +629,9 @@ __global__ void k_axpby(int n, double a, double b, const double *x, const double
 }
 
 // Deterministic dot: block k sums the contiguous chunk k, a single block adds
-// the chunk sums in order.
+// the chunk sums in order.  Chunks of 1,024 until there are kDotBlocks of
+// them: with 4,096 a vector of some ten thousand entries had 16 dependent
+// rounds on ten CUs (6.8 us on 40,401 entries, a launch's 3 us included).
 __global__ __launch_bounds__(kBlock) void k_dot_partial(int n, int chunk,
                                                         const double *__restrict__ a,
                                                         const double *__restrict__ b,
@@ -602,6 +640,7 @@ __global__ __launch_bounds__(kBlock) void k_dot_partial(int n, int chunk,
     const int lo = blockIdx.x * chunk;
     const int hi = min(n, lo + chunk);
     double s[1] = {0.0};
+#pragma unroll 4
     for (int i = lo + threadIdx.x; i < hi; i += kBlock) s[0] = __builtin_fma(a[i], b[i], s[0]);
     block_sum<1, kBlock>(s, lds);
     if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
@@ -616,55 +655,102 @@ __global__ __launch_bounds__(kBlock) void k_dot_final(int nb, const double *__re
     if (threadIdx.x == 0) result[0] += s[0];
 }
 
-// The update of a CG with FP32 directions p (q = A p in FP64) and an FP32
-// preconditioner: x += a p and r -= a q in FP64, r32 = r rounded to FP32
-// (the preconditioner's input), and the partial sums of (r, r) per
-// contiguous chunk in k_dot_partial's order (k_dot_final adds them).
-__global__ __launch_bounds__(kBlock) void k_pcg_update(int n, int chunk, double a,
-                                                       const float *__restrict__ p,
-                                                       const double *__restrict__ q,
-                                                       double *__restrict__ x,
-                                                       double *__restrict__ r,
-                                                       float *__restrict__ r32,
-                                                       double *__restrict__ partial) {
+// The sum of n partials, the same bits in every thread of every block.
+__device__ __forceinline__ double sum_partials(int n, const double *__restrict__ part,
+                                               double *lds) {
+    double s[1] = {0.0};
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += kBlock) s[0] += part[i];
+    block_sum<1, kBlock>(s, lds);
+    return s[0];
+}
+
+// out[block] = the sum of the block's contiguous share of part[0..n)
+__global__ __launch_bounds__(kBlock) void k_fold(int n, const double *__restrict__ part,
+                                                 double *__restrict__ out) {
     __shared__ double lds[kWaves];
+    const int lo = (int)((int64_t)n * blockIdx.x / gridDim.x);
+    const int hi = (int)((int64_t)n * (blockIdx.x + 1) / gridDim.x);
+    const double s = sum_partials(hi - lo, part + lo, lds);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
+// The update of a CG with FP32 directions p (q = A p in FP64) and an FP32
+// preconditioner, step `k`: alpha = (r, z) / (p, q), (p, q) the sum of npq
+// partials that every block adds for itself; x += alpha p and r -= alpha q
+// in FP64, r32 = r rounded to FP32 (the preconditioner's input), x0 = omega
+// dinv r32 (its first Jacobi sweep, from zero), and the partial sums of
+// (r, r) per contiguous chunk.  A (p, q) or (r, z) that is not positive
+// leaves x and r as they are, for the host to see.
+__global__ __launch_bounds__(kBlock) void k_pcg_update(
+    int n, int chunk, PcgScalars *sc, int k, int npq, const double *__restrict__ pq_part,
+    const float *__restrict__ p, const double *__restrict__ q, double *__restrict__ x,
+    double *__restrict__ r, float *__restrict__ r32, const float *__restrict__ dinv, float omega,
+    float *__restrict__ x0, double *__restrict__ partial) {
+    __shared__ double lds[kWaves];
+    const double pq = sum_partials(npq, pq_part, lds);
+    const double rz = sc->rz[k & 1];
+    const double a = pq > 0.0 && rz > 0.0 ? rz / pq : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc->pq = pq;
     const int lo = blockIdx.x * chunk;
     const int hi = min(n, lo + chunk);
     double s[1] = {0.0};
-    for (int i = lo + threadIdx.x; i < hi; i += kBlock) {
-        x[i] = __builtin_fma(a, (double)p[i], x[i]);
-        const double ri = __builtin_fma(-a, q[i], r[i]);
-        r[i] = ri;
-        r32[i] = (float)ri;
-        s[0] = __builtin_fma(ri, ri, s[0]);
+    if (a > 0.0) {
+#pragma unroll 2
+        for (int i = lo + threadIdx.x; i < hi; i += kBlock) {
+            x[i] = __builtin_fma(a, (double)p[i], x[i]);
+            const double ri = __builtin_fma(-a, q[i], r[i]);
+            const float rf = (float)ri;
+            r[i] = ri;
+            r32[i] = rf;
+            x0[i] = (omega * dinv[i]) * rf;
+            s[0] = __builtin_fma(ri, ri, s[0]);
+        }
     }
     block_sum<1, kBlock>(s, lds);
     if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
 }
 
-// Partial sums of (a, b), each operand FP64 or FP32 (widened), per chunk,
-// in k_dot_partial's order.
-template <typename A, typename B>
-__global__ __launch_bounds__(kBlock) void k_dot_any_partial(int n, int chunk,
-                                                            const A *__restrict__ a,
-                                                            const B *__restrict__ b,
-                                                            double *__restrict__ partial) {
+// The step's scalars to the host's page: (r, r) from its partials, (p, q)
+// and (r, z).  One block.
+__global__ __launch_bounds__(kBlock) void k_pcg_report(int nrr, const double *__restrict__ rr_part,
+                                                       const PcgScalars *__restrict__ sc, int k,
+                                                       PcgReport *host) {
     __shared__ double lds[kWaves];
-    const int lo = blockIdx.x * chunk;
-    const int hi = min(n, lo + chunk);
-    double s[1] = {0.0};
-    for (int i = lo + threadIdx.x; i < hi; i += kBlock)
-        s[0] = __builtin_fma((double)a[i], (double)b[i], s[0]);
-    block_sum<1, kBlock>(s, lds);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
+    const double rr = sum_partials(nrr, rr_part, lds);
+    if (threadIdx.x == 0) {
+        host->rr = rr;
+        host->pq = sc->pq;
+        host->rz = sc->rz[k & 1];
+    }
 }
 
-// p = z + b p in FP32 storage (the CG's new direction; the sum in FP64)
-__global__ void k_pcg_direction(int n, const float *__restrict__ z, double b,
-                                float *__restrict__ p) {
+// r32 = r rounded to FP32 and x0 = omega dinv r32 (see k_pcg_update)
+__global__ void k_pcg_round(int n, const double *__restrict__ r, float *__restrict__ r32,
+                            const float *__restrict__ dinv, float omega, float *__restrict__ x0) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x) {
+        const float rf = (float)r[i];
+        r32[i] = rf;
+        x0[i] = (omega * dinv[i]) * rf;
+    }
+}
+
+// The direction of step k: p = z + beta p in FP32 storage, the sum in FP64,
+// beta = (r, z) / the step before's (p = z at k = 0).  (r, z) is the sum of
+// nrz partials, which every block adds for itself.
+__global__ __launch_bounds__(kBlock) void k_pcg_direction(int n, int nrz,
+                                                          const double *__restrict__ rz_part,
+                                                          PcgScalars *sc, int k,
+                                                          const float *__restrict__ z,
+                                                          float *__restrict__ p) {
+    __shared__ double lds[kWaves];
+    const double rz = sum_partials(nrz, rz_part, lds);
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc->rz[k & 1] = rz;
+    const double b = k > 0 ? rz / sc->rz[(k + 1) & 1] : 0.0;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = (float)__builtin_fma(b, (double)p[i], (double)z[i]);
+        p[i] = k > 0 ? (float)__builtin_fma(b, (double)p[i], (double)z[i]) : z[i];
 }
 
 __global__ void k_scatter(int count, const int32_t *__restrict__ idx,
@@ -685,15 +771,6 @@ __global__ void k_add(int n, const T *__restrict__ a, T *__restrict__ y) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
         y[i] = a[i] + y[i];
-}
-
-// x += w * dinv .* r (a damped Jacobi update from the residual r)
-template <typename T>
-__global__ void k_jacobi(int n, T w, const T *__restrict__ dinv, const T *__restrict__ r,
-                         T *__restrict__ x) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        x[i] = __builtin_fma(w * dinv[i], r[i], x[i]);
 }
 
 // x = w * dinv .* b (the damped Jacobi sweep from x = 0)
@@ -726,6 +803,14 @@ __global__ void k_copy(int n, const double *__restrict__ a, double *__restrict__
         y[i] = a[i];
 }
 
+constexpr int kDotBlocks = 1024;  // per-block partials of the dot product
+
+// blocks and chunk of the deterministic dot over n entries
+void dot_shape(int n, int &nb, int &chunk) {
+    nb = (int)std::max<int64_t>(1, std::min<int64_t>(((int64_t)n + 1023) / 1024, kDotBlocks));
+    chunk = (int)std::max<int64_t>(1, ((int64_t)n + nb - 1) / nb);
+}
+
 // One element per thread up to 2^28 elements: a full grid streams at
 // 6.1 TB/s (copy) on MI355X where a grid-stride loop over 8192 blocks
 // reaches 4.5.
@@ -745,21 +830,17 @@ const float *values<float>(Matrix &m) {
     return m.val32.ptr;
 }
 
-template <int MODE, typename IT, typename T, typename S>
-void spmv_launch(Device &d, Matrix &m, const T *x, const S *lhs, S *y, const S *dinv,
-                 S omega) {
-    k_spmv<MODE, IT, T, S><<<m.n_tiles, kBlock, 0, d.stream>>>(
-        m.n_tiles, m.rows, m.nnz, m.tiles.ptr, m.row_start.ptr, m.col.ptr, m.bcol.ptr,
-        values<T>(m), x, lhs, y, dinv, omega);
-}
-
-template <int MODE, typename T, typename S>
+template <int MODE, typename T, typename S, bool DOT = false>
 void spmv_launch(Device &d, Matrix &m, const T *x, const S *lhs, S *y,
-                 const S *dinv = nullptr, S omega = S(0)) {
+                 const SpmvTail<S> &tail = SpmvTail<S>()) {
     if (m.bcol_ok && want_idx16())
-        spmv_launch<MODE, int16_t, T, S>(d, m, x, lhs, y, dinv, omega);
+        k_spmv<MODE, int16_t, T, S, DOT><<<m.n_tiles, kBlock, 0, d.stream>>>(
+            m.n_tiles, m.rows, m.nnz, m.tiles.ptr, m.row_start.ptr, m.col.ptr, m.bcol.ptr,
+            values<T>(m), x, lhs, y, tail);
     else
-        spmv_launch<MODE, int32_t, T, S>(d, m, x, lhs, y, dinv, omega);
+        k_spmv<MODE, int32_t, T, S, DOT><<<m.n_tiles, kBlock, 0, d.stream>>>(
+            m.n_tiles, m.rows, m.nnz, m.tiles.ptr, m.row_start.ptr, m.col.ptr, m.bcol.ptr,
+            values<T>(m), x, lhs, y, tail);
 }
 
 template <typename T>
@@ -788,27 +869,132 @@ void launch_spmv(Device &d, Matrix &m, const float *x, const float *lhs, float *
     spmv_any(d, m, x, lhs, y, mode);
 }
 
-// y = A x with FP32 values and x, the products and sums in FP64
-void launch_spmv_acc64(Device &d, Matrix &m, const float *x, double *y) {
+namespace {
+template <typename T>
+void require_values(const Matrix &m) {
+    NSFEM_REQUIRE((std::is_same<T, double>::value || m.val32.ptr), NSFEM_NOT_READY,
+                  "FP32 product without the FP32 copy of the values");
+}
+}  // namespace
+
+template <typename T>
+void launch_sweep(Device &d, Matrix &m, double w, const T *dinv, const T *x, const T *b, T *y) {
     if (m.rows == 0) return;
-    NSFEM_REQUIRE(m.val32.ptr, NSFEM_NOT_READY, "FP32 product without the FP32 copy of the values");
-    spmv_launch<0, float, double>(d, m, x, (const double *)nullptr, y);
+    require_values<T>(m);
+    SpmvTail<T> tail;
+    tail.dinv = dinv;
+    tail.omega = (T)w;
+    spmv_launch<3>(d, m, x, b, y, tail);
+    NSFEM_HIP(hipGetLastError());
+}
+template void launch_sweep(Device &, Matrix &, double, const double *, const double *,
+                           const double *, double *);
+template void launch_sweep(Device &, Matrix &, double, const float *, const float *, const float *,
+                           float *);
+
+template <typename T>
+void launch_spmv_add(Device &d, Matrix &m, const T *x, T *y) {
+    if (m.rows == 0) return;
+    require_values<T>(m);
+    spmv_launch<4>(d, m, x, (const T *)nullptr, y);
+    NSFEM_HIP(hipGetLastError());
+}
+template void launch_spmv_add(Device &, Matrix &, const double *, double *);
+template void launch_spmv_add(Device &, Matrix &, const float *, float *);
+
+template <typename T>
+void launch_restrict(Device &d, Matrix &m, const T *x, T *y, double w, const T *dinv, T *y2) {
+    if (m.rows == 0) return;
+    require_values<T>(m);
+    SpmvTail<T> tail;
+    tail.dinv = dinv;
+    tail.omega = (T)w;
+    tail.y2 = y2;
+    spmv_launch<5>(d, m, x, (const T *)nullptr, y, tail);
+    NSFEM_HIP(hipGetLastError());
+}
+template void launch_restrict(Device &, Matrix &, const double *, double *, double, const double *,
+                              double *);
+template void launch_restrict(Device &, Matrix &, const float *, float *, double, const float *,
+                              float *);
+
+// --------------------------------- CG with an FP32 preconditioner
+namespace {
+// Partials that a kernel's blocks add for themselves; more of them are folded
+// to one first, which two launches over a thousand tiles hide.
+constexpr int kPcgInline = 1024;
+constexpr int kPcgFold = 256;
+
+void fold_partials(Device &d, PcgDevice &w) {
+    if (w.count <= kPcgInline) {
+        w.sums = w.partial.ptr;
+        return;
+    }
+    double *folded = w.partial.ptr + w.count, *one = folded + kPcgFold;
+    k_fold<<<kPcgFold, kBlock, 0, d.stream>>>(w.count, w.partial.ptr, folded);
+    k_fold<<<1, kBlock, 0, d.stream>>>(kPcgFold, folded, one);
+    NSFEM_HIP(hipGetLastError());
+    w.sums = one;
+    w.count = 1;
+}
+}  // namespace
+
+void pcg_reserve(Device &d, const Matrix &m, PcgDevice &w) {
+    w.partial.ensure((size_t)m.n_tiles + kPcgFold + 1);
+    w.scalars.ensure(1);
+    w.report.ensure();
+    d.dot_partial.ensure(kDotBlocks);
+}
+
+void launch_pcg_round(Device &d, int n, const double *r, float *r32, const float *dinv, double w,
+                      float *x0) {
+    if (n <= 0) return;
+    k_pcg_round<<<ew_grid(n), kBlock, 0, d.stream>>>(n, r, r32, dinv, (float)w, x0);
     NSFEM_HIP(hipGetLastError());
 }
 
-void launch_sweep(Device &d, Matrix &m, double w, const double *dinv, const double *x,
-                  const double *b, double *y) {
-    if (m.rows == 0) return;
-    spmv_launch<3>(d, m, x, b, y, dinv, w);
+void launch_pcg_product(Device &d, Matrix &m, const float *p, double *q, PcgDevice &w) {
+    require_values<float>(m);
+    SpmvTail<double> tail;
+    tail.partial = w.partial.ptr;
+    w.count = m.n_tiles;
+    spmv_launch<0, float, double, true>(d, m, p, (const double *)nullptr, q, tail);
     NSFEM_HIP(hipGetLastError());
 }
 
-void launch_sweep(Device &d, Matrix &m, double w, const float *dinv, const float *x,
-                  const float *b, float *y) {
-    if (m.rows == 0) return;
-    NSFEM_REQUIRE(m.val32.ptr, NSFEM_NOT_READY, "FP32 sweep without the FP32 copy of the values");
-    spmv_launch<3>(d, m, x, b, y, dinv, (float)w);
+void launch_pcg_sweep(Device &d, Matrix &m, double omega, const float *dinv, const float *x,
+                      const float *b, float *y, const double *r, PcgDevice &w) {
+    require_values<float>(m);
+    SpmvTail<float> tail;
+    tail.dinv = dinv;
+    tail.omega = (float)omega;
+    tail.rdot = r;
+    tail.partial = w.partial.ptr;
+    w.count = m.n_tiles;
+    spmv_launch<3, float, float, true>(d, m, x, b, y, tail);
     NSFEM_HIP(hipGetLastError());
+}
+
+void launch_pcg_direction(Device &d, int n, int k, const float *z, float *p, PcgDevice &w) {
+    fold_partials(d, w);
+    k_pcg_direction<<<ew_grid(n), kBlock, 0, d.stream>>>(n, w.count, w.sums, w.scalars.ptr, k, z,
+                                                        p);
+    NSFEM_HIP(hipGetLastError());
+}
+
+PcgReport pcg_update(Device &d, int n, int k, const float *p, const double *q, double *x,
+                     double *r, float *r32, const float *dinv, double omega, float *x0,
+                     PcgDevice &w) {
+    fold_partials(d, w);
+    int nb, chunk;
+    dot_shape(n, nb, chunk);
+    k_pcg_update<<<nb, kBlock, 0, d.stream>>>(n, chunk, w.scalars.ptr, k, w.count, w.sums, p, q, x,
+                                              r, r32, dinv, (float)omega, x0, d.dot_partial.ptr);
+    k_pcg_report<<<1, kBlock, 0, d.stream>>>(nb, d.dot_partial.ptr, w.scalars.ptr, k,
+                                             w.report.device);
+    NSFEM_HIP(hipGetLastError());
+    NSFEM_HIP(hipStreamSynchronize(d.stream));
+    return *w.report.host;
 }
 
 template <typename T>
@@ -860,13 +1046,12 @@ void launch_axpby(Device &d, int n, double a, double b, const double *x, const d
 }
 
 namespace {
-constexpr int kDotBlocks = 1024;  // per-block partials of the dot product
 
 // partial: kDotBlocks doubles of scratch
 void dot_accumulate(Device &d, int n, const double *a, const double *b, double *result,
                     double *partial) {
-    const int nb = std::max(1, std::min((n + 4095) / 4096, kDotBlocks));
-    const int chunk = std::max(1, (n + nb - 1) / nb);
+    int nb, chunk;
+    dot_shape(n, nb, chunk);
     k_dot_partial<<<nb, kBlock, 0, d.stream>>>(n, chunk, a, b, partial);
     k_dot_final<<<1, kBlock, 0, d.stream>>>(nb, partial, result);
     NSFEM_HIP(hipGetLastError());
@@ -877,58 +1062,6 @@ void launch_dot_accumulate(Device &d, int n, const double *a, const double *b,
                            double *result) {
     d.dot_partial.ensure(kDotBlocks);
     dot_accumulate(d, n, a, b, result, d.dot_partial.ptr);
-}
-
-namespace {
-// blocks and chunk of the deterministic dot over n entries
-void dot_shape(int n, int &nb, int &chunk) {
-    nb = std::max(1, std::min((n + 4095) / 4096, kDotBlocks));
-    chunk = std::max(1, (n + nb - 1) / nb);
-}
-}  // namespace
-
-void launch_pcg_update(Device &d, int n, double a, const float *p, const double *q, double *x,
-                       double *r, float *r32, double *rr) {
-    if (n <= 0) return;
-    d.dot_partial.ensure(kDotBlocks);
-    int nb, chunk;
-    dot_shape(n, nb, chunk);
-    k_pcg_update<<<nb, kBlock, 0, d.stream>>>(n, chunk, a, p, q, x, r, r32, d.dot_partial.ptr);
-    k_dot_final<<<1, kBlock, 0, d.stream>>>(nb, d.dot_partial.ptr, rr);
-    NSFEM_HIP(hipGetLastError());
-}
-
-namespace {
-template <typename A, typename B>
-void dot_any(Device &d, int n, const A *a, const B *b, double *result) {
-    if (n <= 0) return;
-    d.dot_partial.ensure(kDotBlocks);
-    int nb, chunk;
-    dot_shape(n, nb, chunk);
-    k_dot_any_partial<<<nb, kBlock, 0, d.stream>>>(n, chunk, a, b, d.dot_partial.ptr);
-    k_dot_final<<<1, kBlock, 0, d.stream>>>(nb, d.dot_partial.ptr, result);
-    NSFEM_HIP(hipGetLastError());
-}
-}  // namespace
-
-void launch_dot_accumulate(Device &d, int n, const double *a, const float *b, double *result) {
-    dot_any(d, n, a, b, result);
-}
-
-void launch_dot_accumulate(Device &d, int n, const float *a, const float *b, double *result) {
-    dot_any(d, n, a, b, result);
-}
-
-void launch_copy(Device &d, int n, const float *a, float *y) {
-    if (n <= 0) return;
-    k_convert<<<ew_grid(n), kBlock, 0, d.stream>>>(n, a, y);
-    NSFEM_HIP(hipGetLastError());
-}
-
-void launch_pcg_direction(Device &d, int n, const float *z, double b, float *p) {
-    if (n <= 0) return;
-    k_pcg_direction<<<ew_grid(n), kBlock, 0, d.stream>>>(n, z, b, p);
-    NSFEM_HIP(hipGetLastError());
 }
 
 void launch_scatter(Device &d, int count, const int32_t *idx, const double *val, double *dst) {
@@ -956,33 +1089,9 @@ void launch_add(Device &d, int n, const double *a, double *y) {
     NSFEM_HIP(hipGetLastError());
 }
 
-void launch_add(Device &d, int n, const float *a, float *y) {
-    if (n <= 0) return;
-    k_add<<<ew_grid(n), kBlock, 0, d.stream>>>(n, a, y);
-    NSFEM_HIP(hipGetLastError());
-}
-
-void launch_jacobi(Device &d, int n, double w, const double *dinv, const double *r, double *x) {
-    if (n <= 0) return;
-    k_jacobi<<<ew_grid(n), kBlock, 0, d.stream>>>(n, w, dinv, r, x);
-    NSFEM_HIP(hipGetLastError());
-}
-
-void launch_jacobi(Device &d, int n, double w, const float *dinv, const float *r, float *x) {
-    if (n <= 0) return;
-    k_jacobi<<<ew_grid(n), kBlock, 0, d.stream>>>(n, (float)w, dinv, r, x);
-    NSFEM_HIP(hipGetLastError());
-}
-
 void launch_jacobi0(Device &d, int n, double w, const double *dinv, const double *b, double *x) {
     if (n <= 0) return;
     k_jacobi0<<<ew_grid(n), kBlock, 0, d.stream>>>(n, w, dinv, b, x);
-    NSFEM_HIP(hipGetLastError());
-}
-
-void launch_jacobi0(Device &d, int n, double w, const float *dinv, const float *b, float *x) {
-    if (n <= 0) return;
-    k_jacobi0<<<ew_grid(n), kBlock, 0, d.stream>>>(n, (float)w, dinv, b, x);
     NSFEM_HIP(hipGetLastError());
 }
 

@@ -319,33 +319,74 @@ void launch_scatter(Device &d, int count, const int32_t *idx, const double *val,
 void launch_scatter_value(Device &d, int count, const int32_t *idx, double v,
                           double *dst);  // dst[idx[i]] = v
 void launch_scatter_value(Device &d, int count, const int32_t *idx, double v, float *dst);
-// The CG with FP32 directions and an FP32 preconditioner: x += a p and
-// r -= a q in FP64, r32 = (float) r, *rr += (r, r) (deterministic order, as
-// launch_dot_accumulate)
-void launch_pcg_update(Device &d, int n, double a, const float *p, const double *q, double *x,
-                       double *r, float *r32, double *rr);
-// y = A x with the FP32 copy of the values and FP32 x, products and sums in
-// FP64 (ensure_val32 first)
-void launch_spmv_acc64(Device &d, Matrix &m, const float *x, double *y);
-// *result += (a, b) accumulated in FP64 with FP32 operands widened
-void launch_dot_accumulate(Device &d, int n, const double *a, const float *b, double *result);
-void launch_dot_accumulate(Device &d, int n, const float *a, const float *b, double *result);
-void launch_copy(Device &d, int n, const float *src, float *dst);
-// p = z + b p, FP32 storage
-void launch_pcg_direction(Device &d, int n, const float *z, double b, float *p);
+// ---- CG with FP32 directions and an FP32 preconditioner, its scalars kept
+// on the device: (r, z) of the last two steps and the last (p, A p)
+struct PcgScalars {
+    double rz[2];
+    double pq;
+};
+// what the host reads after a step, in pinned memory
+struct PcgReport {
+    double rr, pq, rz;
+};
+struct PcgReportPage {
+    PcgReport *host = nullptr, *device = nullptr;
+    PcgReportPage() = default;
+    PcgReportPage(const PcgReportPage &) = delete;
+    PcgReportPage &operator=(const PcgReportPage &) = delete;
+    ~PcgReportPage() {
+        if (host) (void)hipHostFree(host);
+    }
+    void ensure() {
+        if (host) return;
+        void *h = nullptr, *dp = nullptr;
+        NSFEM_HIP(hipHostMalloc(&h, sizeof(PcgReport), hipHostMallocMapped));
+        host = static_cast<PcgReport *>(h);
+        NSFEM_HIP(hipHostGetDevicePointer(&dp, h, 0));
+        device = static_cast<PcgReport *>(dp);
+    }
+};
+struct PcgDevice {
+    DeviceArray<double> partial;  // a product's per-tile sums, then their folds
+    DeviceArray<PcgScalars> scalars;
+    PcgReportPage report;
+    int count = 0;                 // partials of the last product or sweep
+    const double *sums = nullptr;  // they, or their sum
+    void release() {
+        partial.release();
+        scalars.release();
+    }
+};
+void pcg_reserve(Device &d, const Matrix &m, PcgDevice &w);
+// r32 = r rounded to FP32, x0 = omega dinv r32
+void launch_pcg_round(Device &d, int n, const double *r, float *r32, const float *dinv,
+                      double omega, float *x0);
+// q = A p on the FP32 values, products and sums in FP64, and (p, q)'s partials
+void launch_pcg_product(Device &d, Matrix &m, const float *p, double *q, PcgDevice &w);
+// the preconditioner's last sweep (launch_sweep) and (r, y)'s partials
+void launch_pcg_sweep(Device &d, Matrix &m, double omega, const float *dinv, const float *x,
+                      const float *b, float *y, const double *r, PcgDevice &w);
+// step k's direction p = z + beta p from the sweep's partials
+void launch_pcg_direction(Device &d, int n, int k, const float *z, float *p, PcgDevice &w);
+// step k's update from the product's partials: x += alpha p, r -= alpha q,
+// r32 and x0 as launch_pcg_round; returns (r, r), (p, q) and (r, z) (one
+// host synchronisation).  Nothing is updated unless (p, q) and (r, z) > 0.
+PcgReport pcg_update(Device &d, int n, int k, const float *p, const double *q, double *x,
+                     double *r, float *r32, const float *dinv, double omega, float *x0,
+                     PcgDevice &w);
 void launch_add(Device &d, int n, const double *a, double *y);  // y += a
-void launch_add(Device &d, int n, const float *a, float *y);
-// x += w * dinv .* r
-void launch_jacobi(Device &d, int n, double w, const double *dinv, const double *r, double *x);
-void launch_jacobi(Device &d, int n, double w, const float *dinv, const float *r, float *x);
 // x = w * dinv .* b (the sweep from x = 0)
 void launch_jacobi0(Device &d, int n, double w, const double *dinv, const double *b, double *x);
-void launch_jacobi0(Device &d, int n, double w, const float *dinv, const float *b, float *x);
-// y = x + w * dinv .* (b - A x) in one product (y aliases neither x nor b)
-void launch_sweep(Device &d, Matrix &m, double w, const double *dinv, const double *x,
-                  const double *b, double *y);
-void launch_sweep(Device &d, Matrix &m, double w, const float *dinv, const float *x,
-                  const float *b, float *y);
+// y = x + w * dinv .* (b - A x) in one product (y aliases neither x nor b;
+// the FP32 form reads the FP32 copy of the values, as the next two do)
+template <typename T>
+void launch_sweep(Device &d, Matrix &m, double w, const T *dinv, const T *x, const T *b, T *y);
+// y += A x
+template <typename T>
+void launch_spmv_add(Device &d, Matrix &m, const T *x, T *y);
+// y = A x and y2 = w * dinv .* y
+template <typename T>
+void launch_restrict(Device &d, Matrix &m, const T *x, T *y, double w, const T *dinv, T *y2);
 void launch_fill(Device &d, int n, double v, float *y);
 // y = a rounded to FP32 / widened to FP64
 void launch_convert(Device &d, int n, const double *a, float *y);

@@ -171,6 +171,7 @@ struct Simulation {
     bool pmg = false;
     DeviceArray<double> pdinv, pr, pz, pp, pq, pt, pdot;
     DeviceArray<float> pdinv32, pb32, pz32, pt32, pp32;
+    PcgDevice pcg, vcg;  // scalars of the pressure's and the diffusion's FP32-cycle CG
     // the FP32 cycles of the pressure and the diffusion solves (fixed
     // kernels on fixed vectors), captured in a HIP graph on their first run
     // and replayed; dropped with their hierarchies
@@ -720,6 +721,7 @@ void release_pressure_multigrid(Simulation &s) {
     s.pmg = false;
     drop_graph(s.pcycle_graph);
     for (DeviceArray<float> *a : {&s.pdinv32, &s.pb32, &s.pz32, &s.pt32, &s.pp32}) a->release();
+    s.pcg.release();
     s.pdinv.release();
     s.pr.release();
     s.pz.release();
@@ -757,28 +759,36 @@ constexpr double kMgOmega = 0.8;
 constexpr int kMgMaxCycles = 30;
 
 // One V-cycle on A x = b over a level (A of n rows, its 1/diag, a residual
-// vector r) and the levels below it, m.lv[l] the next coarser, from x = 0
-// (zero: the first sweep needs no product) or from the x given: `sweeps`
-// damped Jacobi sweeps, the correction from the level below on the
-// restricted residual, as many sweeps after.  Each sweep with a product is
-// one fused launch (launch_sweep) from one of x and r into the other, so the
-// iterate alternates between them; the sweep from zero writes r, so that the
-// 2 sweeps - 1 moves after it end in x (from a given x: 2 sweeps moves).
+// vector r) and the levels below it, m.lv[l] the next coarser, from x = 0 or
+// from the x given: kMgSweeps damped Jacobi sweeps, the correction from the
+// level below on the restricted residual, as many sweeps after.  Each sweep
+// with a product is one fused launch (launch_sweep) from one of x and r into
+// the other, so the iterate alternates between them; from zero (kSwept) the
+// first sweep, which needs no product, is already in r: the kernel that made
+// b wrote it there.  The correction is added by the prolongation's product.
 // The deepest level
 // (l = m.lv.size()) is solved by its dense inverse when it has one, else by
 // FP64 CG to 1e-10 from zero.  T = float runs the whole cycle in FP32 (the
 // FP32 copies of every level's values and vectors, ensure_fp32_levels; it
-// needs the dense deepest level).
+// needs the dense deepest level).  `last_sweep`, if given, launches the last
+// sweep in launch_sweep's place.
+enum class CycleStart { kSwept, kGiven };
+
 template <typename T>
+struct NoLastSweep {
+    bool operator()(const T *, T *) const { return false; }
+};
+
+template <typename T, class Last = NoLastSweep<T>>
 void mg_cycle(Device &d, Matrix &A, int n, const T *dinv, T *r, MgLevels &m, size_t l,
-              const T *b, T *x, bool zero = true, int sweeps = kMgSweeps,
-              double omega = kMgOmega) {
+              const T *b, T *x, CycleStart start, double omega = kMgOmega,
+              const Last &last_sweep = Last()) {
     if (l == m.lv.size() && m.deep_ok) {
         launch_dense(d, n, deep_inverse<T>(m), b, x);
         return;
     }
-    if (l == m.lv.size() || (zero && sweeps == 0)) launch_fill(d, n, 0.0, x);
     if (l == m.lv.size()) {
+        launch_fill(d, n, 0.0, x);
         if constexpr (std::is_same<T, double>::value) {
             CgRequest rq{};
             rq.m = &A;
@@ -796,26 +806,26 @@ void mg_cycle(Device &d, Matrix &A, int n, const T *dinv, T *r, MgLevels &m, siz
         return;
     }
     // the iterate in cur, the other vector free; a fused sweep moves it across
-    T *cur = x, *spare = r;
+    T *cur = start == CycleStart::kSwept ? r : x, *spare = start == CycleStart::kSwept ? x : r;
     auto sweep = [&] {
-        launch_sweep(d, A, omega, dinv, cur, b, spare);
+        launch_sweep(d, A, omega, dinv, (const T *)cur, b, spare);
         std::swap(cur, spare);
     };
-    if (zero && sweeps > 0) {
-        std::swap(cur, spare);
-        launch_jacobi0(d, n, omega, dinv, b, cur);
-        for (int k = 1; k < sweeps; ++k) sweep();
-    } else {
-        for (int k = 0; k < sweeps; ++k) sweep();
-    }
+    for (int k = start == CycleStart::kSwept ? 1 : 0; k < kMgSweeps; ++k) sweep();
     launch_spmv(d, A, cur, b, spare, 1);
     MgLevel &below = *m.lv[l];
     const LevelVectors<T> v(below);
-    launch_spmv(d, below.PT, spare, nullptr, v.b, 0);
-    mg_cycle<T>(d, below.A, below.n, v.dinv, v.r, m, l + 1, v.b, v.x);
-    launch_spmv(d, below.P, v.x, nullptr, spare, 0);
-    launch_add(d, n, spare, cur);
-    for (int k = 0; k < sweeps; ++k) sweep();
+    if (l + 1 == m.lv.size())
+        launch_spmv(d, below.PT, spare, nullptr, v.b, 0);
+    else
+        launch_restrict(d, below.PT, (const T *)spare, v.b, kMgOmega, v.dinv, v.r);
+    mg_cycle<T>(d, below.A, below.n, v.dinv, v.r, m, l + 1, v.b, v.x, CycleStart::kSwept);
+    launch_spmv_add(d, below.P, (const T *)v.x, cur);
+    for (int k = 0; k + 1 < kMgSweeps; ++k) sweep();
+    if (last_sweep(cur, spare))
+        std::swap(cur, spare);
+    else
+        sweep();
     if (cur != x) fail(NSFEM_ERROR, "V-cycle: the sweeps did not end in the iterate's vector");
 }
 
@@ -840,11 +850,10 @@ void ensure_fp32_levels(Device &d, MgLevels &m) {
 // The pressure coarse space (present while has_coarse).
 MgLevel &coarse(Simulation &s) { return *s.mg.lv[0]; }
 
-// One V-cycle from the pressure coarse level down, from zero or from the x
-// given.
-void vcycle(Simulation &s, const double *b, double *x, bool zero) {
+// One V-cycle from the pressure coarse level down, from the x given.
+void vcycle(Simulation &s, const double *b, double *x) {
     MgLevel &C = coarse(s);
-    mg_cycle<double>(*s.dev, C.A, s.nc, C.dinv.ptr, C.r.ptr, s.mg, 1, b, x, zero);
+    mg_cycle<double>(*s.dev, C.A, s.nc, C.dinv.ptr, C.r.ptr, s.mg, 1, b, x, CycleStart::kGiven);
 }
 
 // V-cycles on A_c e = cr from the current e; returns the status, the cycle
@@ -861,7 +870,7 @@ int mg_solve(Simulation &s, int64_t *cycles, double *seconds) {
         status = NSFEM_OK;  // e = projection guess of a zero right-hand side
     } else {
         while (k < kMgMaxCycles) {
-            vcycle(s, C.b.ptr, C.x.ptr, false);
+            vcycle(s, C.b.ptr, C.x.ptr);
             ++k;
             launch_spmv(d, C.A, C.x.ptr, C.b.ptr, C.r.ptr, 1);
             const double rr = dev_dot(d, s.cproj, C.r.ptr, C.r.ptr);
@@ -989,8 +998,9 @@ void run_captured(Device &d, hipGraphExec_t &exec, F launches) {
 // those rows at their values).
 void fine_vcycle(Simulation &s, const double *r, double *z) {
     Device &d = *s.dev;
+    launch_jacobi0(d, s.P, kMgOmega, s.pdinv.ptr, r, s.pt.ptr);
     mg_cycle<double>(d, s.mats[NSFEM_PRESSURE_STIFFNESS], s.P, s.pdinv.ptr, s.pt.ptr, s.mg, 0, r,
-                     z);
+                     z, CycleStart::kSwept);
     launch_scatter_value(d, s.npb, s.pb_idx.ptr, 0.0, z);
 }
 
@@ -1009,19 +1019,28 @@ void ensure_pressure_fp32(Simulation &s) {
     const int n = s.P;
     ensure_fp32_levels(d, s.mg);
     ensure_val32(d, s.mats[NSFEM_PRESSURE_STIFFNESS]);
+    pcg_reserve(d, s.mats[NSFEM_PRESSURE_STIFFNESS], s.pcg);
     s.pdinv32.resize((size_t)n);
     launch_convert(d, n, s.pdinv.ptr, s.pdinv32.ptr);
     for (DeviceArray<float> *a : {&s.pb32, &s.pz32, &s.pt32, &s.pp32}) a->resize((size_t)n);
 }
 
-// z = M r in FP32 on the fixed vectors r = pb32, z = pz32 (captured)
+// z = M r in FP32 on the fixed vectors r = pb32 with its first sweep in pt32,
+// z = pz32 (captured), and the partials of (r, z).  r is 0 on the Dirichlet
+// rows, so their z (zeroed after the last sweep) adds nothing to them.
 void fine_vcycle32(Simulation &s) {
     Device &d = *s.dev;
+    Matrix &A = s.mats[NSFEM_PRESSURE_STIFFNESS];
     run_captured(d, s.pcycle_graph, [&] {
-        mg_cycle<float>(d, s.mats[NSFEM_PRESSURE_STIFFNESS], s.P, s.pdinv32.ptr, s.pt32.ptr, s.mg,
-                        0, s.pb32.ptr, s.pz32.ptr);
+        mg_cycle<float>(d, A, s.P, s.pdinv32.ptr, s.pt32.ptr, s.mg, 0, s.pb32.ptr, s.pz32.ptr,
+                        CycleStart::kSwept, kMgOmega, [&](const float *x, float *y) {
+                            launch_pcg_sweep(d, A, kMgOmega, s.pdinv32.ptr, x, s.pb32.ptr, y,
+                                             s.pr.ptr, s.pcg);
+                            return true;
+                        });
         launch_scatter_value(d, s.npb, s.pb_idx.ptr, 0.0, s.pz32.ptr);
     });
+    s.pcg.count = A.n_tiles;  // a replay launches without the host's part
 }
 
 // a . b over n entries, through a one-entry device scratch (one host
@@ -1097,16 +1116,6 @@ int pcg_run(Device &d, Matrix &A, int n, const double *b, double *x, const PcgWo
     return status;
 }
 
-// Reads a device scalar accumulated by the dot launchers (one host
-// synchronisation) and clears it for the next.
-double take_scalar(Device &d, double *dot) {
-    double h = 0.0;
-    NSFEM_HIP(hipMemcpyAsync(&h, dot, sizeof(double), hipMemcpyDeviceToHost, d.stream));
-    NSFEM_HIP(hipStreamSynchronize(d.stream));
-    launch_fill(d, 1, 0.0, dot);
-    return h;
-}
-
 // pcg_run with an FP32 preconditioner z32 = precond(r32) and FP32
 // directions: p in FP32, q = A p on the FP32 values with every product and
 // sum in FP64 (an FP32 sum would cancel away smooth directions' products on
@@ -1122,14 +1131,31 @@ double take_scalar(Device &d, double *dot) {
 // tolerance where the recursion had met it, or after kPcgIterationsMax
 // iterations (the V-cycle preconditioned solves take tens); x is then the
 // last iterate, for the FP64 form to finish.
+//
+// The coefficients stay on the device: the product and the preconditioner's
+// last sweep leave the partials of (p, q) and (r, z), which the update and
+// the direction add for themselves, and the host waits once an iteration,
+// for (r, r).  With each dot a pass of its own, two launches, a copy and a
+// wait, the host's three waits and the launches around them were most of an
+// iteration on small grids: eight steps on the 200^2 cavity took 35.1 ms,
+// 26.0 here.
 constexpr int kPcgRecomputeMax = 8;
 constexpr double kPcgUpdateDrop = 1e3;
 constexpr int64_t kPcgIterationsMax = 500;
 
+// Vectors of the FP32 side: the rounded residual, its first Jacobi sweep
+// (omega dinv r32), the preconditioned residual, the direction.
+struct Pcg32Work {
+    float *r32, *x0, *z, *p;
+    const float *dinv;
+    double omega;
+    PcgDevice &dev;
+};
+
 template <class Pre>
 int pcg_run32(Device &d, Matrix &A, int n, const double *b, double *x, const PcgWork &w,
-              float *r32, float *z32, float *p, double rtol, int64_t max_iterations,
-              Pre precond, SolveOut &o, int c) {
+              const Pcg32Work &f, double rtol, int64_t max_iterations, Pre precond, SolveOut &o,
+              int c) {
     const auto t0 = std::chrono::steady_clock::now();
     double *r = w.r, *q = w.q;
     const double bb = vec_dot(d, n, b, b, w.dot);
@@ -1144,29 +1170,23 @@ int pcg_run32(Device &d, Matrix &A, int n, const double *b, double *x, const Pcg
     double rr_true = rr;  // the last recomputed residual
     if (rr > tol2) {
         status = NSFEM_MAX_ITERATIONS_REACHED;
-        launch_fill(d, 1, 0.0, w.dot);
-        launch_convert(d, n, r, r32);
-        precond(r32, z32);
-        launch_copy(d, n, z32, p);
-        launch_dot_accumulate(d, n, r, z32, w.dot);
-        double rz = take_scalar(d, w.dot);
+        launch_pcg_round(d, n, r, f.r32, f.dinv, f.omega, f.x0);
         while (k < max_iter) {
-            launch_spmv_acc64(d, A, p, q);
-            launch_dot_accumulate(d, n, q, p, w.dot);
-            const double pq = take_scalar(d, w.dot);
-            if (!(pq > 0.0) || !(rz > 0.0)) {
+            precond();
+            launch_pcg_direction(d, n, (int)k, f.z, f.p, f.dev);
+            launch_pcg_product(d, A, f.p, q, f.dev);
+            const PcgReport got = pcg_update(d, n, (int)k, f.p, q, x, r, f.r32, f.dinv, f.omega,
+                                             f.x0, f.dev);
+            if (!(got.pq > 0.0) || !(got.rz > 0.0)) {
                 status = NSFEM_BREAKDOWN;
                 break;
             }
-            const double alpha = rz / pq;
-            launch_pcg_update(d, n, alpha, p, q, x, r, r32, w.dot);
-            rr = take_scalar(d, w.dot);
+            rr = got.rr;
             ++k;
             const bool met = rr <= tol2;
             if (met || rr * kPcgUpdateDrop * kPcgUpdateDrop <= rr_true) {
                 launch_spmv(d, A, x, b, r, 1);
-                launch_dot_accumulate(d, n, r, r, w.dot);
-                rr = take_scalar(d, w.dot);
+                rr = vec_dot(d, n, r, r, w.dot);
                 rr_true = rr;
                 if (rr <= tol2) {
                     status = NSFEM_OK;
@@ -1176,18 +1196,12 @@ int pcg_run32(Device &d, Matrix &A, int n, const double *b, double *x, const Pcg
                     status = NSFEM_STAGNATION;
                     break;
                 }
-                launch_convert(d, n, r, r32);
+                launch_pcg_round(d, n, r, f.r32, f.dinv, f.omega, f.x0);
             }
             if (k >= kPcgIterationsMax) {
                 status = NSFEM_STAGNATION;
                 break;
             }
-            precond(r32, z32);
-            launch_dot_accumulate(d, n, r, z32, w.dot);
-            const double rz_new = take_scalar(d, w.dot);
-            const double beta = rz_new / rz;
-            rz = rz_new;
-            launch_pcg_direction(d, n, z32, beta, p);
         }
     }
     o.iters[c] = k;
@@ -1209,9 +1223,10 @@ void pcg_pressure(Simulation &s, SolveOut &o) {
     SolveOut first{};
     if (pressure_cycle_fp32(s)) {
         ensure_pressure_fp32(s);
-        status = pcg_run32(d, A, s.P, s.prhs.ptr, s.p.ptr, w, s.pb32.ptr, s.pz32.ptr, s.pp32.ptr,
-                           s.opt.rtol, s.opt.max_iterations,
-                           [&](const float *, float *) { fine_vcycle32(s); }, o, 0);
+        const Pcg32Work f{s.pb32.ptr,    s.pt32.ptr, s.pz32.ptr, s.pp32.ptr,
+                          s.pdinv32.ptr, kMgOmega,   s.pcg};
+        status = pcg_run32(d, A, s.P, s.prhs.ptr, s.p.ptr, w, f, s.opt.rtol, s.opt.max_iterations,
+                           [&] { fine_vcycle32(s); }, o, 0);
     }
     if (!pressure_cycle_fp32(s) || status == NSFEM_STAGNATION) {
         // FP64 throughout (from the last iterate when the FP32 form stalled)
@@ -1248,8 +1263,9 @@ bool velocity_cycle_fp32(const Simulation &s) {
 
 void velocity_vcycle(Simulation &s, const double *r, double *z) {
     Device &d = *s.dev;
-    mg_cycle<double>(d, s.mats[NSFEM_DIFFUSION], s.V, s.vdinv.ptr, s.vt.ptr, s.vmg, 0, r, z, true,
-                     kMgSweeps, kVmgFineOmega);
+    launch_jacobi0(d, s.V, kVmgFineOmega, s.vdinv.ptr, r, s.vt.ptr);
+    mg_cycle<double>(d, s.mats[NSFEM_DIFFUSION], s.V, s.vdinv.ptr, s.vt.ptr, s.vmg, 0, r, z,
+                     CycleStart::kSwept, kVmgFineOmega);
     launch_scatter_value(d, s.nvb, s.vb_idx.ptr, 0.0, z);
 }
 
@@ -1261,19 +1277,28 @@ void ensure_velocity_fp32(Simulation &s) {
     const int V = s.V;
     ensure_fp32_levels(d, s.vmg);
     ensure_val32(d, s.mats[NSFEM_DIFFUSION]);
+    pcg_reserve(d, s.mats[NSFEM_DIFFUSION], s.vcg);
     s.vdinv32.resize((size_t)V);
     launch_convert(d, V, s.vdinv.ptr, s.vdinv32.ptr);
     for (DeviceArray<float> *a : {&s.vb32, &s.vz32, &s.vt32, &s.vp32}) a->resize((size_t)V);
 }
 
-// z = M r in FP32 on the fixed vectors r = vb32, z = vz32 (captured)
+// z = M r in FP32 on the fixed vectors r = vb32 with its first sweep in vt32,
+// z = vz32 (captured), and the partials of (r, z).  On the Dirichlet rows
+// (identity rows, r = 0 there and the prolongation's rows empty) every sweep
+// and the correction leave z at 0.
 void velocity_vcycle32(Simulation &s) {
     Device &d = *s.dev;
+    Matrix &A = s.mats[NSFEM_DIFFUSION];
     run_captured(d, s.vcycle_graph, [&] {
-        mg_cycle<float>(d, s.mats[NSFEM_DIFFUSION], s.V, s.vdinv32.ptr, s.vt32.ptr, s.vmg, 0,
-                        s.vb32.ptr, s.vz32.ptr, true, kMgSweeps, kVmgFineOmega);
-        launch_scatter_value(d, s.nvb, s.vb_idx.ptr, 0.0, s.vz32.ptr);
+        mg_cycle<float>(d, A, s.V, s.vdinv32.ptr, s.vt32.ptr, s.vmg, 0, s.vb32.ptr, s.vz32.ptr,
+                        CycleStart::kSwept, kVmgFineOmega, [&](const float *x, float *y) {
+                            launch_pcg_sweep(d, A, kVmgFineOmega, s.vdinv32.ptr, x, s.vb32.ptr, y,
+                                             s.vr.ptr, s.vcg);
+                            return true;
+                        });
     });
+    s.vcg.count = A.n_tiles;  // a replay launches without the host's part
 }
 
 // Column c (0: u, 1: v) of the diffusion solve by CG preconditioned with
@@ -1289,9 +1314,10 @@ void pcg_velocity(Simulation &s, int c, SolveOut &o) {
     SolveOut first{};
     if (velocity_cycle_fp32(s)) {
         ensure_velocity_fp32(s);
-        status = pcg_run32(d, A, s.V, s.rhs.ptr + off, x, w, s.vb32.ptr, s.vz32.ptr, s.vp32.ptr,
-                           s.opt.rtol, s.opt.max_iterations,
-                           [&](const float *, float *) { velocity_vcycle32(s); }, o, 0);
+        const Pcg32Work f{s.vb32.ptr,    s.vt32.ptr,    s.vz32.ptr, s.vp32.ptr,
+                          s.vdinv32.ptr, kVmgFineOmega, s.vcg};
+        status = pcg_run32(d, A, s.V, s.rhs.ptr + off, x, w, f, s.opt.rtol, s.opt.max_iterations,
+                           [&] { velocity_vcycle32(s); }, o, 0);
     }
     if (!velocity_cycle_fp32(s) || status == NSFEM_STAGNATION) {
         // FP64 throughout (from the last iterate when the FP32 form stalled)
@@ -1520,6 +1546,7 @@ void release_velocity_multigrid(Simulation &s) {
     for (DeviceArray<double> *a : {&s.vdinv, &s.vr, &s.vz, &s.vp, &s.vq, &s.vt, &s.vdot})
         a->release();
     for (DeviceArray<float> *a : {&s.vdinv32, &s.vb32, &s.vz32, &s.vt32, &s.vp32}) a->release();
+    s.vcg.release();
     for (int c = 0; c < 2; ++c)
         for (int w = 0; w < 2; ++w) {
             s.vmg_sec[c][w] = 0.0;
