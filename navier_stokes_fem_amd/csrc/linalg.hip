@@ -198,6 +198,48 @@ void set_group_loads(Matrix &m) {
 
 }  // namespace
 
+namespace {
+// out = {most nonzeros of a row, most columns below and above the diagonal}
+// (columns ascend within a row)
+__global__ void k_row_shape(int rows, const int32_t *__restrict__ rs,
+                            const int32_t *__restrict__ col, int *__restrict__ out) {
+    int nz = 0, lo = 0, hi = 0;
+    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
+        const int a = rs[r], b = rs[r + 1];
+        if (a == b) continue;
+        nz = max(nz, b - a);
+        lo = max(lo, r - col[a]);
+        hi = max(hi, col[b - 1] - r);
+    }
+    for (int o = 32; o >= 1; o >>= 1) {
+        nz = max(nz, __shfl_xor(nz, o, 64));
+        lo = max(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(out, nz);
+        atomicMax(out + 1, lo);
+        atomicMax(out + 2, hi);
+    }
+}
+
+void row_shape(Matrix &m) {
+    int h[3] = {0, 0, 0};
+    if (m.rows == m.cols && m.nnz > 0) {
+        DeviceArray<int> out;
+        out.resize(3);
+        NSFEM_HIP(hipMemset(out.ptr, 0, sizeof(h)));
+        k_row_shape<<<std::max(1, std::min((m.rows + 255) / 256, 1024)), 256>>>(
+            m.rows, m.row_start.ptr, m.col.ptr, out.ptr);
+        NSFEM_HIP(hipGetLastError());
+        NSFEM_HIP(hipMemcpy(h, out.ptr, sizeof(h), hipMemcpyDeviceToHost));
+    }
+    m.max_row_nz = h[0];
+    m.band_lo = h[1];
+    m.band_hi = h[2];
+}
+}  // namespace
+
 void build_tiles(Matrix &m, const std::vector<int32_t> &rs) {
     std::vector<int32_t> t = cut_rows(rs, m.rows, kTileRows, kSpmvTileNnz);
     m.n_tiles = (int)t.size() - 1;
@@ -209,6 +251,7 @@ void build_tiles(Matrix &m, const std::vector<int32_t> &rs) {
     NSFEM_HIP(hipMemcpy(m.tiles.ptr, meta.data(), meta.size() * sizeof(int4),
                         hipMemcpyHostToDevice));
     m.bcol_ok = col_delta(m, m.n_tiles, m.tiles.ptr, m.bcol);
+    row_shape(m);
     build_wave_tiles(m, kWaveRows, kStageNnz);
 }
 
@@ -220,6 +263,8 @@ void build_wave_tiles(Matrix &m, int rows, int nnz) {
     m.wave_nnz = nnz;
     std::vector<int32_t> w = cut_rows(rs, m.rows, rows, nnz);
     m.n_wtiles = (int)w.size() - 1;
+    m.host_wtiles = w;
+    for (auto &plan : m.res_plan) plan = ResidentPlan{};
     m.host_wtile_prefix.assign(w.size(), 0);
     for (int i = 0; i < m.n_wtiles; ++i)
         m.host_wtile_prefix[i + 1] =
@@ -243,14 +288,10 @@ void build_wave_tiles(Matrix &m, int rows, int nnz) {
     set_group_loads(m);
 }
 
-// Persistent blocks own contiguous wave-tile ranges balanced by (nnz + rows).
-// The table lives in arrays sized for the largest grid at tiling time, so
-// this only computes and copies.
-void ensure_block_tiles(Device &d, Matrix &m, int grid) {
-    NSFEM_REQUIRE(grid >= 1 && grid <= kMaxGridBlocks, NSFEM_ERROR, "grid size out of range");
-    if (m.block_tiles_grid == grid) return;
-    std::vector<int32_t> &bt = m.host_block_tiles;
-    bt.resize((size_t)grid + 1);  // within the reserved capacity
+namespace {
+// Contiguous wave-tile ranges of `grid` blocks, balanced by (nnz + rows).
+void split_tiles(const Matrix &m, int grid, std::vector<int32_t> &bt) {
+    bt.resize((size_t)grid + 1);
     const int64_t total = m.host_wtile_prefix[m.n_wtiles];
     int t = 0;
     for (int b = 0; b <= grid; ++b) {
@@ -260,6 +301,16 @@ void ensure_block_tiles(Device &d, Matrix &m, int grid) {
     }
     bt[0] = 0;
     bt[grid] = m.n_wtiles;
+}
+}  // namespace
+
+// The persistent blocks' tiles.  The table lives in arrays sized for the
+// largest grid at tiling time, so this only computes and copies.
+void ensure_block_tiles(Device &d, Matrix &m, int grid) {
+    NSFEM_REQUIRE(grid >= 1 && grid <= kMaxGridBlocks, NSFEM_ERROR, "grid size out of range");
+    if (m.block_tiles_grid == grid) return;
+    std::vector<int32_t> &bt = m.host_block_tiles;
+    split_tiles(m, grid, bt);  // within the reserved capacity
     NSFEM_HIP(hipMemcpyAsync(m.block_tiles.ptr, bt.data(), bt.size() * sizeof(int32_t),
                              hipMemcpyHostToDevice, d.stream));
     NSFEM_HIP(hipStreamSynchronize(d.stream));
@@ -1176,6 +1227,7 @@ namespace {
 constexpr int kGroup = 16;
 constexpr int kMaxGroups = kMaxGridBlocks / kGroup;
 constexpr int kFlatMax = 128;
+constexpr int kResMaxBlocks = 256;  // blocks of a resident solve
 
 struct alignas(256) SyncState {
     unsigned int arrive_top;
@@ -1193,6 +1245,9 @@ struct alignas(256) SyncState {
     // only after every block has posted the next epoch, i.e. has read them)
     unsigned int flag[kFlatMax];
     double fpart[2][kMaxRed][kFlatMax];
+    // resident solves: per epoch parity, sum and block the two halves of the
+    // block's partial sum, each tagged with the epoch
+    unsigned long long tag[2][kMaxRed][kResMaxBlocks][2];
 };
 
 #ifdef NSFEM_CG_TRACE
@@ -1237,7 +1292,7 @@ namespace {
 #endif
 
 struct CgArgs {
-    int n;
+    int n, nnz;
     const int4 *meta;  // wave tile descriptors
     const int32_t *tiles;
     const int32_t *block_tiles;
@@ -1266,6 +1321,9 @@ struct CgArgs {
     // (r_scaled = scale * (b - A x)), so convergence is decided on the
     // unscaled residual, as without scaling.
     const double *scale;
+    // resident solves: the matrix's bandwidths below and above the diagonal,
+    // and the most rows a block's window holds
+    int band_lo, band_hi, win_cap;
 };
 
 // The FP64 step of x_row along the scaled search direction: x = D^-1/2 y.
@@ -1273,9 +1331,14 @@ __device__ __forceinline__ double x_step(const CgArgs &A, double pend, int row) 
     return A.scale ? pend * A.scale[row] : pend;
 }
 
-// Launched with at least kFlatMax threads.
-__global__ void k_sync_reset(SyncState *s, int ngroups) {
+// Launched with at least kFlatMax threads; blocks > 0 clears that many blocks'
+// tags too (a resident solve; a tag's epoch is never 0).
+__global__ void k_sync_reset(SyncState *s, int ngroups, int blocks) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int k = i; k < 4 * kMaxRed * blocks; k += gridDim.x * blockDim.x) {
+        const int half = k & 1, b = (k >> 1) % blocks, j = (k >> 1) / blocks;
+        s->tag[j / kMaxRed][j % kMaxRed][b][half] = 0ull;
+    }
     if (i == 0) {
         s->arrive_top = 0;
         s->abort = 0;
@@ -2427,92 +2490,165 @@ __device__ void flush_x1(const CgArgs &A, int R0, int R1, const void *st, double
         A.x[row] = __builtin_fma(x_step(A, pend, row), (double)ld_state(st, row).p, A.x[row]);
 }
 
-// Control state of a one-column solve, in LDS: thread 0 updates it after
-// every grid reduction and the block reads the step coefficients from it,
-// so the bookkeeping holds no registers during the phases.
-struct CgCtl1 {
-    double tol2, gamma, rmax2, last_rr, ru_rr, rho;
-    double pend, alpha, beta, g;
-    int iters, status, stall, active, dropped;
-    int k, last_ru, refines, ru, has_pend, out_of_iters;
+// Control state of a single-reduction solve, in LDS: thread 0 updates it after
+// every grid reduction and the block reads the step coefficients from it, so
+// the bookkeeping holds no registers during the phases.  Two columns share
+// one iteration count and reliable updates (a column that did not ask for one
+// gets it too).
+template <int NC>
+struct CgCtl {
+    double tol2[NC], gamma[NC], rmax2[NC], last_rr[NC], ru_rr[NC], rho[NC];
+    double pend[NC], alpha[NC], beta[NC], g[NC];
+    int iters[NC], status[NC], stall[NC], active[NC], dropped[NC];
+    int k, last_ru, refines, ru, has_pend, out_of_iters, any;
 };
+
+// After the set-up residual: acc[c] = (r, r) in FP64, acc[NC + c] = (b, b),
+// acc[2 NC + c] = (r, r) of the stored r.
+template <int NC>
+__device__ void ctl_start(CgCtl<NC> &C, const CgArgs &A, const double (&acc)[3 * NC], bool writer) {
+    C.any = 0;
+    for (int c = 0; c < NC; ++c) {
+        const double bn = sqrt(acc[NC + c]), r0n = sqrt(acc[c]);
+        const double ref = bn > 0.0 ? bn : r0n;
+        const double tol = fmax(A.rtol * ref, A.atol);
+        C.tol2[c] = tol * tol;
+        C.active[c] = acc[c] > C.tol2[c];
+        C.any = C.any || C.active[c];
+        C.gamma[c] = acc[2 * NC + c];
+        // the drop triggers compare the recursion with the true residual in
+        // the iteration's (scaled) space; rho converts a scaled norm into
+        // the unscaled one the tolerance is on
+        C.rmax2[c] = A.scale ? acc[2 * NC + c] : acc[c];
+        C.last_rr[c] = C.ru_rr[c] = acc[c];
+        C.rho[c] = A.scale && acc[2 * NC + c] > 0.0 ? acc[c] / acc[2 * NC + c] : 1.0;
+        C.g[c] = 0.0;
+        C.iters[c] = 0;
+        C.status[c] = NSFEM_OK;
+        C.stall[c] = C.dropped[c] = 0;
+        C.pend[c] = C.alpha[c] = C.beta[c] = 0.0;
+        if (writer) {
+            A.res[c].rhs_norm = bn;
+            A.res[c].initial_residual = r0n;
+            A.res[c].tolerance = tol;
+        }
+    }
+    C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = 0;
+}
 
 // After the phase reduction: alpha_k, gamma_{k+1} and the reliable-update
 // trigger.  A drop of the recursive residual by rdelta triggers the update
 // once ru_min_gap iterations have passed, a drop by rdelta^2 at once (FP32
 // rounding must not pile up over a steep fall); ru_gap iterations and the
-// iteration limit force one.
-__device__ void ctl_after_phase(CgCtl1 &C, const CgArgs &A, const double (&sums)[4]) {
+// iteration limit force one.  sums[4 c ...] = (p, q), (r, r), (r, q), (q, q).
+// MIXED = false (FP64): no updates; a column is done when its recursive
+// residual meets the tolerance.
+template <int NC, bool MIXED = true>
+__device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&sums)[4 * NC]) {
     const int k = ++C.k;
-    double alpha = 0.0, g = 0.0;
-    bool dropped = false;
-    if (C.active) {
-        const double delta = sums[0], gk = sums[1];
-        if (!(delta > 0.0)) {
-            C.status = NSFEM_BREAKDOWN;
-            C.active = 0;
-            C.last_rr = gk;
-        } else {
-            alpha = gk / delta;
-            g = fmax(gk - 2.0 * alpha * sums[2] + alpha * alpha * sums[3], 0.0);
-            C.gamma = gk;
-            C.iters = k;
-            const double d2 = A.rdelta * A.rdelta;
-            dropped = g * C.rho <= C.tol2 ||
-                      (g < d2 * C.rmax2 && (k - C.last_ru >= A.ru_min_gap || g < d2 * d2 * C.rmax2));
+    const double d2 = A.rdelta * A.rdelta;
+    bool want = false, any = false;
+    for (int c = 0; c < NC; ++c) {
+        double alpha = 0.0, g = 0.0;
+        bool dropped = false;
+        if (C.active[c]) {
+            const double delta = sums[4 * c], gk = sums[4 * c + 1];
+            if (!(delta > 0.0)) {
+                C.status[c] = NSFEM_BREAKDOWN;
+                C.active[c] = 0;
+                C.last_rr[c] = gk;
+            } else {
+                alpha = gk / delta;
+                // gk - 2 alpha (r, q) + alpha^2 (q, q), its roundings spelt out:
+                // the same bits in every kernel this is inlined into
+                g = fmax(__builtin_fma(alpha * alpha, sums[4 * c + 3],
+                                       __builtin_fma(-2.0 * alpha, sums[4 * c + 2], gk)),
+                         0.0);
+                C.gamma[c] = gk;
+                C.iters[c] = k;
+                if (MIXED) {
+                    dropped = g * C.rho[c] <= C.tol2[c] ||
+                              (g < d2 * C.rmax2[c] &&
+                               (k - C.last_ru >= A.ru_min_gap || g < d2 * d2 * C.rmax2[c]));
+                } else if (g <= C.tol2[c]) {
+                    C.active[c] = 0;  // its last step is still pending
+                    C.last_rr[c] = g;
+                }
+            }
         }
+        want = want || dropped;
+        any = any || C.active[c];
+        C.pend[c] = alpha;
+        C.alpha[c] = alpha;
+        C.g[c] = g;
+        C.dropped[c] = dropped;
     }
-    C.pend = alpha;
-    C.alpha = alpha;
-    C.g = g;
-    C.dropped = dropped;
     C.has_pend = 1;
     C.out_of_iters = k >= A.max_iter;
-    C.ru = C.active && (dropped || k - C.last_ru >= A.ru_gap || C.out_of_iters);
+    C.ru = MIXED && any && (want || k - C.last_ru >= A.ru_gap || C.out_of_iters);
     if (C.ru) C.last_ru = k;
 }
 
-// After a reliable update (x flushed, r := b - A x in FP64): the FP64
-// residual decides convergence; after a drop reported by the recursion the
-// FP64 residual must fall below (1 + rdelta)/2 of its best value so far, and
-// three misses in a row end the FP32 iteration (stagnation; an update
-// forced by ru_gap alone is not judged).
-__device__ void ctl_after_update(CgCtl1 &C, const CgArgs &A, const double (&ra)[3]) {
+// After a reliable update (x flushed, r := b - A x in FP64; ra as ctl_start's
+// acc): the FP64 residual decides convergence; after a drop reported by the
+// recursion the FP64 residual must fall below (1 + rdelta)/2 of its best
+// value so far, and three misses in a row end the FP32 iteration
+// (stagnation; an update forced by ru_gap alone is not judged).
+template <int NC>
+__device__ void ctl_after_update(CgCtl<NC> &C, const CgArgs &A, const double (&ra)[3 * NC]) {
     C.has_pend = 0;
-    C.pend = 0.0;
-    C.alpha = 0.0;
     ++C.refines;
-    C.last_rr = ra[0];
-    if (ra[0] <= C.tol2) {
-        C.active = 0;
-    } else {
-        C.g = ra[2];
-        C.rmax2 = A.scale ? ra[2] : ra[0];
-        C.rho = A.scale && ra[2] > 0.0 ? ra[0] / ra[2] : 1.0;
-        if (C.dropped) {
-            const double sr = 0.5 * (1.0 + A.rdelta);
-            C.stall = ra[0] > sr * sr * C.ru_rr ? C.stall + 1 : 0;
+    for (int c = 0; c < NC; ++c) {
+        C.pend[c] = 0.0;
+        C.alpha[c] = 0.0;
+        C.last_rr[c] = ra[c];
+        if (!C.active[c]) continue;
+        if (ra[c] <= C.tol2[c]) {
+            C.active[c] = 0;
+            continue;
         }
-        C.ru_rr = fmin(C.ru_rr, ra[0]);
-        if (C.stall >= 3) {
-            C.status = NSFEM_STAGNATION;
-            C.active = 0;
+        C.g[c] = ra[2 * NC + c];
+        C.rmax2[c] = A.scale ? ra[2 * NC + c] : ra[c];
+        C.rho[c] = A.scale && ra[2 * NC + c] > 0.0 ? ra[c] / ra[2 * NC + c] : 1.0;
+        if (C.dropped[c]) {
+            const double sr = 0.5 * (1.0 + A.rdelta);
+            C.stall[c] = ra[c] > sr * sr * C.ru_rr[c] ? C.stall[c] + 1 : 0;
+        }
+        C.ru_rr[c] = fmin(C.ru_rr[c], ra[c]);
+        if (C.stall[c] >= 3) {
+            C.status[c] = NSFEM_STAGNATION;
+            C.active[c] = 0;
         } else if (C.refines >= A.max_refine) {
-            C.status = NSFEM_MAX_ITERATIONS_REACHED;
-            C.active = 0;
+            C.status[c] = NSFEM_MAX_ITERATIONS_REACHED;
+            C.active[c] = 0;
         }
     }
 }
 
 // End of an iteration: iteration limit, beta_{k+1} = gamma_{k+1} / gamma_k.
-__device__ void ctl_end(CgCtl1 &C) {
-    if (C.active && C.out_of_iters) {
-        C.status = NSFEM_MAX_ITERATIONS_REACHED;
-        C.active = 0;
-        C.last_rr = C.g;
+template <int NC>
+__device__ void ctl_end(CgCtl<NC> &C) {
+    C.any = 0;
+    for (int c = 0; c < NC; ++c) {
+        if (C.active[c] && C.out_of_iters) {
+            C.status[c] = NSFEM_MAX_ITERATIONS_REACHED;
+            C.active[c] = 0;
+            C.last_rr[c] = C.g[c];
+        }
+        C.beta[c] = C.active[c] ? C.g[c] / C.gamma[c] : 0.0;
+        if (!C.active[c]) C.alpha[c] = 0.0;
+        C.any = C.any || C.active[c];
     }
-    C.beta = C.active ? C.g / C.gamma : 0.0;
-    if (!C.active) C.alpha = 0.0;
+}
+
+template <int NC>
+__device__ void ctl_finish(const CgCtl<NC> &C, const CgArgs &A) {
+    for (int c = 0; c < NC; ++c) {
+        A.res[c].iterations = C.iters[c];
+        A.res[c].refinements = C.refines;
+        A.res[c].status = C.status[c];
+        A.res[c].last_residual = sqrt(C.last_rr[c]);
+    }
 }
 
 // The one-column mixed persistent CG run by one block (arguments as
@@ -2525,7 +2661,7 @@ __device__ __forceinline__ void cg_body1_m(const CgArgs &A, MP meta, const int b
     // WI 1: group loads (16-bit offsets only); else WI items per lane
     constexpr bool GROUPS = WI == 1;
     static_assert(!GROUPS || std::is_same<IT, int16_t>::value, "group loads read 16-bit words");
-    __shared__ CgCtl1 C;
+    __shared__ CgCtl<1> C;
     const int T0 = A.block_tiles[L], T1 = A.block_tiles[L + 1];
     const int R0 = A.tiles[T0], R1 = A.tiles[T1];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2541,36 +2677,13 @@ __device__ __forceinline__ void cg_body1_m(const CgArgs &A, MP meta, const int b
         double acc[3] = {0.0, 0.0, 0.0};
         residual_phase<1, BS, MIXED, true, IT, true, MP>(A, meta, T0, T1, lds64, acc, A.st[0]);
         if (!grid_sum<3, BS>(A.sync, acc, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
-        if (t0) {
-            const double bn = sqrt(acc[1]), r0n = sqrt(acc[0]);
-            const double ref = bn > 0.0 ? bn : r0n;
-            const double tol = fmax(A.rtol * ref, A.atol);
-            C.tol2 = tol * tol;
-            C.active = acc[0] > C.tol2;
-            C.gamma = acc[2];
-            C.rmax2 = C.last_rr = C.ru_rr = acc[0];
-            // drop triggers in the iteration's (scaled) space; rho converts
-            // a scaled norm into the unscaled one the tolerance is on
-            if (A.scale) C.rmax2 = acc[2];
-            C.rho = A.scale && acc[2] > 0.0 ? acc[0] / acc[2] : 1.0;
-            C.g = 0.0;
-            C.iters = 0;
-            C.status = NSFEM_OK;
-            C.stall = C.dropped = 0;
-            C.pend = C.alpha = C.beta = 0.0;
-            C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = 0;
-            if (writer) {
-                A.res[0].rhs_norm = bn;
-                A.res[0].initial_residual = r0n;
-                A.res[0].tolerance = tol;
-            }
-        }
+        if (t0) ctl_start<1>(C, A, acc, writer);
         __syncthreads();
     }
-    while (C.active) {
+    while (C.any) {
         const int nx = cur ^ 1;
-        const float alpha = (float)C.alpha, beta = (float)C.beta;
-        const double pend = C.pend;
+        const float alpha = (float)C.alpha[0], beta = (float)C.beta[0];
+        const double pend = C.pend[0];
         const bool has_pend = C.has_pend != 0;
         double sums[4] = {0.0, 0.0, 0.0, 0.0};
         CG_TRACE_STAMP(C.k, 0);
@@ -2584,37 +2697,32 @@ __device__ __forceinline__ void cg_body1_m(const CgArgs &A, MP meta, const int b
         if (!grid_sum<4, BS>(A.sync, sums, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
         CG_TRACE_STAMP(C.k, 2);
         if (t0) {
-            ctl_after_phase(C, A, sums);
-            if (!C.ru) ctl_end(C);
+            ctl_after_phase<1>(C, A, sums);
+            if (!C.ru) ctl_end<1>(C);
         }
         __syncthreads();
         if (C.ru) {
             // apply the pending x += alpha p_k (FP64), then replace the
             // recursive residual: r_k := b - A x, alpha := 0
-            flush_x1<BS>(A, R0, R1, A.st[nx], C.pend);
+            flush_x1<BS>(A, R0, R1, A.st[nx], C.pend[0]);
             double dummy[1] = {0.0};
             if (!grid_sum<1, BS>(A.sync, dummy, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
             double ra[3] = {0.0, 0.0, 0.0};
             residual_phase<1, BS, MIXED, false, IT, true, MP>(A, meta, T0, T1, lds64, ra, A.st[nx]);
             if (!grid_sum<3, BS>(A.sync, ra, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
             if (t0) {
-                ctl_after_update(C, A, ra);
-                ctl_end(C);
+                ctl_after_update<1>(C, A, ra);
+                ctl_end<1>(C);
             }
             __syncthreads();
         }
-        if (!C.active) {
-            if (C.has_pend) flush_x1<BS>(A, R0, R1, A.st[nx], C.pend);
+        if (!C.any) {
+            if (C.has_pend) flush_x1<BS>(A, R0, R1, A.st[nx], C.pend[0]);
             break;
         }
         cur = nx;
     }
-    if (writer) {
-        A.res[0].iterations = C.iters;
-        A.res[0].refinements = C.refines;
-        A.res[0].status = C.status;
-        A.res[0].last_residual = sqrt(C.last_rr);
-    }
+    if (writer) ctl_finish<1>(C, A);
     return;
 timeout:
     if (writer) A.res[0].status = NSFEM_BARRIER_TIMEOUT;
@@ -2782,105 +2890,12 @@ __device__ void flush_x2(const CgArgs &A, int R0, int R1, const void *st,
     }
 }
 
-// Control state of a two-column solve (LDS, updated by thread 0): the
-// one-column rules per column, with one iteration count and one reliable
-// update for both (the FP64 residual pass reads the matrix once for both
-// columns; a column that did not ask for the update restarts its recursion
-// from the true residual, like one that did).
-struct CgCtl2 {
-    double tol2[2], gamma[2], rmax2[2], last_rr[2], ru_rr[2], rho[2];
-    double pend[2], alpha[2], beta[2], g[2];
-    int iters[2], status[2], stall[2], active[2], dropped[2];
-    int k, last_ru, refines, ru, has_pend, out_of_iters, any;
-};
-
-__device__ void ctl2_after_phase(CgCtl2 &C, const CgArgs &A, const double (&sums)[8]) {
-    const int k = ++C.k;
-    const double d2 = A.rdelta * A.rdelta;
-    bool want = false;
-    for (int c = 0; c < 2; ++c) {
-        double alpha = 0.0, g = 0.0;
-        bool dropped = false;
-        if (C.active[c]) {
-            const double delta = sums[4 * c], gk = sums[4 * c + 1];
-            if (!(delta > 0.0)) {
-                C.status[c] = NSFEM_BREAKDOWN;
-                C.active[c] = 0;
-                C.last_rr[c] = gk;
-            } else {
-                alpha = gk / delta;
-                g = fmax(gk - 2.0 * alpha * sums[4 * c + 2] + alpha * alpha * sums[4 * c + 3], 0.0);
-                C.gamma[c] = gk;
-                C.iters[c] = k;
-                dropped = g * C.rho[c] <= C.tol2[c] ||
-                          (g < d2 * C.rmax2[c] &&
-                           (k - C.last_ru >= A.ru_min_gap || g < d2 * d2 * C.rmax2[c]));
-            }
-        }
-        want = want || dropped;
-        C.pend[c] = alpha;
-        C.alpha[c] = alpha;
-        C.g[c] = g;
-        C.dropped[c] = dropped;
-    }
-    C.has_pend = 1;
-    C.out_of_iters = k >= A.max_iter;
-    const bool any = C.active[0] || C.active[1];
-    C.ru = any && (want || k - C.last_ru >= A.ru_gap || C.out_of_iters);
-    if (C.ru) C.last_ru = k;
-}
-
-// After a reliable update; ra as residual_phase<2>: ra[c] = FP64 (r, r),
-// ra[4 + c] = (FP32 r, FP32 r).
-__device__ void ctl2_after_update(CgCtl2 &C, const CgArgs &A, const double (&ra)[6]) {
-    C.has_pend = 0;
-    ++C.refines;
-    for (int c = 0; c < 2; ++c) {
-        C.pend[c] = 0.0;
-        C.alpha[c] = 0.0;
-        C.last_rr[c] = ra[c];
-        if (!C.active[c]) continue;
-        if (ra[c] <= C.tol2[c]) {
-            C.active[c] = 0;
-            continue;
-        }
-        C.g[c] = ra[4 + c];
-        C.rmax2[c] = A.scale ? ra[4 + c] : ra[c];
-        C.rho[c] = A.scale && ra[4 + c] > 0.0 ? ra[c] / ra[4 + c] : 1.0;
-        if (C.dropped[c]) {
-            const double sr = 0.5 * (1.0 + A.rdelta);
-            C.stall[c] = ra[c] > sr * sr * C.ru_rr[c] ? C.stall[c] + 1 : 0;
-        }
-        C.ru_rr[c] = fmin(C.ru_rr[c], ra[c]);
-        if (C.stall[c] >= 3) {
-            C.status[c] = NSFEM_STAGNATION;
-            C.active[c] = 0;
-        } else if (C.refines >= A.max_refine) {
-            C.status[c] = NSFEM_MAX_ITERATIONS_REACHED;
-            C.active[c] = 0;
-        }
-    }
-}
-
-__device__ void ctl2_end(CgCtl2 &C) {
-    for (int c = 0; c < 2; ++c) {
-        if (C.active[c] && C.out_of_iters) {
-            C.status[c] = NSFEM_MAX_ITERATIONS_REACHED;
-            C.active[c] = 0;
-            C.last_rr[c] = C.g[c];
-        }
-        C.beta[c] = C.active[c] ? C.g[c] / C.gamma[c] : 0.0;
-        if (!C.active[c]) C.alpha[c] = 0.0;
-    }
-    C.any = C.active[0] || C.active[1];
-}
-
 // The two-column mixed persistent CG run by one block (arguments as
 // cg_body), single-reduction iteration over the packed state.
 template <int BS, typename IT, int IB, typename MP>
 __device__ __forceinline__ void cg_body2_m(const CgArgs &A, MP meta, const int bid, const int nb,
                                            const int L, double *prod_raw, double *lds) {
-    __shared__ CgCtl2 C;
+    __shared__ CgCtl<2> C;
     const int T0 = A.block_tiles[L], T1 = A.block_tiles[L + 1];
     const int R0 = A.tiles[T0], R1 = A.tiles[T1];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2894,31 +2909,7 @@ __device__ __forceinline__ void cg_body2_m(const CgArgs &A, MP meta, const int b
         double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         residual_phase<2, BS, true, true, IT, true, MP>(A, meta, T0, T1, lds64, acc, A.st[0]);
         if (!grid_sum<6, BS>(A.sync, acc, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
-        if (t0) {
-            for (int c = 0; c < 2; ++c) {
-                const double bn = sqrt(acc[2 + c]), r0n = sqrt(acc[c]);
-                const double ref = bn > 0.0 ? bn : r0n;
-                const double tol = fmax(A.rtol * ref, A.atol);
-                C.tol2[c] = tol * tol;
-                C.active[c] = acc[c] > C.tol2[c];
-                C.gamma[c] = acc[4 + c];
-                C.rmax2[c] = A.scale ? acc[4 + c] : acc[c];
-                C.last_rr[c] = C.ru_rr[c] = acc[c];
-                C.rho[c] = A.scale && acc[4 + c] > 0.0 ? acc[c] / acc[4 + c] : 1.0;
-                C.g[c] = 0.0;
-                C.iters[c] = 0;
-                C.status[c] = NSFEM_OK;
-                C.stall[c] = C.dropped[c] = 0;
-                C.pend[c] = C.alpha[c] = C.beta[c] = 0.0;
-                if (writer) {
-                    A.res[c].rhs_norm = bn;
-                    A.res[c].initial_residual = r0n;
-                    A.res[c].tolerance = tol;
-                }
-            }
-            C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = 0;
-            C.any = C.active[0] || C.active[1];
-        }
+        if (t0) ctl_start<2>(C, A, acc, writer);
         __syncthreads();
     }
     while (C.any) {
@@ -2935,8 +2926,8 @@ __device__ __forceinline__ void cg_body2_m(const CgArgs &A, MP meta, const int b
         if (!grid_sum<8, BS>(A.sync, sums, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
         CG_TRACE_STAMP(C.k, 2);
         if (t0) {
-            ctl2_after_phase(C, A, sums);
-            if (!C.ru) ctl2_end(C);
+            ctl_after_phase<2>(C, A, sums);
+            if (!C.ru) ctl_end<2>(C);
         }
         __syncthreads();
         if (C.ru) {
@@ -2950,8 +2941,8 @@ __device__ __forceinline__ void cg_body2_m(const CgArgs &A, MP meta, const int b
             residual_phase<2, BS, true, false, IT, true, MP>(A, meta, T0, T1, lds64, ra, A.st[nx]);
             if (!grid_sum<6, BS>(A.sync, ra, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
             if (t0) {
-                ctl2_after_update(C, A, ra);
-                ctl2_end(C);
+                ctl_after_update<2>(C, A, ra);
+                ctl_end<2>(C);
             }
             __syncthreads();
         }
@@ -2964,14 +2955,7 @@ __device__ __forceinline__ void cg_body2_m(const CgArgs &A, MP meta, const int b
         }
         cur = nx;
     }
-    if (writer) {
-        for (int c = 0; c < 2; ++c) {
-            A.res[c].iterations = C.iters[c];
-            A.res[c].refinements = C.refines;
-            A.res[c].status = C.status[c];
-            A.res[c].last_residual = sqrt(C.last_rr[c]);
-        }
-    }
+    if (writer) ctl_finish<2>(C, A);
     return;
 timeout:
     if (writer) {
@@ -3113,7 +3097,7 @@ __device__ void phase_q2(const CgArgs &A, MP meta, int T0, int T1, double *lds_w
 template <int BS, typename IT, int IB, typename MP>
 __device__ __forceinline__ void cg_body2n_m(const CgArgs &A, MP meta, const int bid, const int nb,
                                             const int L, double *prod_raw, double *lds) {
-    __shared__ CgCtl2 C;
+    __shared__ CgCtl<2> C;
     const int T0 = A.block_tiles[L], T1 = A.block_tiles[L + 1];
     const int R0 = A.tiles[T0], R1 = A.tiles[T1];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -3129,31 +3113,7 @@ __device__ __forceinline__ void cg_body2n_m(const CgArgs &A, MP meta, const int 
         residual_phase<2, BS, true, true, IT, false, MP>(A, meta, T0, T1, lds64, acc);
         for (int row = R0 + (int)threadIdx.x; row < R1; row += BS) q[row] = make_float2(0.f, 0.f);
         if (!grid_sum<6, BS>(A.sync, acc, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
-        if (t0) {
-            for (int c = 0; c < 2; ++c) {
-                const double bn = sqrt(acc[2 + c]), r0n = sqrt(acc[c]);
-                const double ref = bn > 0.0 ? bn : r0n;
-                const double tol = fmax(A.rtol * ref, A.atol);
-                C.tol2[c] = tol * tol;
-                C.active[c] = acc[c] > C.tol2[c];
-                C.gamma[c] = acc[4 + c];
-                C.rmax2[c] = A.scale ? acc[4 + c] : acc[c];
-                C.last_rr[c] = C.ru_rr[c] = acc[c];
-                C.rho[c] = A.scale && acc[4 + c] > 0.0 ? acc[c] / acc[4 + c] : 1.0;
-                C.g[c] = 0.0;
-                C.iters[c] = 0;
-                C.status[c] = NSFEM_OK;
-                C.stall[c] = C.dropped[c] = 0;
-                C.pend[c] = C.alpha[c] = C.beta[c] = 0.0;
-                if (writer) {
-                    A.res[c].rhs_norm = bn;
-                    A.res[c].initial_residual = r0n;
-                    A.res[c].tolerance = tol;
-                }
-            }
-            C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = 0;
-            C.any = C.active[0] || C.active[1];
-        }
+        if (t0) ctl_start<2>(C, A, acc, writer);
         __syncthreads();
     }
     while (C.any) {
@@ -3169,8 +3129,8 @@ __device__ __forceinline__ void cg_body2n_m(const CgArgs &A, MP meta, const int 
         phase_q2<BS, IT, IB, MP>(A, meta, T0, T1, lds64, p, r, q, sums);
         if (!grid_sum<8, BS>(A.sync, sums, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
         if (t0) {
-            ctl2_after_phase(C, A, sums);
-            if (!C.ru) ctl2_end(C);
+            ctl_after_phase<2>(C, A, sums);
+            if (!C.ru) ctl_end<2>(C);
         }
         __syncthreads();
         if (C.ru) {
@@ -3183,8 +3143,8 @@ __device__ __forceinline__ void cg_body2n_m(const CgArgs &A, MP meta, const int 
             residual_phase<2, BS, true, false, IT, false, MP>(A, meta, T0, T1, lds64, ra);
             if (!grid_sum<6, BS>(A.sync, ra, epoch, lds, A.timeout_ticks, bid, nb, A.flat)) goto timeout;
             if (t0) {
-                ctl2_after_update(C, A, ra);
-                ctl2_end(C);
+                ctl_after_update<2>(C, A, ra);
+                ctl_end<2>(C);
             }
             __syncthreads();
         }
@@ -3196,14 +3156,7 @@ __device__ __forceinline__ void cg_body2n_m(const CgArgs &A, MP meta, const int 
             break;
         }
     }
-    if (writer) {
-        for (int c = 0; c < 2; ++c) {
-            A.res[c].iterations = C.iters[c];
-            A.res[c].refinements = C.refines;
-            A.res[c].status = C.status[c];
-            A.res[c].last_residual = sqrt(C.last_rr[c]);
-        }
-    }
+    if (writer) ctl_finish<2>(C, A);
     return;
 timeout:
     if (writer) {
@@ -3240,6 +3193,523 @@ __global__ __launch_bounds__(BS, BS / 256) void k_cg_p2(const CgArgs A) {
         cg_body2n_m<BS, IT, IB>(A, A.meta, blockIdx.x, gridDim.x, L, prod_raw, lds);
     else
         cg_body2_m<BS, IT, IB>(A, A.meta, blockIdx.x, gridDim.x, L, prod_raw, lds);
+}
+
+// =====================================================================
+// Resident CG: a solve whose matrix stays in the blocks' registers
+// =====================================================================
+//
+// The persistent forms above stream the matrix from memory and gather the
+// neighbours' vector entries every iteration, and publish what they wrote
+// with an L2 write-back and invalidate at every grid reduction.  On a system
+// of up to a few hundred thousand rows none of that is bandwidth: an
+// iteration is a chain of load latencies and cache maintenance (12 us on the
+// 512 x 128 channel's 65,656 pressure rows in FP32, 15-24 us in FP64).  Here,
+// when the rows are short (at most W nonzeros) and banded:
+//
+// * a lane owns one row of up to R wave tiles and keeps the row's values, its
+//   columns (16-bit positions in the block's window) and its r, q and x in
+//   registers for the whole solve;
+// * the block keeps p for its window -- its own rows and the rows its columns
+//   reach, one contiguous run -- in LDS, and r for the window's rows that
+//   other blocks own.  It updates both for itself from the neighbours' q, the
+//   only vector that crosses blocks: r = r - alpha q and p = r + beta p round
+//   the same in every block that computes them;
+// * q and the sums cross through agent-scope relaxed stores and loads, which
+//   meet at the coherence point and pass the caches by, so that nothing is
+//   written back or invalidated: a wave waits for its stores of q, the block
+//   meets, and the sums are posted with the epoch beside their bits, one read
+//   giving arrival and value together.
+//
+// One exchange an iteration (the single-reduction iteration of the one-column
+// mixed solves, in FP64 too).  In the one-column mixed form every product,
+// sum and reduction has phase_f1g's order (wave tiles to waves, lanes to rows,
+// the same grid), so its iterates are that form's, bit for bit.
+//
+// Measured per iteration, streaming -> resident: 1,089 pressure rows in one
+// block, FP64 11.1 -> 2.2 us; 65,656 rows on 42 blocks, FP64 18.1 -> 4.5,
+// refined 12.4 -> 4.9 with its residual passes; 261,247 rows on 170 blocks,
+// FP64 25.9 -> 6.3, refined 20.8 -> 6.6; 261,241 P2 rows on 256 blocks, FP64
+// 55.9 -> 16.2, both columns refined 121 -> 50 (23 residual passes in 47
+// iterations).  Systems past the registers or the window (a million P2 rows,
+// the vertices-first node order of larger meshes) keep the streaming forms.
+
+constexpr int kResWaves = 12;  // 3 waves a SIMD: 168 VGPRs each
+constexpr int kResBlock = 64 * kResWaves;
+
+template <typename T>
+__device__ __forceinline__ T ld_agent(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void st_agent(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// rows of NC interleaved columns
+template <int NC, typename T>
+__device__ __forceinline__ VecN<NC, T> ldv_agent(const T *p, int i) {
+    VecN<NC, T> o;
+    if constexpr (NC == 2 && sizeof(T) == 4) {
+        const unsigned long long t =
+            ld_agent(reinterpret_cast<const unsigned long long *>(p) + i);
+        o.v[0] = __uint_as_float((unsigned)t);
+        o.v[1] = __uint_as_float((unsigned)(t >> 32));
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) o.v[c] = ld_agent(p + (size_t)i * NC + c);
+    }
+    return o;
+}
+template <int NC, typename T>
+__device__ __forceinline__ void stv_agent(T *p, int i, const VecN<NC, T> &v) {
+    if constexpr (NC == 2 && sizeof(T) == 4) {
+        const unsigned long long t =
+            (unsigned long long)__float_as_uint(v.v[0]) |
+            ((unsigned long long)__float_as_uint(v.v[1]) << 32);
+        st_agent(reinterpret_cast<unsigned long long *>(p) + i, t);
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) st_agent(p + (size_t)i * NC + c, v.v[c]);
+    }
+}
+
+// wave_sum's sum, in its order, without the LDS pipe: lanes 32 and 16 apart
+// by row swaps, then rotations within rows of 16 (after each step the values
+// repeat with that period, so a rotation pairs what an exclusive-or does).
+template <int CTRL>
+__device__ __forceinline__ double dpp_rotated(double v) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                            (unsigned long long)(unsigned)lo));
+}
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+    {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32),
+                                                         false, false);
+        v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
+    {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32),
+                                                         false, false);
+        v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
+    v += dpp_rotated<0x128>(v);  // row_ror:8
+    v += dpp_rotated<0x124>(v);
+    v += dpp_rotated<0x122>(v);
+    v += dpp_rotated<0x121>(v);
+    return v;
+}
+
+struct ResShared {
+    double part[2][kMaxRed][kResWaves];  // by epoch parity
+    double sum[kMaxRed];
+    int fail;
+};
+
+// The grid's sums of K values a thread, into S.sum, and a barrier over the
+// solve's blocks: every block's agent-scope stores before it are visible to
+// agent-scope loads after it.  False when a block did not arrive in time.
+//
+// Wave k adds the block's partials of sum k in wave order, posts the two
+// halves of the result, each in one 8-byte word with the epoch, and polls the
+// other blocks' words; a word that carries the epoch is whole, so nothing
+// orders the two halves.  The words alternate between two slots by epoch
+// parity: a block posts epoch e + 2 only after every block has posted e + 1,
+// which each does after it has read all of e.  Sums are added as in
+// grid_sum_flat.  The waits on vmcnt before the first barrier are what makes
+// the block's stores visible before its post.
+template <int K>
+__device__ __forceinline__ bool res_exchange(SyncState *G, ResShared &S, double (&v)[K],
+                                             unsigned &epoch, const unsigned long long timeout,
+                                             const int b, const int nb) {
+    static_assert(K <= kMaxRed && K <= kResWaves, "reduction width");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned e = ++epoch;
+    const int par = e & 1u;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = wave_sum_dpp(v[k]);
+        if (lane == 0) S.part[par][k][wave] = v[k];
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
+    __syncthreads();
+    if (wave < K) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < kResWaves; ++i) s += S.part[par][wave][i];
+        if (nb == 1) {
+            if (lane == 0) S.sum[wave] = s;
+        } else {
+            unsigned long long(*words)[2] = G->tag[par][wave];
+            const unsigned long long mark = (unsigned long long)e << 32;
+            const unsigned long long bits = (unsigned long long)__double_as_longlong(s);
+            if (lane < 2)
+                st_agent(&words[b][lane], mark | (lane ? bits >> 32 : bits & 0xffffffffull));
+            double t = 0.0;
+            bool ok = true;
+            const unsigned long long t0 = wall_clock64();
+            for (int i = lane; i < nb; i += 64) {
+                unsigned long long w0 = ld_agent(&words[i][0]), w1 = ld_agent(&words[i][1]);
+                while (ok && ((w0 ^ mark) >> 32 != 0 || (w1 ^ mark) >> 32 != 0)) {
+                    if (ld_agent(&G->abort) != 0u) {
+                        ok = false;
+                    } else if (wall_clock64() - t0 > timeout) {
+                        st_agent(&G->abort, 1u);
+                        ok = false;
+                    }
+                    w0 = ld_agent(&words[i][0]);
+                    w1 = ld_agent(&words[i][1]);
+                }
+                t += __longlong_as_double((long long)((w1 << 32) | (w0 & 0xffffffffull)));
+            }
+            t = wave_sum_dpp(t);
+            if (lane == 0) S.sum[wave] = t;
+            if (!ok) S.fail = 1;
+        }
+    }
+    __syncthreads();
+    return S.fail == 0;
+}
+
+// The FP64 residual of the wave's rows: r = b - A x, scaled and rounded to VT,
+// published in rbuf; the sums as residual_phase's, which it rounds as (the
+// products before they are added, in column order).  SHARED: x as other
+// blocks published it.  The loop over the wave's tiles stays rolled, so that
+// its loads take no registers from the resident matrix more than once.
+template <int NC, typename VT, bool SHARED>
+__device__ __forceinline__ void res_residual(const CgArgs &A, const int T0, const int T1,
+                                             const int wave, const int lane, VT *rbuf,
+                                             double (&acc)[3 * NC]) {
+#pragma unroll 1
+    for (int t = T0 + wave; t < T1; t += kResWaves) {
+        const int4 m = A.meta[t];
+        const int row = m.x + lane;
+        if (row >= m.y) continue;
+        double s[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) s[c] = 0.0;
+        const int ka = A.rs[row], kb = A.rs[row + 1];
+        // four nonzeros' loads in flight (past the row: its last, not added)
+#pragma unroll 1
+        for (int k0 = ka; k0 < kb; k0 += 4) {
+            double pr[4][NC];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = min(k0 + u, kb - 1);
+                const double v = A.val64[k];
+                const int j = A.col[k];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const double *xp = A.x + (size_t)c * A.n + j;
+                    pr[u][c] = v * (SHARED ? ld_agent(xp) : *xp);
+                    asm("" : "+v"(pr[u][c]));  // no fused multiply-add
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+                    if (k0 + u < kb) s[c] += pr[u][c];
+        }
+        const double sc = A.scale ? A.scale[row] : 1.0;
+        VecN<NC, VT> r;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const double bb = A.b[(size_t)c * A.n + row];
+            const double rr = bb - s[c];
+            acc[c] += rr * rr;
+            if (!SHARED) acc[NC + c] += bb * bb;
+            r.v[c] = (VT)(A.scale ? rr * sc : rr);
+            acc[2 * NC + c] += (double)r.v[c] * (double)r.v[c];
+        }
+        stv_agent<NC, VT>(rbuf, row, r);
+    }
+}
+
+// One block's part of a resident solve of `nb` blocks (`b`: its reduction
+// slot, `L`: its index among the tiles' owners, as cg_body).  W: the most
+// nonzeros of a row; R: the most wave tiles of a wave (the host checks both,
+// and that the window fits win_cap).  smem: win_cap + 1 rows of p, then r of
+// the window's rows that other blocks own.
+template <int NC, bool MIXED, int W, int R>
+__device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const int nb,
+                                            const int L, unsigned char *smem) {
+    using VT = typename std::conditional<MIXED, float, double>::type;
+    using Row = VecN<NC, VT>;
+    __shared__ CgCtl<NC> C;
+    __shared__ ResShared S;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int T0 = A.block_tiles[L], T1 = A.block_tiles[L + 1];
+    const int R0 = A.tiles[T0], R1 = A.tiles[T1];
+    const int win0 = max(0, R0 - A.band_lo), win1 = min(A.n, R1 + A.band_hi);
+    const int nl = R0 - win0, nh = nl + (win1 - R1), wn = win1 - win0;
+    Row *pw = reinterpret_cast<Row *>(smem);
+    Row *rh = pw + A.win_cap + 1;
+    VT *rbuf = (VT *)A.r;
+    VT *qbuf[2] = {(VT *)A.p0, (VT *)A.p1};
+    const bool t0 = tid == 0, writer = L == 0 && t0;
+    unsigned epoch = 0;
+
+    int row[R];  // -1: none
+    VT val[R][W];
+    unsigned idx[R][(W + 1) / 2];
+    Row r[R], q[R];
+    VecN<NC, double> x[R];
+    if (t0) S.fail = 0;
+    {
+        Row zero;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) zero.v[c] = (VT)0;
+        for (int i = tid; i <= wn; i += kResBlock) pw[i] = zero;
+        for (int i = tid; i < nh; i += kResBlock) rh[i] = zero;
+        double acc[3 * NC];
+#pragma unroll
+        for (int k = 0; k < 3 * NC; ++k) acc[k] = 0.0;
+        res_residual<NC, VT, false>(A, T0, T1, wave, lane, rbuf, acc);
+        if (!res_exchange<3 * NC>(A.sync, S, acc, epoch, A.timeout_ticks, b, nb)) goto timeout;
+        if (t0) {
+            double sums[3 * NC];
+#pragma unroll
+            for (int k = 0; k < 3 * NC; ++k) sums[k] = S.sum[k];
+            ctl_start<NC>(C, A, sums, writer);
+        }
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            row[j] = -1;
+            q[j] = zero;
+            r[j] = zero;
+#pragma unroll
+            for (int w = 0; w < W; ++w) val[j][w] = (VT)0;
+#pragma unroll
+            for (int w = 0; w < (W + 1) / 2; ++w) idx[j][w] = (unsigned)wn * 0x10001u;
+            const int t = T0 + wave + kResWaves * j;
+            if (t >= T1) continue;  // wave-uniform
+            const int4 m = A.meta[t];
+            const bool has = m.x + lane < m.y;
+            const int k0 = A.rs[has ? m.x + lane : m.x];
+            const int len = has ? A.rs[m.x + lane + 1] - k0 : 0;
+            row[j] = has ? m.x + lane : -1;
+            // a lane past its row's nonzeros reads the matrix's last entry
+            // and keeps 0 x (the window's zero)
+            const int last = A.nnz - 1;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const int k = min(k0 + w, last);
+                VT v;
+                if constexpr (MIXED) v = A.val32[k];
+                else v = A.val64[k];
+                const unsigned pos = w < len ? (unsigned)(A.col[k] - win0) : (unsigned)wn;
+                val[j][w] = w < len ? v : (VT)0;
+                if (w % 2) idx[j][w / 2] |= pos << 16;
+                else idx[j][w / 2] = pos;
+                if (w % 5 == 4) __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (!has) continue;
+            r[j] = ldv_agent<NC, VT>(rbuf, row[j]);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) x[j].v[c] = A.x[(size_t)c * A.n + row[j]];
+        }
+        __syncthreads();
+    }
+    {
+        bool fresh = true;  // rbuf holds r (after a residual), not qbuf the step's q
+        int par = 0;
+        while (C.any) {
+            VT alpha[NC], beta[NC];
+            double pend[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                alpha[c] = (VT)C.alpha[c];
+                beta[c] = (VT)C.beta[c];
+                pend[c] = C.pend[c];
+            }
+            const bool has_pend = C.has_pend != 0;
+            // the window's rows of other blocks: kAhead loads in flight
+            constexpr int kAhead = 4;
+            const VT *src = fresh ? rbuf : qbuf[par ^ 1];
+            for (int base = tid; base < nh; base += kAhead * kResBlock) {
+                Row in[kAhead];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) {
+                    const int i = min(base + u * kResBlock, nh - 1);
+                    in[u] = ldv_agent<NC, VT>(src, i < nl ? win0 + i : R1 + (i - nl));
+                }
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) {
+                    const int i = base + u * kResBlock;
+                    if (i >= nh) break;
+                    const int slot = i < nl ? i : i + (R1 - R0);
+                    Row rn, pn = pw[slot];
+                    if (fresh) {
+                        rn = in[u];
+                    } else {
+                        rn = rh[i];
+#pragma unroll
+                        for (int c = 0; c < NC; ++c)
+                            rn.v[c] = fma_t<VT>(-alpha[c], in[u].v[c], rn.v[c]);
+                    }
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) pn.v[c] = fma_t<VT>(beta[c], pn.v[c], rn.v[c]);
+                    rh[i] = rn;
+                    pw[slot] = pn;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                if (row[j] < 0) continue;
+                Row pn = pw[row[j] - win0];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    if (has_pend)
+                        x[j].v[c] = __builtin_fma(x_step(A, pend[c], row[j]), (double)pn.v[c],
+                                                  x[j].v[c]);
+                    r[j].v[c] = fma_t<VT>(-alpha[c], q[j].v[c], r[j].v[c]);
+                    pn.v[c] = fma_t<VT>(beta[c], pn.v[c], r[j].v[c]);
+                }
+                pw[row[j] - win0] = pn;
+            }
+            __syncthreads();
+            double sums[4 * NC];
+#pragma unroll
+            for (int k = 0; k < 4 * NC; ++k) sums[k] = 0.0;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                if (T0 + wave + kResWaves * j >= T1) continue;  // wave-uniform
+                double s[NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) s[c] = 0.0;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    unsigned word = idx[j][w / 2];
+                    VT v = val[j][w];
+                    // keeps the widened value and the address out of the
+                    // registers across iterations: they would double the
+                    // matrix's
+                    asm volatile("" : "+v"(word), "+v"(v));
+                    const Row pv = pw[w % 2 ? word >> 16 : word & 0xffffu];
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        s[c] = __builtin_fma((double)v, (double)pv.v[c], s[c]);
+                    // five reads in flight: all W of them would not fit
+                    if (w % 5 == 4) __builtin_amdgcn_sched_barrier(0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (row[j] < 0) continue;
+                const Row pn = pw[row[j] - win0];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    q[j].v[c] = (VT)s[c];
+                    const double rd = (double)r[j].v[c], qd = (double)q[j].v[c];
+                    sums[4 * c] += (double)pn.v[c] * s[c];
+                    sums[4 * c + 1] += rd * rd;
+                    sums[4 * c + 2] += rd * qd;
+                    sums[4 * c + 3] += qd * qd;
+                }
+                stv_agent<NC, VT>(qbuf[par], row[j], q[j]);
+            }
+            if (!res_exchange<4 * NC>(A.sync, S, sums, epoch, A.timeout_ticks, b, nb)) goto timeout;
+            if (t0) {
+#pragma unroll
+                for (int k = 0; k < 4 * NC; ++k) sums[k] = S.sum[k];
+                ctl_after_phase<NC, MIXED>(C, A, sums);
+                if (!C.ru) ctl_end<NC>(C);
+            }
+            __syncthreads();
+            fresh = false;
+            if constexpr (MIXED) {
+                if (C.ru) {
+                    // apply the pending x += alpha p_k (FP64), then replace
+                    // the recursive residual: r_k := b - A x, alpha := 0
+#pragma unroll
+                    for (int j = 0; j < R; ++j) {
+                        if (row[j] < 0) continue;
+                        const Row pn = pw[row[j] - win0];
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) {
+                            x[j].v[c] = __builtin_fma(x_step(A, C.pend[c], row[j]),
+                                                      (double)pn.v[c], x[j].v[c]);
+                            st_agent(A.x + (size_t)c * A.n + row[j], x[j].v[c]);
+                        }
+                    }
+                    double none[1] = {0.0};
+                    if (!res_exchange<1>(A.sync, S, none, epoch, A.timeout_ticks, b, nb))
+                        goto timeout;
+                    double ra[3 * NC];
+#pragma unroll
+                    for (int k = 0; k < 3 * NC; ++k) ra[k] = 0.0;
+                    res_residual<NC, VT, true>(A, T0, T1, wave, lane, rbuf, ra);
+                    if (!res_exchange<3 * NC>(A.sync, S, ra, epoch, A.timeout_ticks, b, nb))
+                        goto timeout;
+                    if (t0) {
+#pragma unroll
+                        for (int k = 0; k < 3 * NC; ++k) ra[k] = S.sum[k];
+                        ctl_after_update<NC>(C, A, ra);
+                        ctl_end<NC>(C);
+                    }
+#pragma unroll
+                    for (int j = 0; j < R; ++j)
+                        if (row[j] >= 0) r[j] = ldv_agent<NC, VT>(rbuf, row[j]);
+                    __syncthreads();
+                    fresh = true;
+                }
+            }
+            if (!C.any) {
+                if (C.has_pend) {
+#pragma unroll
+                    for (int j = 0; j < R; ++j) {
+                        if (row[j] < 0) continue;
+                        const Row pn = pw[row[j] - win0];
+#pragma unroll
+                        for (int c = 0; c < NC; ++c)
+                            x[j].v[c] = __builtin_fma(x_step(A, C.pend[c], row[j]),
+                                                      (double)pn.v[c], x[j].v[c]);
+                    }
+                }
+                break;
+            }
+            par ^= 1;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        if (row[j] < 0) continue;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) A.x[(size_t)c * A.n + row[j]] = x[j].v[c];
+    }
+    if (writer) ctl_finish<NC>(C, A);
+    return;
+timeout:
+    if (writer) {
+        for (int c = 0; c < NC; ++c) A.res[c].status = NSFEM_BARRIER_TIMEOUT;
+    }
+}
+
+template <int NC, bool MIXED, int W, int R>
+__global__ __launch_bounds__(kResBlock, kResBlock / 256) void k_cg_res(const CgArgs A) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    cg_resident<NC, MIXED, W, R>(A, blockIdx.x, gridDim.x, xcd_swizzle(blockIdx.x, gridDim.x),
+                                 smem);
+}
+
+// Many resident solves in one launch (block map as k_cg_batch).
+template <int NC, bool MIXED, int W, int R>
+__global__ __launch_bounds__(kResBlock, kResBlock / 256) void k_cg_res_batch(
+    const CgArgs *__restrict__ args, const int2 *__restrict__ map) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int2 m = map[blockIdx.x];
+    const int inst = __builtin_amdgcn_readfirstlane(m.x);
+    const int lb = __builtin_amdgcn_readfirstlane(m.y);
+    const CgArgs A = args[inst];
+    cg_resident<NC, MIXED, W, R>(A, lb, A.nblocks, lb, smem);
 }
 
 // Many independent systems in one persistent launch: block i works for
@@ -3429,6 +3899,154 @@ struct CgLaunch {
 };
 
 
+// ---- resident solves
+// Most nonzeros of a row and most wave tiles of a wave of the resident
+// kernels: what 168 registers hold beside the solve's state.
+constexpr int kResRowShort = 8, kResRowLong = 20;
+constexpr int res_tiles(bool mixed, int w) { return w == kResRowShort ? 4 : mixed ? 3 : 2; }
+// Most LDS of a resident block (160 KB a CU; one block a CU).
+constexpr size_t kResLds = 120 * 1024;
+
+// Calls f.template run<NC, MIXED, W, R>() for a resident solve whose waves own
+// `tiles` wave tiles at most.
+template <int NC, bool MIXED, int W, typename F>
+void res_dispatch_tiles(int tiles, F &f) {
+    constexpr int most = res_tiles(MIXED, W);
+    if (tiles <= 1) f.template run<NC, MIXED, W, 1>();
+    else if (tiles == 2) f.template run<NC, MIXED, W, 2>();
+    else f.template run<NC, MIXED, W, most>();
+}
+template <typename F>
+void res_dispatch(int nc, bool mixed, int w, int tiles, F &&f) {
+    constexpr int S = kResRowShort, L = kResRowLong;
+    if (nc == 1 && mixed) {
+        if (w == S) res_dispatch_tiles<1, true, S>(tiles, f);
+        else res_dispatch_tiles<1, true, L>(tiles, f);
+    } else if (nc == 1) {
+        if (w == S) res_dispatch_tiles<1, false, S>(tiles, f);
+        else res_dispatch_tiles<1, false, L>(tiles, f);
+    } else if (mixed) {
+        res_dispatch_tiles<2, true, L>(tiles, f);
+    } else {
+        res_dispatch_tiles<2, false, L>(tiles, f);
+    }
+}
+
+template <int NC, bool MIXED, int W, int R>
+const void *res_kernel(bool batch) {
+    return batch ? (const void *)k_cg_res_batch<NC, MIXED, W, R>
+                 : (const void *)k_cg_res<NC, MIXED, W, R>;
+}
+// Allows a kernel its dynamic LDS and returns the blocks a device holds.
+struct ResMaxGrid {
+    Device &d;
+    size_t lds;
+    bool batch;
+    int out;
+    template <int NC, bool MX, int W, int R>
+    void run() {
+        const void *k = res_kernel<NC, MX, W, R>(batch);
+        if (lds > 48 * 1024)
+            NSFEM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        int per_cu = 0;
+        NSFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, kResBlock, lds));
+        out = std::min(per_cu * d.cu_count, kResMaxBlocks);
+    }
+};
+struct ResLaunch {
+    Device &d;
+    void **kargs;
+    int grid;
+    size_t lds;
+    bool batch;
+    template <int NC, bool MX, int W, int R>
+    void run() {
+        NSFEM_HIP(hipLaunchCooperativeKernel(res_kernel<NC, MX, W, R>(batch), dim3(grid),
+                                             dim3(kResBlock), kargs, (unsigned)lds, d.stream));
+    }
+};
+
+// Window rows and LDS of a matrix split over `grid` blocks; false when a
+// block's tiles, window or LDS go past what the kernel holds.
+// Wave tiles a wave that a solve's grid aims at.  Short rows (P1): two, as the
+// grid reductions grow with the blocks (resident, 65,656 rows: 4.5 us an
+// iteration on 42 or 64 blocks, 5.2 on 128, 6.3 on 256).  Long rows (P2): one,
+// as a tile's work and the residual passes outweigh them (65,657 rows, two
+// columns: FP64 19.1 us on 63 blocks, 13.9 on 128; refined 38.9 and 25.3).
+int cg_tiles_per_wave(const Matrix &m) { return m.max_row_nz > kResRowShort ? 1 : 2; }
+
+bool res_fits(const Matrix &m, int nc, bool mixed, int w, int grid, ResidentPlan &plan) {
+    std::vector<int32_t> bt;
+    split_tiles(m, grid, bt);
+    int64_t cap = 0, halo = 0;
+    int tiles = 0;
+    for (int b = 0; b < grid; ++b) {
+        tiles = std::max(tiles, (bt[b + 1] - bt[b] + kResWaves - 1) / kResWaves);
+        if (bt[b + 1] <= bt[b] || tiles > res_tiles(mixed, w)) return false;
+        const int64_t r0 = m.host_wtiles[bt[b]], r1 = m.host_wtiles[bt[b + 1]];
+        const int64_t w0 = std::max<int64_t>(0, r0 - m.band_lo);
+        const int64_t w1 = std::min<int64_t>(m.rows, r1 + m.band_hi);
+        cap = std::max(cap, w1 - w0);
+        halo = std::max(halo, (w1 - w0) - (r1 - r0));
+    }
+    const size_t bytes = (size_t)(cap + 1 + halo) * nc * (mixed ? sizeof(float) : sizeof(double));
+    if (cap >= 65535 || bytes > kResLds) return false;
+    plan.ok = true;
+    plan.width = w;
+    plan.tiles = tiles;
+    plan.grid = grid;
+    plan.cap = (int)cap;
+    plan.lds = bytes;
+    return true;
+}
+
+// The resident form of a solve on this matrix, or ok = false: rows of at most
+// kResRowLong nonzeros, a window that fits the LDS, and a grid, the device's
+// blocks at most, that leaves every wave its tiles.  `want` > 0 asks for a
+// grid; else cg_tiles_per_wave, more blocks where a wave would get more tiles
+// than it holds.
+ResidentPlan plan_resident(const Matrix &m, int nc, bool mixed, int want, int max_blocks) {
+    ResidentPlan plan;
+    if (m.rows != m.cols || m.nnz <= 0 || m.max_row_nz > kResRowLong) return plan;
+    const int w = nc == 1 && m.max_row_nz <= kResRowShort ? kResRowShort : kResRowLong;
+    const int most = std::min(std::min(max_blocks, kResMaxBlocks), m.n_wtiles);
+    if (most < 1) return plan;
+    if (want > 0) {
+        res_fits(m, nc, mixed, w, std::min(want, most), plan);
+        return plan;
+    }
+    int grid = std::max(1, std::min(m.n_wtiles / (cg_tiles_per_wave(m) * kResWaves), most));
+    const int room = kResWaves * res_tiles(mixed, w);
+    if ((int64_t)room * most < m.n_wtiles) return plan;
+    for (int tries = 0; tries < 8 && grid <= most; ++tries) {
+        if (res_fits(m, nc, mixed, w, grid, plan)) return plan;
+        grid = std::max(grid + 1, std::max((m.n_wtiles + room - 1) / room, grid + grid / 8));
+    }
+    return plan;
+}
+
+// The plan of single solves, kept with the matrix's tiles.
+const ResidentPlan &resident_plan(Device &d, Matrix &m, int nc, bool mixed) {
+    ResidentPlan &plan = m.res_plan[2 * (nc - 1) + (mixed ? 1 : 0)];
+    if (!plan.made) {
+        plan = plan_resident(m, nc, mixed, 0, d.cu_count);
+        plan.made = true;
+    }
+    return plan;
+}
+
+// Whether a solve may take the resident form: not when a comparison run asks
+// for one of the streaming forms (NSFEM_CG_RESIDENT=0, or the form's own
+// switches; read at every solve).
+bool want_resident(int nc, bool mixed) {
+    const char *e = std::getenv("NSFEM_CG_RESIDENT");
+    if (e && std::atoi(e) == 0) return false;
+    if (!mixed) return true;
+    if (nc == 1) return !std::getenv("NSFEM_CG_PHASE") && !std::getenv("NSFEM_CG_BLOCK");
+    return !std::getenv("NSFEM_CG_PAIRED") && !std::getenv("NSFEM_CG_P2_BLOCK") &&
+           !std::getenv("NSFEM_CG_P2_LOADS");
+}
+
 }  // namespace
 
 
@@ -3598,9 +4216,21 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
         const char *env = std::getenv("NSFEM_CG_GRID");
         if (env) want = std::atoi(env);
     }
+    // (the one-column mixed form shares its grid with its resident form)
+    const int per_wave = mixed && nc == 1 ? cg_tiles_per_wave(m) : 2;
     int grid = want > 0 ? std::min(want, maxg)
-                        : std::min(maxg, std::max(1, m.n_wtiles / (2 * (bs / 64))));
+                        : std::min(maxg, std::max(1, m.n_wtiles / (per_wave * (bs / 64))));
     grid = std::max(1, std::min(grid, std::max(1, m.n_wtiles)));
+    ResidentPlan res;
+    if (want_resident(nc, mixed))
+        res = want > 0 ? plan_resident(m, nc, mixed, want, d.cu_count)
+                       : resident_plan(d, m, nc, mixed);
+    if (res.ok) {
+        ResMaxGrid rg{d, res.lds, false, 0};
+        res_dispatch(nc, mixed, res.width, res.tiles, rg);
+        res.ok = rg.out >= res.grid;
+        if (res.ok) grid = res.grid;
+    }
     const bool verbose = std::getenv("NSFEM_CG_VERBOSE") != nullptr;
     ensure_block_tiles(d, m, grid);
 
@@ -3610,6 +4240,7 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
 
     CgArgs a{};
     a.n = n;
+    a.nnz = (int)m.nnz;
     a.meta = m.wmeta.ptr;
     a.tiles = m.wtiles.ptr;
     a.block_tiles = m.block_tiles.ptr;
@@ -3631,20 +4262,30 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
     set_cg_params(d, req, n, a);
     a.sync = ws.sync;
     a.res = ws.res;
+    a.band_lo = m.band_lo;
+    a.band_hi = m.band_hi;
+    a.win_cap = res.cap;
     const int ngroups = (grid + kGroup - 1) / kGroup;
 
     for (int attempt = 0; attempt < 3; ++attempt) {
         if (verbose)  // one line per launch, in launch order
             std::fprintf(stderr,
                          "[nsfem] cg launch matrix=%p rows=%d cols=%d wave tiles=%d grid=%d "
-                         "maxgrid=%d mixed=%d idx16=%d form=%d block=%d attempt=%d\n",
+                         "maxgrid=%d mixed=%d idx16=%d form=%d block=%d resident=%d attempt=%d\n",
                          (const void *)&m, n, nc, m.n_wtiles, grid, maxg, (int)mixed, (int)idx16,
-                         wi, bs, attempt);
+                         wi, res.ok ? kResBlock : bs, res.ok ? res.width : 0, attempt);
         NSFEM_HIP(hipEventRecord(d.ev_start, d.stream));
-        k_sync_reset<<<(ngroups + 255) / 256, 256, 0, d.stream>>>(a.sync, ngroups);
+        k_sync_reset<<<(ngroups + 255) / 256, 256, 0, d.stream>>>(a.sync, ngroups,
+                                                                  res.ok ? grid : 0);
         NSFEM_HIP(hipGetLastError());
-        CgLaunch ln{d, a, grid, bs, p2, ib};
-        cg_dispatch(nc, mixed, idx16, wi, ln);
+        if (res.ok) {
+            void *kargs[] = {(void *)&a};
+            res_dispatch(nc, mixed, res.width, res.tiles,
+                         ResLaunch{d, kargs, grid, res.lds, false});
+        } else {
+            CgLaunch ln{d, a, grid, bs, p2, ib};
+            cg_dispatch(nc, mixed, idx16, wi, ln);
+        }
         NSFEM_HIP(hipEventRecord(d.ev_stop, d.stream));
         NSFEM_HIP(hipMemcpyAsync(P.res, ws.res, sizeof(CgColumnResult) * nc,
                                  hipMemcpyDeviceToHost, d.stream));
@@ -3912,6 +4553,7 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
             CgArgs &a = args[i];
             a = CgArgs{};
             a.n = m.rows;
+            a.nnz = (int)m.nnz;
             a.meta = m.wmeta.ptr;
             a.tiles = m.wtiles.ptr;
             a.block_tiles = m.block_tiles.ptr;
@@ -3943,7 +4585,7 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
                                  hipMemcpyHostToDevice, d.stream));
         for (size_t i = 0; i < I; ++i) {
             const int ng = (nb[i] + kGroup - 1) / kGroup;
-            k_sync_reset<<<(ng + 255) / 256, 256, 0, d.stream>>>(args[i].sync, ng);
+            k_sync_reset<<<(ng + 255) / 256, 256, 0, d.stream>>>(args[i].sync, ng, 0);
         }
         NSFEM_HIP(hipGetLastError());
         NSFEM_HIP(hipEventRecord(d.ev_start, d.stream));

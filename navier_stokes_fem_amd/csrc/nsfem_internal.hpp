@@ -110,6 +110,16 @@ constexpr int kWaveNnz = 512;   // LDS room of a wave tile's products
 constexpr int kStageNnz = kWaveNnz - 8;
 constexpr int kMaxGridBlocks = 4096;
 
+// How a solve runs on a matrix in the persistent CG's resident form.
+struct ResidentPlan {
+    bool made = false, ok = false;
+    int width = 0;   // nonzeros a row's registers hold
+    int tiles = 0;   // wave tiles of a wave, at most
+    int grid = 0;    // blocks
+    int cap = 0;     // rows of the largest block window
+    size_t lds = 0;  // bytes of dynamic LDS
+};
+
 struct Matrix {
     int rows = 0, cols = 0;
     int64_t nnz = 0;
@@ -125,6 +135,11 @@ struct Matrix {
     std::vector<int32_t> host_rs;            // row_start (wave tiles are rebuilt from it)
     int wave_rows = kWaveRows, wave_nnz = kWaveNnz;  // current wave-tile shape
     int max_multirow_nz = 0;  // most nonzeros of a wave tile with more than one row
+    std::vector<int32_t> host_wtiles;  // [n_wtiles + 1] first row of each wave tile
+    // square matrices: most nonzeros of a row, most columns below and above
+    // the diagonal, and the resident solves' plans by columns and precision
+    int max_row_nz = 0, band_lo = 0, band_hi = 0;
+    ResidentPlan res_plan[4];
     // ownership of wave tiles by persistent blocks, cached per grid size:
     // both arrays hold kMaxGridBlocks + 1 entries from the tiling on, so a
     // change of grid size copies and never allocates

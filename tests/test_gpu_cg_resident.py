@@ -1,0 +1,149 @@
+"""The resident form of the CG (the matrix in the blocks' registers, p in an
+LDS window, the sums and q crossing blocks at the coherence point) against the
+streaming forms, at the sizes where its tiles, windows and grids end.
+
+The one-column mixed form has the streaming form's products, sums and grid:
+bit-identical.  The others reach the same tolerance by another order of sums:
+the true residual is checked, and the iteration counts agree to a few."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def banded(n, offsets, seed, empty=()):
+    """A strictly diagonally dominant symmetric matrix with these sub- and
+    superdiagonals; rows in `empty` hold their diagonal alone."""
+    rng = np.random.default_rng(seed)
+    rows, cols, vals = [np.arange(n)], [np.arange(n)], [np.full(n, 1.0 + 2.02 * len(offsets))]
+    lone = np.zeros(n, bool)
+    lone[[e for e in empty if e < n]] = True
+    for o in offsets:
+        i = np.arange(max(n - o, 0))
+        i = i[~lone[i] & ~lone[i + o]]
+        v = -rng.uniform(0.5, 1.0, len(i))
+        rows += [i, i + o]
+        cols += [i + o, i]
+        vals += [v, v]
+    r, c, v = np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    order = np.lexsort((c, r))
+    rs = np.zeros(n + 1, np.int64)
+    np.cumsum(np.bincount(r, minlength=n), out=rs[1:])
+    return rs.astype(np.int32), c[order].astype(np.int32), v[order]
+
+
+def solve(gpu, A, b, x0, columns, precision, capfd, rtol=1e-10, max_iterations=-1):
+    gpu.upload_csr(6, *A)
+    bb, bx = gpu.buffer(b), gpu.buffer(x0)
+    capfd.readouterr()
+    st = gpu.cg_solve(6, bb, bx, columns=columns, rtol=rtol, precision=precision,
+                      max_iterations=max_iterations, raise_on_error=False)
+    resident = "resident=0" not in capfd.readouterr().err
+    x = bx.download()
+    bb.close()
+    bx.close()
+    return x, st, resident
+
+
+# (rows, off-diagonals): one row; less than a wave; the edges of a wave tile;
+# two and three tiles a wave of one block; several blocks with windows that
+# reach past them; rows of 19 nonzeros (the long-row kernels), 20 and of all
+# lengths
+SYSTEMS = [(1, ()), (2, (1,)), (63, (1, 5)), (64, (1, 5)), (65, (1, 5)), (767, (1, 2, 30)),
+           (1600, (1, 40, 41)), (6000, (1, 60, 61)), (20011, (1, 140, 141)),
+           (1100, tuple(range(1, 10))), (9000, (1, 2, 3, 90, 91, 92, 180, 181, 182)),
+           (700, (1, 2, 3, 4, 5, 6, 7, 8, 600))]
+
+
+@pytest.mark.parametrize("columns,precision", [(1, "fp64"), (2, "fp64"), (1, "fp32_refined"),
+                                               (2, "fp32_refined")])
+@pytest.mark.parametrize("n,offsets", SYSTEMS, ids=lambda v: str(v) if isinstance(v, int) else None)
+def test_resident_equals_streaming(gpu, oracle, monkeypatch, capfd, n, offsets, columns, precision):
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    A = banded(n, offsets, n, empty=(0, 64, 65, 1023))
+    rng = np.random.default_rng(n + 1)
+    b = rng.standard_normal(columns * n)
+    b[n:] *= 7.0
+    x0 = 0.1 * rng.standard_normal(columns * n)
+    got, st, resident = solve(gpu, A, b, x0, columns, precision, capfd, max_iterations=1000)
+    assert resident
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", "0")
+    want, ref, resident = solve(gpu, A, b, x0, columns, precision, capfd, max_iterations=1000)
+    assert not resident
+    if columns == 1 and precision == "fp32_refined":
+        np.testing.assert_array_equal(got, want)
+        assert [s["iterations"] for s in st] == [s["iterations"] for s in ref]
+        assert [s["refinements"] for s in st] == [s["refinements"] for s in ref]
+    for c in range(columns):
+        bc, xc = b[c * n:(c + 1) * n], got[c * n:(c + 1) * n]
+        assert st[c]["status"] == 0 and ref[c]["status"] == 0
+        r = np.linalg.norm(oracle.spmv_sub(A, bc, xc))
+        assert r <= 1e-10 * np.linalg.norm(bc) * (1 + 1e-9)
+        assert abs(st[c]["final_residual"] - r) <= 1e-3 * r + 1e-13 * np.linalg.norm(bc)
+        assert abs(st[c]["iterations"] - ref[c]["iterations"]) <= 2 + 0.1 * ref[c]["iterations"]
+        assert st[c]["rhs_norm"] == pytest.approx(ref[c]["rhs_norm"], rel=1e-13)
+        assert st[c]["initial_residual"] == pytest.approx(ref[c]["initial_residual"], rel=1e-12)
+
+
+@pytest.mark.parametrize("grid", ["1", "3", "97", "256"])
+def test_resident_grids(gpu, oracle, monkeypatch, capfd, grid):
+    """One system over few and many blocks, at most one wave tile a wave and
+    several words a polling lane."""
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    n = 3000 if grid == "1" else 8500 if grid == "3" else 30011
+    A = banded(n, (1, 170, 171), 5)
+    b = np.random.default_rng(6).standard_normal(n)
+    monkeypatch.setenv("NSFEM_CG_GRID", grid)
+    for precision in ("fp64", "fp32_refined"):
+        x, st, resident = solve(gpu, A, b, np.zeros(n), 1, precision, capfd)
+        assert resident and st[0]["status"] == 0
+        assert np.linalg.norm(oracle.spmv_sub(A, b, x)) <= 1e-10 * np.linalg.norm(b) * (1 + 1e-9)
+
+
+def test_systems_that_stay_streaming(gpu, monkeypatch, capfd):
+    """A row of 21 nonzeros, a window past the LDS and an explicit streaming
+    form keep the streaming kernels."""
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    b = np.random.default_rng(7).standard_normal(60000)
+    for n, offsets in ((500, tuple(range(1, 11))), (60000, (1, 30000))):
+        A = banded(n, offsets, 8)
+        _, st, resident = solve(gpu, A, b[:n], np.zeros(n), 1, "fp64", capfd)
+        assert not resident and st[0]["status"] == 0
+    A = banded(500, (1, 9), 9)
+    monkeypatch.setenv("NSFEM_CG_PHASE", "items")
+    _, st, resident = solve(gpu, A, b[:500], np.zeros(500), 1, "fp32_refined", capfd)
+    assert not resident and st[0]["status"] == 0
+
+
+@pytest.mark.parametrize("columns,precision", [(1, "fp64"), (2, "fp64"), (1, "fp32_refined"),
+                                               (2, "fp32_refined")])
+def test_resident_ends_as_streaming(gpu, monkeypatch, capfd, columns, precision):
+    """Ends other than convergence: the iteration limit with the last iterate,
+    a matrix that is not positive definite, a zero right-hand side, a guess
+    that is the solution, infinities and NaN in the right-hand side."""
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    n = 4000
+    A = banded(n, (1, 50, 51), 11)
+    neg = (A[0], A[1], -A[2])
+    rng = np.random.default_rng(12)
+    b = rng.standard_normal(columns * n)
+    zero = np.zeros(columns * n)
+    inf, nan = b.copy(), b.copy()
+    inf[17] = np.inf
+    nan[-5] = np.nan
+    cases = [(A, b, zero, 3), (neg, b, zero, -1), (A, zero, zero, -1), (A, zero, b, -1),
+             (A, inf, zero, 40), (A, nan, zero, 40)]
+    for i, (M, rhs, x0, limit) in enumerate(cases):
+        monkeypatch.delenv("NSFEM_CG_RESIDENT", raising=False)
+        got, st, resident = solve(gpu, M, rhs, x0, columns, precision, capfd, 1e-12, limit)
+        assert resident
+        monkeypatch.setenv("NSFEM_CG_RESIDENT", "0")
+        want, ref, _ = solve(gpu, M, rhs, x0, columns, precision, capfd, 1e-12, limit)
+        assert [s["status"] for s in st] == [s["status"] for s in ref], i
+        assert [s["iterations"] for s in st] == [s["iterations"] for s in ref], i
+        same = np.isfinite(got) == np.isfinite(want)
+        assert same.all(), i
+        fine = np.isfinite(want)
+        # a few steps from the same start: only the sums' order differs
+        np.testing.assert_allclose(got[fine], want[fine], rtol=1e-4 if i == 1 else 1e-6,
+                                   atol=1e-9 * (1 + np.abs(want[fine]).max(initial=0.0)))
