@@ -4458,19 +4458,17 @@ inline size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 // Poisson-type solve growing like the mesh width (tiles^0.5).  So the
 // largest system, which needs the most iterations, does not become the
 // batch's critical path on a fair share.
-std::vector<int> split_blocks(const std::vector<const CgRequest *> &rq, int maxg, int scale) {
+std::vector<int> share_blocks(const std::vector<const CgRequest *> &rq, int maxg,
+                              const std::vector<int> &want, std::vector<int> nb) {
     const size_t I = rq.size();
-    std::vector<int> want(I), nb(I, 1);
     std::vector<double> work(I);
-    int64_t total = 0;
+    int64_t total = 0, left = maxg;
     for (size_t i = 0; i < I; ++i) {
-        const int tiles = std::max(1, rq[i]->m->n_wtiles);
-        want[i] = std::min(tiles, std::max(1, tiles * scale / 32));
-        work[i] = std::pow((double)tiles, 1.5);
+        work[i] = std::pow((double)std::max(1, rq[i]->m->n_wtiles), 1.5);
         total += want[i];
+        left -= nb[i];
     }
     if (total <= maxg) return want;
-    int64_t left = maxg - (int64_t)I;
     while (left > 0) {
         size_t big = I;
         double worst = -1.0;
@@ -4487,6 +4485,98 @@ std::vector<int> split_blocks(const std::vector<const CgRequest *> &rq, int maxg
         --left;
     }
     return nb;
+}
+
+std::vector<int> split_blocks(const std::vector<const CgRequest *> &rq, int maxg, int scale) {
+    std::vector<int> want(rq.size());
+    for (size_t i = 0; i < rq.size(); ++i) {
+        const int tiles = std::max(1, rq[i]->m->n_wtiles);
+        want[i] = std::min(tiles, std::max(1, tiles * scale / 32));
+    }
+    return share_blocks(rq, maxg, want, std::vector<int>(rq.size(), 1));
+}
+
+// One launch of a batch: its requests' numbers, the blocks of each and, for
+// the resident form, what its kernel and windows hold.
+struct BatchLaunch {
+    std::vector<size_t> which;
+    std::vector<int> blocks;
+    std::vector<int> cap;
+    bool resident = false;
+    int width = 0, tiles = 0;
+    size_t lds = 0;
+};
+
+// The launches of a batch in the resident form, or none when a system does
+// not allow it.  Systems go largest first, so that those of like iteration
+// counts share a launch, each with the fewest blocks it fits in; a launch's
+// other blocks go where share_blocks sends them, up to a single solve's.
+std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgRequest> &reqs, int nc,
+                                           bool mixed, int scale) {
+    std::vector<BatchLaunch> out;
+    if (!want_resident(nc, mixed)) return out;
+    int w = nc == 1 ? kResRowShort : kResRowLong;
+    for (const CgRequest &r : reqs) {
+        const Matrix &m = *r.m;
+        if (m.nnz <= 0 || m.max_row_nz > kResRowLong || m.n_wtiles < 1) return out;
+        if (m.max_row_nz > kResRowShort) w = kResRowLong;
+    }
+    const int room = kResWaves * res_tiles(mixed, w);
+    int maxg = 0;
+    {
+        ResMaxGrid mg{d, kResLds, true, 0};
+        res_dispatch(nc, mixed, w, res_tiles(mixed, w), mg);
+        maxg = mg.out;
+    }
+    std::vector<size_t> order(reqs.size());
+    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+    std::sort(order.begin(), order.end(), [&](size_t a, size_t b) {
+        return reqs[a].m->n_wtiles != reqs[b].m->n_wtiles
+                   ? reqs[a].m->n_wtiles > reqs[b].m->n_wtiles
+                   : a < b;
+    });
+    std::vector<int> least(reqs.size());
+    int used = maxg + 1;
+    for (size_t i : order) {
+        const Matrix &m = *reqs[i].m;
+        ResidentPlan plan;
+        int g = (m.n_wtiles + room - 1) / room;
+        while (g <= std::min(maxg, m.n_wtiles) && !res_fits(m, nc, mixed, w, g, plan)) ++g;
+        if (!plan.ok) return std::vector<BatchLaunch>();
+        least[i] = g;
+        if (used + g > maxg) {
+            out.emplace_back();
+            used = 0;
+        }
+        used += g;
+        out.back().which.push_back(i);
+    }
+    for (BatchLaunch &l : out) {
+        std::vector<const CgRequest *> rq;
+        std::vector<int> want, nb;
+        for (size_t i : l.which) {
+            const Matrix &m = *reqs[i].m;
+            rq.push_back(&reqs[i]);
+            nb.push_back(least[i]);
+            want.push_back(std::max(
+                least[i], std::min(m.n_wtiles, scale * m.n_wtiles /
+                                                   (cg_tiles_per_wave(m) * kResWaves))));
+        }
+        l.blocks = share_blocks(rq, maxg, want, nb);
+        l.resident = true;
+        l.width = w;
+        for (size_t k = 0; k < rq.size(); ++k) {
+            ResidentPlan plan;
+            if (!res_fits(*rq[k]->m, nc, mixed, w, l.blocks[k], plan)) {
+                l.blocks[k] = nb[k];
+                res_fits(*rq[k]->m, nc, mixed, w, nb[k], plan);
+            }
+            l.cap.push_back(plan.cap);
+            l.tiles = std::max(l.tiles, plan.tiles);
+            l.lds = std::max(l.lds, plan.lds);
+        }
+    }
+    return out;
 }
 
 }  // namespace
@@ -4507,27 +4597,42 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
         NSFEM_REQUIRE(nc == 1 || nc == 2, NSFEM_INVALID_ARGUMENT, "columns must be 1 or 2");
     }
     bool idx16 = want_idx16();
-    // batched launches run 1024-thread blocks: one load per nonzero per
-    // lane unless NSFEM_CG_PHASE says otherwise
-    int form = mixed && nc == 1 ? phase_form(*reqs[0].m, false) : -1;
     int wi = 4;
-    for (const CgRequest &r : reqs) {
-        idx16 = idx16 && r.m->dcol_ok;
-        if (phase_form(*r.m, false) != form) form = -1;
-        wi = std::max(wi, items_per_lane(*r.m));
+    std::vector<BatchLaunch> launches =
+        resident_launches(d, reqs, nc, mixed, std::max(1, block_scale));
+    if (launches.empty()) {
+        // batched launches run 1024-thread blocks: one load per nonzero per
+        // lane unless NSFEM_CG_PHASE says otherwise
+        int form = mixed && nc == 1 ? phase_form(*reqs[0].m, false) : -1;
+        for (const CgRequest &r : reqs) {
+            idx16 = idx16 && r.m->dcol_ok;
+            if (phase_form(*r.m, false) != form) form = -1;
+            wi = std::max(wi, items_per_lane(*r.m));
+        }
+        if (form >= 0 && idx16) wi = form;
+        CgBatchMaxGrid mg{d, 0};
+        cg_dispatch(nc, mixed, idx16, wi, mg);
+        const int maxg = mg.out;
+        // instances beyond the co-resident block count run in further launches
+        for (size_t first = 0; first < reqs.size(); first += (size_t)maxg) {
+            BatchLaunch l;
+            std::vector<const CgRequest *> rq;
+            for (size_t i = first; i < std::min(reqs.size(), first + (size_t)maxg); ++i) {
+                l.which.push_back(i);
+                rq.push_back(&reqs[i]);
+            }
+            l.blocks = split_blocks(rq, maxg, std::max(1, block_scale));
+            l.cap.assign(rq.size(), 0);
+            launches.push_back(std::move(l));
+        }
     }
-    if (form >= 0 && idx16) wi = form;
-    CgBatchMaxGrid mg{d, 0};
-    cg_dispatch(nc, mixed, idx16, wi, mg);
-    const int maxg = mg.out;
     int worst = NSFEM_OK;
     const size_t vt = mixed ? sizeof(float) : sizeof(double);
-    // instances beyond the co-resident block count run in further launches
-    for (size_t first = 0; first < reqs.size(); first += (size_t)maxg) {
-        const size_t I = std::min(reqs.size() - first, (size_t)maxg);
+    for (const BatchLaunch &launch : launches) {
+        const size_t I = launch.which.size();
         std::vector<const CgRequest *> rq(I);
-        for (size_t i = 0; i < I; ++i) rq[i] = &reqs[first + i];
-        const std::vector<int> nb = split_blocks(rq, maxg, std::max(1, block_scale));
+        for (size_t i = 0; i < I; ++i) rq[i] = &reqs[launch.which[i]];
+        const std::vector<int> &nb = launch.blocks;
         // per-instance memory
         std::vector<size_t> voff(I), vbytes(I);
         size_t work = 0;
@@ -4574,10 +4679,12 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
             a.sync = reinterpret_cast<SyncState *>(sm + i * sync_bytes);
             a.res = d.batch_res.ptr + 2 * i;
             a.nblocks = nb[i];
+            a.band_lo = m.band_lo;
+            a.band_hi = m.band_hi;
+            a.win_cap = launch.cap[i];
             for (int k = 0; k < nb[i]; ++k) map.push_back(make_int2((int)i, k));
         }
         const int grid = (int)map.size();
-        NSFEM_REQUIRE(grid <= maxg, NSFEM_ERROR, "batched CG: block split exceeds co-residency");
         d.batch_map.ensure(map.size());
         NSFEM_HIP(hipMemcpyAsync(d.batch_args.ptr, args.data(), sizeof(CgArgs) * I,
                                  hipMemcpyHostToDevice, d.stream));
@@ -4585,13 +4692,25 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
                                  hipMemcpyHostToDevice, d.stream));
         for (size_t i = 0; i < I; ++i) {
             const int ng = (nb[i] + kGroup - 1) / kGroup;
-            k_sync_reset<<<(ng + 255) / 256, 256, 0, d.stream>>>(args[i].sync, ng, 0);
+            k_sync_reset<<<(ng + 255) / 256, 256, 0, d.stream>>>(args[i].sync, ng,
+                                                                  launch.resident ? nb[i] : 0);
         }
         NSFEM_HIP(hipGetLastError());
         NSFEM_HIP(hipEventRecord(d.ev_start, d.stream));
         const CgArgs *dargs = reinterpret_cast<const CgArgs *>(d.batch_args.ptr);
-        CgBatchLaunch ln{d, dargs, d.batch_map.ptr, grid};
-        cg_dispatch(nc, mixed, idx16, wi, ln);
+        const int2 *dmap = d.batch_map.ptr;
+        if (launch.resident) {
+            void *kargs[] = {(void *)&dargs, (void *)&dmap};
+            ResMaxGrid mg{d, launch.lds, true, 0};
+            res_dispatch(nc, mixed, launch.width, launch.tiles, mg);
+            NSFEM_REQUIRE(grid <= mg.out, NSFEM_ERROR,
+                          "batched CG: block split exceeds co-residency");
+            res_dispatch(nc, mixed, launch.width, launch.tiles,
+                         ResLaunch{d, kargs, grid, launch.lds, true});
+        } else {
+            CgBatchLaunch ln{d, dargs, dmap, grid};
+            cg_dispatch(nc, mixed, idx16, wi, ln);
+        }
         NSFEM_HIP(hipEventRecord(d.ev_stop, d.stream));
         // FP64 true residuals of every instance, one host synchronisation
         if (!mixed) {
@@ -4626,7 +4745,7 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
                     fail(NSFEM_BARRIER_TIMEOUT, "batched CG kernel barrier timed out");
                 const double fin = mixed ? cr.last_residual : std::sqrt(tres[nc * i + c]);
                 if (cr.status != NSFEM_OK || fin > cr.tolerance * (1.0 + 1e-12)) redo = true;
-                nsfem_cg_stats &st = stats[2 * (first + i) + c];
+                nsfem_cg_stats &st = stats[2 * launch.which[i] + c];
                 st.iterations = cr.iterations;
                 st.refinements = cr.refinements;
                 st.status = cr.status;
@@ -4651,7 +4770,7 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
                 nsfem_cg_stats s2[2]{};
                 const int st2 = run_cg(d, r2, s2);
                 for (int c = 0; c < nc; ++c) {
-                    nsfem_cg_stats &st = stats[2 * (first + i) + c];
+                    nsfem_cg_stats &st = stats[2 * launch.which[i] + c];
                     st.iterations += s2[c].iterations;
                     st.refinements += s2[c].refinements + 1;
                     st.status = s2[c].status;
