@@ -810,6 +810,12 @@ __global__ void k_scatter(int count, const int32_t *__restrict__ idx,
     if (i < count) dst[idx[i]] = val[i];
 }
 
+__global__ void k_gather(int count, const int32_t *__restrict__ idx,
+                         const double *__restrict__ src, double *__restrict__ dst) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) dst[i] = src[idx[i]];
+}
+
 template <typename T>
 __global__ void k_scatter_value(int count, const int32_t *__restrict__ idx, T v,
                                 T *__restrict__ dst) {
@@ -1118,6 +1124,12 @@ void launch_dot_accumulate(Device &d, int n, const double *a, const double *b,
 void launch_scatter(Device &d, int count, const int32_t *idx, const double *val, double *dst) {
     if (count <= 0) return;
     k_scatter<<<(count + kBlock - 1) / kBlock, kBlock, 0, d.stream>>>(count, idx, val, dst);
+    NSFEM_HIP(hipGetLastError());
+}
+
+void launch_gather(Device &d, int count, const int32_t *idx, const double *src, double *dst) {
+    if (count <= 0) return;
+    k_gather<<<(count + kBlock - 1) / kBlock, kBlock, 0, d.stream>>>(count, idx, src, dst);
     NSFEM_HIP(hipGetLastError());
 }
 

@@ -331,6 +331,8 @@ void build_tri_xy(Device &d, KdTreeGpu &t);
 // elementwise helpers for the step driver
 void launch_scatter(Device &d, int count, const int32_t *idx, const double *val,
                     double *dst);
+// dst[i] = src[idx[i]]
+void launch_gather(Device &d, int count, const int32_t *idx, const double *src, double *dst);
 void launch_scatter_value(Device &d, int count, const int32_t *idx, double v,
                           double *dst);  // dst[idx[i]] = v
 void launch_scatter_value(Device &d, int count, const int32_t *idx, double v, float *dst);
