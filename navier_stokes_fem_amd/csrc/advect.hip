@@ -14,9 +14,23 @@
 //
 // Layout in HBM: tree nodes as 8-byte pairs (flags, split|offset) in the
 // reference's KDNode layout, leaf triangle indices, node coordinates as
-// float2, elements as 6 ints, plus tri_xy: the 3 vertex coordinates of each
-// element (24 bytes) so that a leaf test reads one contiguous record
-// instead of three indices and three dependent coordinate gathers.
+// float2, elements as 6 ints, plus tri: each element as the point test uses
+// it, {A, B - A} and {C - A, D} (the test's own float operations on the
+// corners, done once), 32 bytes.
+//
+// Bound by the vector-memory instructions, whatever their width: some 14
+// triangles of a leaf for the slowest lane of a wave, 18 levels of descent
+// and the six nodes' velocities.  A leaf's indices are read four at a time
+// and a triangle with two loads, the next one's already in flight: 2.25
+// instructions a triangle where an index and three corners took 4: on the
+// 1024^2 cavity 288 -> 233 us (225 -> 194 in lattice order) over one state's
+// fields, 253 -> 238 over changing ones, whose tree comes from memory; 16,641
+// nodes 7.9 -> 7.5.  Records
+// in leaf order (no index at all) were slower, 307 against 255 us on the
+// 1024^2 cavity: a triangle stands in four leaves, so they take four times
+// the cache.  Walking the levels that a wave's points share once for the wave
+// gained 3% there and lost 6% on 16,641 nodes, a node and its left child in
+// one load gained 2% and lost 12%.
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
@@ -33,15 +47,17 @@ struct TreeView {
     const int32_t *leaf;
     const float2 *xy;
     const int32_t *elem;
-    const float2 *tri;  // 3 float2 per element
+    const float4 *tri;  // 2 per element: {A, AB}, {AC, D, unused}
 };
 
-__device__ __forceinline__ bool point_in_triangle(float px, float py, float2 A, float2 B,
-                                                  float2 Cc, float &xi, float &eta) {
-    const float abx = B.x - A.x, aby = B.y - A.y;
-    const float acx = Cc.x - A.x, acy = Cc.y - A.y;
-    const float apx = px - A.x, apy = py - A.y;
-    const float D = (abx * acy) - (aby * acx);
+// four leaf indices, at any leaf offset
+typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// isPointInTriagle on an element's record {A, AB}, {AC, D}.
+__device__ __forceinline__ bool point_in_triangle(float px, float py, float4 a, float4 c,
+                                                  float &xi, float &eta) {
+    const float abx = a.z, aby = a.w, acx = c.x, acy = c.y, D = c.z;
+    const float apx = px - a.x, apy = py - a.y;
     const float dsign = D > 0 ? 1.0f : -1.0f;
     const float b1 = (apx * acy - apy * acx) * dsign;
     if (b1 < 0 || b1 > D) return false;
@@ -132,10 +148,27 @@ __device__ __forceinline__ int find_element(const TreeView &T, float px, float p
         nd = T.nodes[cur];
     }
     const int off = (int)nd.y, cnt = (int)(nd.x >> 2);
-    for (int i = 0; i < cnt; ++i) {
-        const int e = T.leaf[off + i];
-        const float2 a = T.tri[3 * e], b = T.tri[3 * e + 1], c = T.tri[3 * e + 2];
-        if (point_in_triangle(px, py, a, b, c, xi, eta)) return e;
+    if (cnt > 0) {
+        // (the index array has entries to read past its last leaf)
+        i32x4u q = *reinterpret_cast<const i32x4u *>(T.leaf + off);
+        float4 a = T.tri[2 * (size_t)q[0]], c = T.tri[2 * (size_t)q[0] + 1];
+        for (int i = 0; i < cnt; i += 4) {
+            i32x4u qn = q;
+            if (i + 4 < cnt) qn = *reinterpret_cast<const i32x4u *>(T.leaf + off + i + 4);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int e = q[u];
+                const float4 ae = a, ce = c;
+                if (i + u + 1 < cnt) {
+                    const size_t next = 2 * (size_t)(u < 3 ? q[u < 3 ? u + 1 : 3] : qn[0]);
+                    a = T.tri[next];
+                    c = T.tri[next + 1];
+                }
+                if (point_in_triangle(px, py, ae, ce, xi, eta)) return e;
+                if (i + u + 1 >= cnt) break;
+            }
+            q = qn;
+        }
     }
     nearest = nn_search(T, px, py);
     return -1;
@@ -243,30 +276,34 @@ __global__ __launch_bounds__(256) void k_locate(TreeView T, int n, const float2 
     nearest[i] = e >= 0 ? -1 : nn;
 }
 
-__global__ void k_tri_xy(int ne, const int32_t *__restrict__ elem, const float2 *__restrict__ xy,
-                         float2 *__restrict__ tri) {
+__global__ void k_tri(int ne, const int32_t *__restrict__ elem, const float2 *__restrict__ xy,
+                      float4 *__restrict__ tri) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= ne) return;
-    tri[3 * e] = xy[elem[6 * e]];
-    tri[3 * e + 1] = xy[elem[6 * e + 1]];
-    tri[3 * e + 2] = xy[elem[6 * e + 2]];
+    const int32_t *v = elem + 6 * (size_t)e;
+    const float2 A = xy[v[0]], B = xy[v[1]], Cc = xy[v[2]];
+    const float abx = B.x - A.x, aby = B.y - A.y;
+    const float acx = Cc.x - A.x, acy = Cc.y - A.y;
+    const float D = (abx * acy) - (aby * acx);
+    tri[2 * (size_t)e] = make_float4(A.x, A.y, abx, aby);
+    tri[2 * (size_t)e + 1] = make_float4(acx, acy, D, 0.f);
 }
 
 TreeView view(const KdTreeGpu &t) {
     NSFEM_REQUIRE(t.ready, NSFEM_NOT_READY, "KD tree not uploaded");
     return TreeView{reinterpret_cast<const uint2 *>(t.nodes.ptr), t.leaf.ptr,
                     reinterpret_cast<const float2 *>(t.xy.ptr), t.elements.ptr,
-                    reinterpret_cast<const float2 *>(t.tri_xy.ptr)};
+                    reinterpret_cast<const float4 *>(t.tri.ptr)};
 }
 
 }  // namespace
 
-void build_tri_xy(Device &d, KdTreeGpu &t) {
-    t.tri_xy.resize((size_t)t.elements_count * 6);
+void build_tri(Device &d, KdTreeGpu &t) {
+    t.tri.resize((size_t)t.elements_count * 8);
     if (t.elements_count == 0) return;
-    k_tri_xy<<<(t.elements_count + 255) / 256, 256, 0, d.stream>>>(
+    k_tri<<<(t.elements_count + 255) / 256, 256, 0, d.stream>>>(
         t.elements_count, t.elements.ptr, reinterpret_cast<const float2 *>(t.xy.ptr),
-        reinterpret_cast<float2 *>(t.tri_xy.ptr));
+        reinterpret_cast<float4 *>(t.tri.ptr));
     NSFEM_HIP(hipGetLastError());
 }
 

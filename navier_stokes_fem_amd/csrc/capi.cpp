@@ -127,7 +127,7 @@ void upload_tree(Device &d, KdTreeGpu &t, int32_t tn, const uint32_t *w, int64_t
     d.set_current();
     t.ready = false;
     t.nodes.resize(2 * (size_t)tn);
-    t.leaf.resize((size_t)std::max<int64_t>(lc, 1));
+    t.leaf.resize((size_t)lc + 4);  // leaves are read four entries at a time
     t.xy.resize(2 * (size_t)V);
     t.elements.resize(6 * (size_t)E);
     NSFEM_HIP(hipMemcpy(t.nodes.ptr, w, sizeof(uint32_t) * 2 * tn, hipMemcpyHostToDevice));
@@ -138,7 +138,7 @@ void upload_tree(Device &d, KdTreeGpu &t, int32_t tn, const uint32_t *w, int64_t
     t.leaf_count = lc;
     t.mesh_nodes = V;
     t.elements_count = E;
-    build_tri_xy(d, t);
+    build_tri(d, t);
     NSFEM_HIP(hipStreamSynchronize(d.stream));
     t.ready = true;
     if (&t == &d.tree) {

@@ -187,7 +187,7 @@ struct KdTreeGpu {
     DeviceArray<int32_t> leaf;       // leaf triangle indices
     DeviceArray<float> xy;           // 2 per mesh node
     DeviceArray<int32_t> elements;   // 6 per element
-    DeviceArray<float> tri_xy;       // 6 per element: vertex coordinates
+    DeviceArray<float> tri;       // 8 words per element (advect.hip)
     int32_t node_count = 0;          // tree nodes
     int64_t leaf_count = 0;
     int mesh_nodes = 0;
@@ -195,7 +195,7 @@ struct KdTreeGpu {
     bool ready = false;
 };
 inline void kdtree_release(KdTreeGpu &t) {
-    t.nodes.release(); t.leaf.release(); t.xy.release(); t.elements.release(); t.tri_xy.release();
+    t.nodes.release(); t.leaf.release(); t.xy.release(); t.elements.release(); t.tri.release();
     t.ready = false;
 }
 
@@ -326,7 +326,7 @@ void launch_advect_f64(Device &d, const KdTreeGpu &t, int n, const double *u, co
                        double *uo, double *vo);
 void launch_locate(Device &d, const KdTreeGpu &t, int n, const float *pts, int32_t *elem, float *xi,
                    float *eta, int32_t *nearest);
-void build_tri_xy(Device &d, KdTreeGpu &t);
+void build_tri(Device &d, KdTreeGpu &t);
 
 // elementwise helpers for the step driver
 void launch_scatter(Device &d, int count, const int32_t *idx, const double *val,
