@@ -218,6 +218,26 @@ struct GnnNet;
 struct GnnGraph;
 void simulation_forget_gnn(Simulation *s, GnnNet *g);  // a network is being destroyed
 
+// Pinned host memory that a kernel writes and the host reads after it.
+template <typename T>
+struct PinnedPage {
+    T *host = nullptr, *device = nullptr;
+    PinnedPage() = default;
+    PinnedPage(const PinnedPage &) = delete;
+    PinnedPage &operator=(const PinnedPage &) = delete;
+    ~PinnedPage() {
+        if (host) (void)hipHostFree(host);
+    }
+    void ensure(size_t count) {
+        if (host) return;
+        void *h = nullptr, *dp = nullptr;
+        NSFEM_HIP(hipHostMalloc(&h, count * sizeof(T), hipHostMallocMapped));
+        host = static_cast<T *>(h);
+        NSFEM_HIP(hipHostGetDevicePointer(&dp, h, 0));
+        device = static_cast<T *>(dp);
+    }
+};
+
 struct Device {
     int index = 0;
     hipStream_t stream = nullptr;
@@ -232,6 +252,7 @@ struct Device {
     DeviceArray<unsigned char> sync_mem;  // persistent-kernel barrier state
     DeviceArray<CgColumnResult> cg_res;
     DeviceArray<double> dot_partial;
+    PinnedPage<double> dots;  // results of launch_dots
     DeviceArray<double> scalars;
     // this device's copy of the library's static scratch array (the
     // no-allocation solve), looked up once at device creation
@@ -288,6 +309,13 @@ void launch_combine(Device &d, int n, int l, const double *a, const double *X, s
                     bool accumulate, double *y, double *y2 = nullptr);
 void launch_dot_accumulate(Device &d, int n, const double *a, const double *b,
                            double *result);
+// X_i . y for i < l (X_i = X + i * stride) to entries at .. at + l - 1 of the
+// device's page of dots, which the host reads through wait_dots (one host
+// synchronisation): each has the bits of launch_dot_accumulate onto zero
+constexpr int kDotPage = 1024;
+void launch_dots(Device &d, int n, int l, const double *X, size_t stride, const double *y,
+                 int at = 0);
+const double *wait_dots(Device &d);
 
 struct CgRequest {
     Matrix *m;
@@ -346,27 +374,10 @@ struct PcgScalars {
 struct PcgReport {
     double rr, pq, rz;
 };
-struct PcgReportPage {
-    PcgReport *host = nullptr, *device = nullptr;
-    PcgReportPage() = default;
-    PcgReportPage(const PcgReportPage &) = delete;
-    PcgReportPage &operator=(const PcgReportPage &) = delete;
-    ~PcgReportPage() {
-        if (host) (void)hipHostFree(host);
-    }
-    void ensure() {
-        if (host) return;
-        void *h = nullptr, *dp = nullptr;
-        NSFEM_HIP(hipHostMalloc(&h, sizeof(PcgReport), hipHostMallocMapped));
-        host = static_cast<PcgReport *>(h);
-        NSFEM_HIP(hipHostGetDevicePointer(&dp, h, 0));
-        device = static_cast<PcgReport *>(dp);
-    }
-};
 struct PcgDevice {
     DeviceArray<double> partial;  // a product's per-tile sums, then their folds
     DeviceArray<PcgScalars> scalars;
-    PcgReportPage report;
+    PinnedPage<PcgReport> report;
     int count = 0;                 // partials of the last product or sweep
     const double *sums = nullptr;  // they, or their sum
     void release() {

@@ -39,7 +39,7 @@ void simulation_reset(Simulation &s);
 // correction); w, dx, guess: vectors of the matrix's size; s: dot results.
 struct ProjBasis {
     int n = 0, dim = 0, max = 0;
-    DeviceArray<double> x, ax, w, dx, guess, s;
+    DeviceArray<double> x, ax, w, dx, guess;
     void reserve(int rows, int depth) {
         n = rows;
         max = depth;
@@ -49,7 +49,6 @@ struct ProjBasis {
         w.resize(rows);
         dx.resize(rows);
         guess.resize(rows);
-        s.resize((size_t)depth + 1);
     }
     void release() {
         x.release();
@@ -57,7 +56,6 @@ struct ProjBasis {
         w.release();
         dx.release();
         guess.release();
-        s.release();
         n = dim = max = 0;
     }
 };
@@ -169,7 +167,7 @@ struct Simulation {
     // vectors r, z, p, q, a smoothing residual t and a dot scratch, and the
     // FP32 cycle's fine-level vectors
     bool pmg = false;
-    DeviceArray<double> pdinv, pr, pz, pp, pq, pt, pdot;
+    DeviceArray<double> pdinv, pr, pz, pp, pq, pt;
     DeviceArray<float> pdinv32, pb32, pz32, pt32, pp32;
     PcgDevice pcg, vcg;  // scalars of the pressure's and the diffusion's FP32-cycle CG
     // the FP32 cycles of the pressure and the diffusion solves (fixed
@@ -185,7 +183,7 @@ struct Simulation {
     // since each way last ran
     MgLevels vmg;
     int vmg_mode = 0;
-    DeviceArray<double> vdinv, vr, vz, vp, vq, vt, vdot;
+    DeviceArray<double> vdinv, vr, vz, vp, vq, vt;
     DeviceArray<float> vdinv32, vb32, vz32, vt32;  // the FP32 cycle's fine level
     DeviceArray<float> vp32;                       // the FP32 CG direction
     double vmg_sec[2][2] = {{0.0, 0.0}, {0.0, 0.0}};  // [column][plain, V-cycle]
@@ -545,20 +543,15 @@ void solve(Simulation &s, int slot, const double *b, double *x, int ncol, SolveO
 
 // out[i] = X_i . y for the first l basis vectors (one host synchronisation)
 void proj_dots(Device &d, ProjBasis &B, int l, const double *y, double *out) {
-    launch_fill(d, l, 0.0, B.s.ptr);
-    for (int i = 0; i < l; ++i)
-        launch_dot_accumulate(d, B.n, B.x.ptr + (size_t)i * B.n, y, B.s.ptr + i);
-    NSFEM_HIP(hipMemcpyAsync(out, B.s.ptr, sizeof(double) * l, hipMemcpyDeviceToHost, d.stream));
-    NSFEM_HIP(hipStreamSynchronize(d.stream));
+    launch_dots(d, B.n, l, B.x.ptr, (size_t)B.n, y);
+    const double *h = wait_dots(d);
+    std::copy(h, h + l, out);
 }
 
-double dev_dot(Device &d, ProjBasis &B, const double *a, const double *b) {
-    double h = 0.0;
-    launch_fill(d, 1, 0.0, B.s.ptr);
-    launch_dot_accumulate(d, B.n, a, b, B.s.ptr);
-    NSFEM_HIP(hipMemcpyAsync(&h, B.s.ptr, sizeof(double), hipMemcpyDeviceToHost, d.stream));
-    NSFEM_HIP(hipStreamSynchronize(d.stream));
-    return h;
+// a . b over n entries (one host synchronisation)
+double vec_dot(Device &d, int n, const double *a, const double *b) {
+    launch_dots(d, n, 1, a, 0, b);
+    return wait_dots(d)[0];
 }
 
 // Projection onto the span of past solutions (P. F. Fischer, "Projection
@@ -597,7 +590,7 @@ void projection_update(Device &d, ProjBasis &B, Matrix &A, const double *x) {
     else
         launch_axpby(d, n, 1.0, -1.0, x, B.guess.ptr, dx);
     launch_spmv(d, A, dx, nullptr, w, 0);
-    const double n0 = dev_dot(d, B, dx, w);
+    const double n0 = vec_dot(d, B.n, dx, w);
     if (!(n0 > 0.0)) return;
     std::vector<double> c(std::max(l, 1));
     double n1 = n0, before = n0;
@@ -606,7 +599,7 @@ void projection_update(Device &d, ProjBasis &B, Matrix &A, const double *x) {
         for (int i = 0; i < l; ++i) c[i] = -c[i];
         launch_combine(d, n, l, c.data(), B.x.ptr, (size_t)n, true, dx);
         launch_combine(d, n, l, c.data(), B.ax.ptr, (size_t)n, true, w);
-        n1 = dev_dot(d, B, dx, w);
+        n1 = vec_dot(d, B.n, dx, w);
         if (n1 > 0.5 * before) break;
         before = n1;
     }
@@ -729,7 +722,6 @@ void release_pressure_multigrid(Simulation &s) {
     s.pp.release();
     s.pq.release();
     s.pt.release();
-    s.pdot.release();
 }
 
 // 1/diag of a square host CSR, uploaded (a zero diagonal is rejected)
@@ -863,7 +855,7 @@ int mg_solve(Simulation &s, int64_t *cycles, double *seconds) {
     Device &d = *s.dev;
     MgLevel &C = coarse(s);
     const auto t0 = std::chrono::steady_clock::now();
-    const double bb = dev_dot(d, s.cproj, C.b.ptr, C.b.ptr);
+    const double bb = vec_dot(d, s.cproj.n, C.b.ptr, C.b.ptr);
     const double tol2 = s.coarse_rtol * s.coarse_rtol * bb;
     int status = NSFEM_MAX_ITERATIONS_REACHED;
     int k = 0;
@@ -874,7 +866,7 @@ int mg_solve(Simulation &s, int64_t *cycles, double *seconds) {
             vcycle(s, C.b.ptr, C.x.ptr);
             ++k;
             launch_spmv(d, C.A, C.x.ptr, C.b.ptr, C.r.ptr, 1);
-            const double rr = dev_dot(d, s.cproj, C.r.ptr, C.r.ptr);
+            const double rr = vec_dot(d, s.cproj.n, C.r.ptr, C.r.ptr);
             if (!std::isfinite(rr)) {
                 status = NSFEM_BREAKDOWN;
                 break;
@@ -1044,21 +1036,21 @@ void fine_vcycle32(Simulation &s) {
     s.pcg.count = A.n_tiles;  // a replay launches without the host's part
 }
 
-// a . b over n entries, through a one-entry device scratch (one host
-// synchronisation)
-double vec_dot(Device &d, int n, const double *a, const double *b, double *scratch) {
-    double h = 0.0;
-    launch_fill(d, 1, 0.0, scratch);
-    launch_dot_accumulate(d, n, a, b, scratch);
-    NSFEM_HIP(hipMemcpyAsync(&h, scratch, sizeof(double), hipMemcpyDeviceToHost, d.stream));
-    NSFEM_HIP(hipStreamSynchronize(d.stream));
-    return h;
+// b . b and, with r = b - A x left in `r`, r . r (one host synchronisation)
+void start_dots(Device &d, Matrix &A, int n, const double *b, const double *x, double *r,
+                double &bb, double &rr) {
+    launch_dots(d, n, 1, b, 0, b, 0);
+    launch_spmv(d, A, x, b, r, 1);
+    launch_dots(d, n, 1, r, 0, r, 1);
+    const double *h = wait_dots(d);
+    bb = h[0];
+    rr = h[1];
 }
 
 // Vectors of a preconditioned CG over n rows: residual, preconditioned
-// residual, direction, product, and a one-entry dot scratch.
+// residual, direction and product.
 struct PcgWork {
-    double *r, *z, *p, *q, *dot;
+    double *r, *z, *p, *q;
 };
 
 // CG preconditioned by z = precond(r) (symmetric positive definite), in
@@ -1070,9 +1062,8 @@ int pcg_run(Device &d, Matrix &A, int n, const double *b, double *x, const PcgWo
             double rtol, int64_t max_iterations, Pre precond, SolveOut &o, int c) {
     const auto t0 = std::chrono::steady_clock::now();
     double *r = w.r, *z = w.z, *p = w.p, *q = w.q;
-    const double bb = vec_dot(d, n, b, b, w.dot);
-    launch_spmv(d, A, x, b, r, 1);
-    double rr = vec_dot(d, n, r, r, w.dot);
+    double bb, rr;
+    start_dots(d, A, n, b, x, r, bb, rr);
     const double ref = bb > 0.0 ? bb : rr;
     const double tol2 = rtol * rtol * ref;
     const int64_t max_iter = max_iterations > 0 ? max_iterations : n;
@@ -1082,10 +1073,10 @@ int pcg_run(Device &d, Matrix &A, int n, const double *b, double *x, const PcgWo
         status = NSFEM_MAX_ITERATIONS_REACHED;
         precond(r, z);
         launch_copy(d, n, z, p);
-        double rz = vec_dot(d, n, r, z, w.dot);
+        double rz = vec_dot(d, n, r, z);
         while (k < max_iter) {
             launch_spmv(d, A, p, nullptr, q, 0);
-            const double pq = vec_dot(d, n, p, q, w.dot);
+            const double pq = vec_dot(d, n, p, q);
             if (!(pq > 0.0) || !(rz > 0.0)) {
                 status = NSFEM_BREAKDOWN;
                 break;
@@ -1094,17 +1085,17 @@ int pcg_run(Device &d, Matrix &A, int n, const double *b, double *x, const PcgWo
             launch_axpy(d, n, alpha, p, x);
             launch_axpy(d, n, -alpha, q, r);
             ++k;
-            rr = vec_dot(d, n, r, r, w.dot);
+            rr = vec_dot(d, n, r, r);
             if (rr <= tol2) {
                 launch_spmv(d, A, x, b, r, 1);
-                rr = vec_dot(d, n, r, r, w.dot);
+                rr = vec_dot(d, n, r, r);
                 if (rr <= tol2) {
                     status = NSFEM_OK;
                     break;
                 }
             }
             precond(r, z);
-            const double rz_new = vec_dot(d, n, r, z, w.dot);
+            const double rz_new = vec_dot(d, n, r, z);
             const double beta = rz_new / rz;
             rz = rz_new;
             launch_axpby(d, n, 1.0, beta, z, p, p);
@@ -1159,9 +1150,8 @@ int pcg_run32(Device &d, Matrix &A, int n, const double *b, double *x, const Pcg
               int c) {
     const auto t0 = std::chrono::steady_clock::now();
     double *r = w.r, *q = w.q;
-    const double bb = vec_dot(d, n, b, b, w.dot);
-    launch_spmv(d, A, x, b, r, 1);
-    double rr = vec_dot(d, n, r, r, w.dot);
+    double bb, rr;
+    start_dots(d, A, n, b, x, r, bb, rr);
     const double ref = bb > 0.0 ? bb : rr;
     const double tol2 = rtol * rtol * ref;
     const int64_t max_iter = max_iterations > 0 ? max_iterations : n;
@@ -1187,7 +1177,7 @@ int pcg_run32(Device &d, Matrix &A, int n, const double *b, double *x, const Pcg
             const bool met = rr <= tol2;
             if (met || rr * kPcgUpdateDrop * kPcgUpdateDrop <= rr_true) {
                 launch_spmv(d, A, x, b, r, 1);
-                rr = vec_dot(d, n, r, r, w.dot);
+                rr = vec_dot(d, n, r, r);
                 rr_true = rr;
                 if (rr <= tol2) {
                     status = NSFEM_OK;
@@ -1218,7 +1208,7 @@ int pcg_run32(Device &d, Matrix &A, int n, const double *b, double *x, const Pcg
 void pcg_pressure(Simulation &s, SolveOut &o) {
     Device &d = *s.dev;
     launch_scatter(d, s.npb, s.pb_idx.ptr, s.pb_val.ptr, s.p.ptr);
-    const PcgWork w{s.pr.ptr, s.pz.ptr, s.pp.ptr, s.pq.ptr, s.pdot.ptr};
+    const PcgWork w{s.pr.ptr, s.pz.ptr, s.pp.ptr, s.pq.ptr};
     Matrix &A = s.mats[NSFEM_PRESSURE_STIFFNESS];
     int status = NSFEM_OK;
     SolveOut first{};
@@ -1309,7 +1299,7 @@ void pcg_velocity(Simulation &s, int c, SolveOut &o) {
     const size_t off = (size_t)c * s.V;
     double *x = s.uv.ptr + off;
     launch_scatter(d, s.nvb, s.vb_idx.ptr, c ? s.vb_v.ptr : s.vb_u.ptr, x);
-    const PcgWork w{s.vr.ptr, s.vz.ptr, s.vp.ptr, s.vq.ptr, s.vdot.ptr};
+    const PcgWork w{s.vr.ptr, s.vz.ptr, s.vp.ptr, s.vq.ptr};
     Matrix &A = s.mats[NSFEM_DIFFUSION];
     int status = NSFEM_OK;
     SolveOut first{};
@@ -1533,7 +1523,6 @@ void simulation_set_pressure_multigrid(Simulation &s, int enable) {
     s.pp.resize(s.P);
     s.pq.resize(s.P);
     s.pt.resize(s.P);
-    s.pdot.resize(1);
     s.pmg = true;
 }
 
@@ -1544,7 +1533,7 @@ void release_velocity_multigrid(Simulation &s) {
     drop_graph(s.vcycle_graph);
     s.vmg.release();
     s.vmg_mode = 0;
-    for (DeviceArray<double> *a : {&s.vdinv, &s.vr, &s.vz, &s.vp, &s.vq, &s.vt, &s.vdot})
+    for (DeviceArray<double> *a : {&s.vdinv, &s.vr, &s.vz, &s.vp, &s.vq, &s.vt})
         a->release();
     for (DeviceArray<float> *a : {&s.vdinv32, &s.vb32, &s.vz32, &s.vt32, &s.vp32}) a->release();
     s.vcg.release();
@@ -1589,7 +1578,6 @@ void build_velocity_coarse_space(Simulation &s, int nc, int64_t nnz, const int32
     append_level(d, s.vmg, V, A.host_rs, acol, aval, nc, nnz, prs.data(), pcol.data(),
                  pval.data(), host_threads(s));
     for (DeviceArray<double> *a : {&s.vr, &s.vz, &s.vp, &s.vq, &s.vt}) a->resize((size_t)V);
-    s.vdot.resize(1);
     s.vmg_mode = 1;
 }
 }  // namespace

@@ -49,3 +49,36 @@ def test_chain_step_against_oracle(gpu, oracle, n, min_size, precision):
         assert np.abs(a - b).max() < 1e-6 * scale
     assert st["vcycle_solves"][:3] == [2, 2, 2]
     assert max(st["vcycle_iterations"][:3]) <= 2 * 20
+
+
+# a basis of one vector (the plain dot), of the most that one launch of dots
+# takes (8), one more, and two launches and one more; 961 velocity nodes end
+# inside the first block's chunk of 1,024, 1,089 in the second's
+@pytest.mark.parametrize("depth", [1, 8, 9, 17])
+@pytest.mark.parametrize("n", [15, 16])
+def test_projection_basis_at_its_edges(gpu, n, depth):
+    """The projection changes only where a solve starts: past a restart of
+    the basis the fields are those of the run without it to what solves to
+    1e-11 leave (cond * 1e-11 of a cavity this small is far below 1e-6), and
+    the diffusion solves take fewer iterations (a basis whose coefficients
+    were wrong in any vector would start them further away)."""
+    from navier_stokes_fem_amd import mesh
+    from navier_stokes_fem_amd.simulation import Simulation
+
+    m = mesh.cavity(n)
+    out = []
+    for d in (0, depth):
+        s = Simulation(m, 1e-3, 1e-3, device=gpu, rtol=1e-11, precision="fp64")
+        s.set_velocity_projection(d)
+        s.set_mass_projection(d)
+        st = s.step(depth + 4)
+        out.append((st, s.fields()))
+        s.close()
+    (s0, f0), (s1, f1) = out
+    assert max(s1["max_relative_residual"]) <= 1e-11 * (1 + 1e-6)
+    scale = max(np.abs(f).max() for f in f0)
+    for a, b in zip(f1, f0):
+        assert np.abs(a - b).max() < 1e-6 * scale
+    d0, d1 = (sum(s["cg_iterations"][:2]) for s in (s0, s1))
+    print(f"diffusion iterations {d0} -> {d1}")
+    assert d1 < d0
