@@ -112,6 +112,43 @@ def test_gradient_sums_at_their_edges(gpu, n):
     pg.close()
 
 
+@pytest.mark.parametrize("n", [1, 15, 130])
+def test_a_step_leaves_the_operands_of_its_weights(gpu, n):
+    """After an Adam step the BF16 operands are those of the new weights: the
+    prediction and the gradients have the bits of another network that is
+    given the same weights (and of a prediction that keeps nothing for a
+    backward pass, before and after one that does)."""
+    from navier_stokes_fem_amd import learned as L, mesh
+    from navier_stokes_fem_amd.device import DeviceBuffer
+    from oracle import gnn
+
+    og, pg, b, p, bb, pb = _setup(gpu, mesh.cavity(n), seed=n)
+    params = gnn.init_params(9)
+    rng = np.random.default_rng(10)
+    for k in params:
+        params[k] = (params[k] + 0.05 * rng.standard_normal(params[k].shape)).astype(np.float32)
+    nets = [L.WarmStartNet(gpu, seed=k) for k in (1, 2)]
+    nets[0].set_params(L.WarmStartNet.flatten(params))
+    nets[0].train_step(pg, bb, pb, 1e-2)
+    nets[1].set_params(nets[0].get_params())
+    out = DeviceBuffer(gpu, 8 * og.n)
+    got = []
+    for net in nets:
+        net.predict(pg, bb, out)
+        first = out.download()
+        loss, flat = net.gradients(pg, bb, pb)
+        net.predict(pg, bb, out)
+        np.testing.assert_array_equal(out.download(), first)
+        got.append((first, flat, loss))
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    assert got[0][2] == got[1][2]
+    out.close()
+    for net in nets:
+        net.close()
+    pg.close()
+
+
 def test_adam_step_clips_outlier_gradients(gpu):
     """Two Adam steps against the update restated on the host: an ordinary
     pair (its norm starts the running average, no clipping), then the same
