@@ -747,9 +747,13 @@ __global__ __launch_bounds__(kBlock) void k_dots_final(int nb, const double *__r
     if (threadIdx.x == 0) out[blockIdx.x] = 0.0 + s[0];
 }
 
-// The sum of n partials, the same bits in every thread of every block.
+// The sum of n partials, the same bits in every thread of every block.  One
+// partial (folded before) is read as it is: with a block sum's two barriers
+// in front of each block's work k_pcg_direction took 71 us on the 16.8 M
+// velocity nodes of the 2048^2 cavity, without 51.
 __device__ __forceinline__ double sum_partials(int n, const double *__restrict__ part,
                                                double *lds) {
+    if (n == 1) return 0.0 + part[0];
     double s[1] = {0.0};
 #pragma unroll 4
     for (int i = threadIdx.x; i < n; i += kBlock) s[0] += part[i];
