@@ -408,7 +408,7 @@ namespace {
 // MODE 0: y = A x.  MODE 1: y = lhs - A x (y may alias lhs).
 // MODE 2: y = A x - lhs.  MODE 3: y = x + omega dinv (lhs - A x), a damped
 // Jacobi sweep into another vector (y aliases neither x nor lhs; the same
-// roundings as the residual product followed by k_jacobi).
+// roundings as the residual product followed by a Jacobi update).
 // MODE 4: y += A x (the roundings of the product followed by k_add).
 // MODE 5: y = A x and y2 = omega dinv y, the Jacobi sweep from zero that
 // follows a restriction (k_jacobi0's roundings).
