@@ -3318,7 +3318,9 @@ __global__ __launch_bounds__(BS, BS / 256) void k_cg_p2(const CgArgs A) {
 // the vertices-first node order of larger meshes) keep the streaming forms.
 
 constexpr int kResWaves = 12;  // 3 waves a SIMD: 168 VGPRs each
-constexpr int kResBlock = 64 * kResWaves;
+// Waves of a block of the refined one-column batch: those of the streaming
+// batch's blocks, whose sums it repeats (4 waves a SIMD: 128 VGPRs each).
+constexpr int kResWavesBatch = 16;
 
 template <typename T>
 __device__ __forceinline__ T ld_agent(const T *p) {
@@ -3389,8 +3391,9 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
     return v;
 }
 
+template <int NW>
 struct ResShared {
-    double part[2][kMaxRed][kResWaves];  // by epoch parity
+    double part[2][kMaxRed][NW];  // by epoch parity
     double sum[kMaxRed];
     int fail;
 };
@@ -3407,11 +3410,11 @@ struct ResShared {
 // which each does after it has read all of e.  Sums are added as in
 // grid_sum_flat.  The waits on vmcnt before the first barrier are what makes
 // the block's stores visible before its post.
-template <int K>
-__device__ __forceinline__ bool res_exchange(SyncState *G, ResShared &S, double (&v)[K],
+template <int K, int NW>
+__device__ __forceinline__ bool res_exchange(SyncState *G, ResShared<NW> &S, double (&v)[K],
                                              unsigned &epoch, const unsigned long long timeout,
                                              const int b, const int nb) {
-    static_assert(K <= kMaxRed && K <= kResWaves, "reduction width");
+    static_assert(K <= kMaxRed && K <= NW, "reduction width");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned e = ++epoch;
@@ -3426,7 +3429,7 @@ __device__ __forceinline__ bool res_exchange(SyncState *G, ResShared &S, double 
     if (wave < K) {
         double s = 0.0;
 #pragma unroll
-        for (int i = 0; i < kResWaves; ++i) s += S.part[par][wave][i];
+        for (int i = 0; i < NW; ++i) s += S.part[par][wave][i];
         if (nb == 1) {
             if (lane == 0) S.sum[wave] = s;
         } else {
@@ -3466,12 +3469,12 @@ __device__ __forceinline__ bool res_exchange(SyncState *G, ResShared &S, double 
 // products before they are added, in column order).  SHARED: x as other
 // blocks published it.  The loop over the wave's tiles stays rolled, so that
 // its loads take no registers from the resident matrix more than once.
-template <int NC, typename VT, bool SHARED>
+template <int NC, typename VT, bool SHARED, int NW>
 __device__ __forceinline__ void res_residual(const CgArgs &A, const int T0, const int T1,
                                              const int wave, const int lane, VT *rbuf,
                                              double (&acc)[3 * NC]) {
 #pragma unroll 1
-    for (int t = T0 + wave; t < T1; t += kResWaves) {
+    for (int t = T0 + wave; t < T1; t += NW) {
         const int4 m = A.meta[t];
         const int row = m.x + lane;
         if (row >= m.y) continue;
@@ -3519,15 +3522,16 @@ __device__ __forceinline__ void res_residual(const CgArgs &A, const int T0, cons
 // One block's part of a resident solve of `nb` blocks (`b`: its reduction
 // slot, `L`: its index among the tiles' owners, as cg_body).  W: the most
 // nonzeros of a row; R: the most wave tiles of a wave (the host checks both,
-// and that the window fits win_cap).  smem: win_cap + 1 rows of p, then r of
+// and that the window fits win_cap); NW: the block's waves.  smem: win_cap + 1 rows of p, then r of
 // the window's rows that other blocks own.
-template <int NC, bool MIXED, int W, int R>
+template <int NC, bool MIXED, int W, int R, int NW>
 __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const int nb,
                                             const int L, unsigned char *smem) {
     using VT = typename std::conditional<MIXED, float, double>::type;
     using Row = VecN<NC, VT>;
     __shared__ CgCtl<NC> C;
-    __shared__ ResShared S;
+    __shared__ ResShared<NW> S;
+    constexpr int BS = 64 * NW;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int T0 = A.block_tiles[L], T1 = A.block_tiles[L + 1];
@@ -3551,13 +3555,13 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
         Row zero;
 #pragma unroll
         for (int c = 0; c < NC; ++c) zero.v[c] = (VT)0;
-        for (int i = tid; i <= wn; i += kResBlock) pw[i] = zero;
-        for (int i = tid; i < nh; i += kResBlock) rh[i] = zero;
+        for (int i = tid; i <= wn; i += BS) pw[i] = zero;
+        for (int i = tid; i < nh; i += BS) rh[i] = zero;
         double acc[3 * NC];
 #pragma unroll
         for (int k = 0; k < 3 * NC; ++k) acc[k] = 0.0;
-        res_residual<NC, VT, false>(A, T0, T1, wave, lane, rbuf, acc);
-        if (!res_exchange<3 * NC>(A.sync, S, acc, epoch, A.timeout_ticks, b, nb)) goto timeout;
+        res_residual<NC, VT, false, NW>(A, T0, T1, wave, lane, rbuf, acc);
+        if (!res_exchange<3 * NC, NW>(A.sync, S, acc, epoch, A.timeout_ticks, b, nb)) goto timeout;
         if (t0) {
             double sums[3 * NC];
 #pragma unroll
@@ -3573,7 +3577,7 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             for (int w = 0; w < W; ++w) val[j][w] = (VT)0;
 #pragma unroll
             for (int w = 0; w < (W + 1) / 2; ++w) idx[j][w] = (unsigned)wn * 0x10001u;
-            const int t = T0 + wave + kResWaves * j;
+            const int t = T0 + wave + NW * j;
             if (t >= T1) continue;  // wave-uniform
             const int4 m = A.meta[t];
             const bool has = m.x + lane < m.y;
@@ -3619,16 +3623,16 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             // the window's rows of other blocks: kAhead loads in flight
             constexpr int kAhead = 4;
             const VT *src = fresh ? rbuf : qbuf[par ^ 1];
-            for (int base = tid; base < nh; base += kAhead * kResBlock) {
+            for (int base = tid; base < nh; base += kAhead * BS) {
                 Row in[kAhead];
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u) {
-                    const int i = min(base + u * kResBlock, nh - 1);
+                    const int i = min(base + u * BS, nh - 1);
                     in[u] = ldv_agent<NC, VT>(src, i < nl ? win0 + i : R1 + (i - nl));
                 }
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u) {
-                    const int i = base + u * kResBlock;
+                    const int i = base + u * BS;
                     if (i >= nh) break;
                     const int slot = i < nl ? i : i + (R1 - R0);
                     Row rn, pn = pw[slot];
@@ -3666,7 +3670,7 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             for (int k = 0; k < 4 * NC; ++k) sums[k] = 0.0;
 #pragma unroll
             for (int j = 0; j < R; ++j) {
-                if (T0 + wave + kResWaves * j >= T1) continue;  // wave-uniform
+                if (T0 + wave + NW * j >= T1) continue;  // wave-uniform
                 double s[NC];
 #pragma unroll
                 for (int c = 0; c < NC; ++c) s[c] = 0.0;
@@ -3699,7 +3703,7 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
                 }
                 stv_agent<NC, VT>(qbuf[par], row[j], q[j]);
             }
-            if (!res_exchange<4 * NC>(A.sync, S, sums, epoch, A.timeout_ticks, b, nb)) goto timeout;
+            if (!res_exchange<4 * NC, NW>(A.sync, S, sums, epoch, A.timeout_ticks, b, nb)) goto timeout;
             if (t0) {
 #pragma unroll
                 for (int k = 0; k < 4 * NC; ++k) sums[k] = S.sum[k];
@@ -3724,13 +3728,13 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
                         }
                     }
                     double none[1] = {0.0};
-                    if (!res_exchange<1>(A.sync, S, none, epoch, A.timeout_ticks, b, nb))
+                    if (!res_exchange<1, NW>(A.sync, S, none, epoch, A.timeout_ticks, b, nb))
                         goto timeout;
                     double ra[3 * NC];
 #pragma unroll
                     for (int k = 0; k < 3 * NC; ++k) ra[k] = 0.0;
-                    res_residual<NC, VT, true>(A, T0, T1, wave, lane, rbuf, ra);
-                    if (!res_exchange<3 * NC>(A.sync, S, ra, epoch, A.timeout_ticks, b, nb))
+                    res_residual<NC, VT, true, NW>(A, T0, T1, wave, lane, rbuf, ra);
+                    if (!res_exchange<3 * NC, NW>(A.sync, S, ra, epoch, A.timeout_ticks, b, nb))
                         goto timeout;
                     if (t0) {
 #pragma unroll
@@ -3776,23 +3780,23 @@ timeout:
     }
 }
 
-template <int NC, bool MIXED, int W, int R>
-__global__ __launch_bounds__(kResBlock, kResBlock / 256) void k_cg_res(const CgArgs A) {
+template <int NC, bool MIXED, int W, int R, int NW>
+__global__ __launch_bounds__(64 * NW, NW / 4) void k_cg_res(const CgArgs A) {
     extern __shared__ __align__(16) unsigned char smem[];
-    cg_resident<NC, MIXED, W, R>(A, blockIdx.x, gridDim.x, xcd_swizzle(blockIdx.x, gridDim.x),
-                                 smem);
+    cg_resident<NC, MIXED, W, R, NW>(A, blockIdx.x, gridDim.x,
+                                     xcd_swizzle(blockIdx.x, gridDim.x), smem);
 }
 
 // Many resident solves in one launch (block map as k_cg_batch).
-template <int NC, bool MIXED, int W, int R>
-__global__ __launch_bounds__(kResBlock, kResBlock / 256) void k_cg_res_batch(
+template <int NC, bool MIXED, int W, int R, int NW>
+__global__ __launch_bounds__(64 * NW, NW / 4) void k_cg_res_batch(
     const CgArgs *__restrict__ args, const int2 *__restrict__ map) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int2 m = map[blockIdx.x];
     const int inst = __builtin_amdgcn_readfirstlane(m.x);
     const int lb = __builtin_amdgcn_readfirstlane(m.y);
     const CgArgs A = args[inst];
-    cg_resident<NC, MIXED, W, R>(A, lb, A.nblocks, lb, smem);
+    cg_resident<NC, MIXED, W, R, NW>(A, lb, A.nblocks, lb, smem);
 }
 
 // Many independent systems in one persistent launch: block i works for
@@ -3990,64 +3994,53 @@ constexpr int res_tiles(bool mixed, int w) { return w == kResRowShort ? 4 : mixe
 // Most LDS of a resident block (160 KB a CU; one block a CU).
 constexpr size_t kResLds = 120 * 1024;
 
-// Calls f.template run<NC, MIXED, W, R>() for a resident solve whose waves own
-// `tiles` wave tiles at most.
-template <int NC, bool MIXED, int W, typename F>
-void res_dispatch_tiles(int tiles, F &f) {
-    constexpr int most = res_tiles(MIXED, W);
-    if (tiles <= 1) f.template run<NC, MIXED, W, 1>();
-    else if (tiles == 2) f.template run<NC, MIXED, W, 2>();
-    else f.template run<NC, MIXED, W, most>();
-}
-template <typename F>
-void res_dispatch(int nc, bool mixed, int w, int tiles, F &&f) {
-    constexpr int S = kResRowShort, L = kResRowLong;
-    if (nc == 1 && mixed) {
-        if (w == S) res_dispatch_tiles<1, true, S>(tiles, f);
-        else res_dispatch_tiles<1, true, L>(tiles, f);
-    } else if (nc == 1) {
-        if (w == S) res_dispatch_tiles<1, false, S>(tiles, f);
-        else res_dispatch_tiles<1, false, L>(tiles, f);
-    } else if (mixed) {
-        res_dispatch_tiles<2, true, L>(tiles, f);
-    } else {
-        res_dispatch_tiles<2, false, L>(tiles, f);
+// The kernel of a resident solve whose waves own `tiles` wave tiles at most;
+// batch: of many solves, with `waves` waves a block (a refined batch: short
+// rows and one column only, in kResWaves or kResWavesBatch waves).
+template <int NC, bool MIXED, int W, int R>
+const void *res_kernel(bool batch, int waves) {
+    if (!batch) return (const void *)k_cg_res<NC, MIXED, W, R, kResWaves>;
+    if constexpr (MIXED && W == kResRowShort) {
+        if (waves == kResWavesBatch)
+            return (const void *)k_cg_res_batch<NC, MIXED, W, R, kResWavesBatch>;
     }
+    NSFEM_REQUIRE(waves == kResWaves, NSFEM_ERROR, "waves of a resident batch");
+    if constexpr (!MIXED || W == kResRowShort)
+        return (const void *)k_cg_res_batch<NC, MIXED, W, R, kResWaves>;
+    fail(NSFEM_ERROR, "this refined batch streams");
+}
+template <int NC, bool MIXED, int W>
+const void *res_kernel_tiles(bool batch, int waves, int tiles) {
+    if (tiles <= 1) return res_kernel<NC, MIXED, W, 1>(batch, waves);
+    if (tiles == 2) return res_kernel<NC, MIXED, W, 2>(batch, waves);
+    if constexpr (MIXED && W == kResRowShort) {
+        // 128 registers hold three tiles, not four (58 spilled): what two
+        // tiles a wave come to where the blocks do not divide them evenly
+        if (waves == kResWavesBatch && tiles == 3)
+            return (const void *)k_cg_res_batch<NC, MIXED, W, 3, kResWavesBatch>;
+    }
+    return res_kernel<NC, MIXED, W, res_tiles(MIXED, W)>(batch, waves);
+}
+const void *res_kernel(int nc, bool mixed, int w, int tiles, bool batch, int waves = kResWaves) {
+    constexpr int S = kResRowShort, L = kResRowLong;
+    if (nc == 2)
+        return mixed ? res_kernel_tiles<2, true, L>(batch, waves, tiles)
+                     : res_kernel_tiles<2, false, L>(batch, waves, tiles);
+    if (w == S)
+        return mixed ? res_kernel_tiles<1, true, S>(batch, waves, tiles)
+                     : res_kernel_tiles<1, false, S>(batch, waves, tiles);
+    return mixed ? res_kernel_tiles<1, true, L>(batch, waves, tiles)
+                 : res_kernel_tiles<1, false, L>(batch, waves, tiles);
 }
 
-template <int NC, bool MIXED, int W, int R>
-const void *res_kernel(bool batch) {
-    return batch ? (const void *)k_cg_res_batch<NC, MIXED, W, R>
-                 : (const void *)k_cg_res<NC, MIXED, W, R>;
-}
 // Allows a kernel its dynamic LDS and returns the blocks a device holds.
-struct ResMaxGrid {
-    Device &d;
-    size_t lds;
-    bool batch;
-    int out;
-    template <int NC, bool MX, int W, int R>
-    void run() {
-        const void *k = res_kernel<NC, MX, W, R>(batch);
-        if (lds > 48 * 1024)
-            NSFEM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        int per_cu = 0;
-        NSFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, kResBlock, lds));
-        out = std::min(per_cu * d.cu_count, kResMaxBlocks);
-    }
-};
-struct ResLaunch {
-    Device &d;
-    void **kargs;
-    int grid;
-    size_t lds;
-    bool batch;
-    template <int NC, bool MX, int W, int R>
-    void run() {
-        NSFEM_HIP(hipLaunchCooperativeKernel(res_kernel<NC, MX, W, R>(batch), dim3(grid),
-                                             dim3(kResBlock), kargs, (unsigned)lds, d.stream));
-    }
-};
+int res_max_grid(Device &d, const void *kernel, int waves, size_t lds) {
+    if (lds > 48 * 1024)
+        NSFEM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int per_cu = 0;
+    NSFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, lds));
+    return std::min(per_cu * d.cu_count, kResMaxBlocks);
+}
 
 // Window rows and LDS of a matrix split over `grid` blocks; false when a
 // block's tiles, window or LDS go past what the kernel holds.
@@ -4058,13 +4051,13 @@ struct ResLaunch {
 // columns: FP64 19.1 us on 63 blocks, 13.9 on 128; refined 38.9 and 25.3).
 int cg_tiles_per_wave(const Matrix &m) { return m.max_row_nz > kResRowShort ? 1 : 2; }
 
-bool res_fits(const Matrix &m, int nc, bool mixed, int w, int grid, ResidentPlan &plan) {
+bool res_fits(const Matrix &m, int nc, bool mixed, int w, int waves, int grid, ResidentPlan &plan) {
     std::vector<int32_t> bt;
     split_tiles(m, grid, bt);
     int64_t cap = 0, halo = 0;
     int tiles = 0;
     for (int b = 0; b < grid; ++b) {
-        tiles = std::max(tiles, (bt[b + 1] - bt[b] + kResWaves - 1) / kResWaves);
+        tiles = std::max(tiles, (bt[b + 1] - bt[b] + waves - 1) / waves);
         if (bt[b + 1] <= bt[b] || tiles > res_tiles(mixed, w)) return false;
         const int64_t r0 = m.host_wtiles[bt[b]], r1 = m.host_wtiles[bt[b + 1]];
         const int64_t w0 = std::max<int64_t>(0, r0 - m.band_lo);
@@ -4095,14 +4088,14 @@ ResidentPlan plan_resident(const Matrix &m, int nc, bool mixed, int want, int ma
     const int most = std::min(std::min(max_blocks, kResMaxBlocks), m.n_wtiles);
     if (most < 1) return plan;
     if (want > 0) {
-        res_fits(m, nc, mixed, w, std::min(want, most), plan);
+        res_fits(m, nc, mixed, w, kResWaves, std::min(want, most), plan);
         return plan;
     }
     int grid = std::max(1, std::min(m.n_wtiles / (cg_tiles_per_wave(m) * kResWaves), most));
     const int room = kResWaves * res_tiles(mixed, w);
     if ((int64_t)room * most < m.n_wtiles) return plan;
     for (int tries = 0; tries < 8 && grid <= most; ++tries) {
-        if (res_fits(m, nc, mixed, w, grid, plan)) return plan;
+        if (res_fits(m, nc, mixed, w, kResWaves, grid, plan)) return plan;
         grid = std::max(grid + 1, std::max((m.n_wtiles + room - 1) / room, grid + grid / 8));
     }
     return plan;
@@ -4308,10 +4301,10 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
     if (want_resident(nc, mixed))
         res = want > 0 ? plan_resident(m, nc, mixed, want, d.cu_count)
                        : resident_plan(d, m, nc, mixed);
+    const void *res_fn = nullptr;
     if (res.ok) {
-        ResMaxGrid rg{d, res.lds, false, 0};
-        res_dispatch(nc, mixed, res.width, res.tiles, rg);
-        res.ok = rg.out >= res.grid;
+        res_fn = res_kernel(nc, mixed, res.width, res.tiles, false);
+        res.ok = res_max_grid(d, res_fn, kResWaves, res.lds) >= res.grid;
         if (res.ok) grid = res.grid;
     }
     const bool verbose = std::getenv("NSFEM_CG_VERBOSE") != nullptr;
@@ -4356,15 +4349,15 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
                          "[nsfem] cg launch matrix=%p rows=%d cols=%d wave tiles=%d grid=%d "
                          "maxgrid=%d mixed=%d idx16=%d form=%d block=%d resident=%d attempt=%d\n",
                          (const void *)&m, n, nc, m.n_wtiles, grid, maxg, (int)mixed, (int)idx16,
-                         wi, res.ok ? kResBlock : bs, res.ok ? res.width : 0, attempt);
+                         wi, res.ok ? 64 * kResWaves : bs, res.ok ? res.width : 0, attempt);
         NSFEM_HIP(hipEventRecord(d.ev_start, d.stream));
         k_sync_reset<<<(ngroups + 255) / 256, 256, 0, d.stream>>>(a.sync, ngroups,
                                                                   res.ok ? grid : 0);
         NSFEM_HIP(hipGetLastError());
         if (res.ok) {
             void *kargs[] = {(void *)&a};
-            res_dispatch(nc, mixed, res.width, res.tiles,
-                         ResLaunch{d, kargs, grid, res.lds, false});
+            NSFEM_HIP(hipLaunchCooperativeKernel(res_fn, dim3(grid), dim3(64 * kResWaves), kargs,
+                                                 (unsigned)res.lds, d.stream));
         } else {
             CgLaunch ln{d, a, grid, bs, p2, ib};
             cg_dispatch(nc, mixed, idx16, wi, ln);
@@ -4586,31 +4579,29 @@ struct BatchLaunch {
     std::vector<int> blocks;
     std::vector<int> cap;
     bool resident = false;
-    int width = 0, tiles = 0;
+    int width = 0, tiles = 0, waves = 0;
     size_t lds = 0;
 };
 
 // The launches of a batch in the resident form, or none when a system does
-// not allow it.  Systems go largest first, so that those of like iteration
-// counts share a launch, each with the fewest blocks it fits in; a launch's
-// other blocks go where share_blocks sends them, up to a single solve's.
+// not allow it (refined: two columns and long rows never do).  Systems go
+// largest first, so that those of like iteration counts share a launch, each
+// with the fewest blocks it fits in; a launch's other blocks go where
+// share_blocks sends them, up to a single solve's.
 std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgRequest> &reqs, int nc,
                                            bool mixed, int scale) {
     std::vector<BatchLaunch> out;
-    if (!want_resident(nc, mixed)) return out;
+    if (!want_resident(nc, mixed) || (mixed && nc == 2)) return out;
     int w = nc == 1 ? kResRowShort : kResRowLong;
     for (const CgRequest &r : reqs) {
         const Matrix &m = *r.m;
         if (m.nnz <= 0 || m.max_row_nz > kResRowLong || m.n_wtiles < 1) return out;
         if (m.max_row_nz > kResRowShort) w = kResRowLong;
     }
+    if (mixed && w == kResRowLong) return out;
     const int room = kResWaves * res_tiles(mixed, w);
-    int maxg = 0;
-    {
-        ResMaxGrid mg{d, kResLds, true, 0};
-        res_dispatch(nc, mixed, w, res_tiles(mixed, w), mg);
-        maxg = mg.out;
-    }
+    const int maxg = res_max_grid(d, res_kernel(nc, mixed, w, res_tiles(mixed, w), true), kResWaves,
+                                  kResLds);
     std::vector<size_t> order(reqs.size());
     for (size_t i = 0; i < order.size(); ++i) order[i] = i;
     std::sort(order.begin(), order.end(), [&](size_t a, size_t b) {
@@ -4624,7 +4615,7 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
         const Matrix &m = *reqs[i].m;
         ResidentPlan plan;
         int g = (m.n_wtiles + room - 1) / room;
-        while (g <= std::min(maxg, m.n_wtiles) && !res_fits(m, nc, mixed, w, g, plan)) ++g;
+        while (g <= std::min(maxg, m.n_wtiles) && !res_fits(m, nc, mixed, w, kResWaves, g, plan)) ++g;
         if (!plan.ok) return std::vector<BatchLaunch>();
         least[i] = g;
         if (used + g > maxg) {
@@ -4648,11 +4639,12 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
         l.blocks = share_blocks(rq, maxg, want, nb);
         l.resident = true;
         l.width = w;
+        l.waves = kResWaves;
         for (size_t k = 0; k < rq.size(); ++k) {
             ResidentPlan plan;
-            if (!res_fits(*rq[k]->m, nc, mixed, w, l.blocks[k], plan)) {
+            if (!res_fits(*rq[k]->m, nc, mixed, w, kResWaves, l.blocks[k], plan)) {
                 l.blocks[k] = nb[k];
-                res_fits(*rq[k]->m, nc, mixed, w, nb[k], plan);
+                res_fits(*rq[k]->m, nc, mixed, w, kResWaves, nb[k], plan);
             }
             l.cap.push_back(plan.cap);
             l.tiles = std::max(l.tiles, plan.tiles);
@@ -4660,6 +4652,46 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
         }
     }
     return out;
+}
+
+// Puts a launch of refined one-column solves, split as the streaming form
+// splits it, on the resident form where every system allows it: rows of at
+// most kResRowShort nonzeros, windows that fit, and at most kFlatMax blocks
+// each (past them the streaming form adds its sums as a tree).  Same blocks,
+// same waves, same sums: the iterates are the streaming form's, bit for bit.
+// Returns whether it did.  (Two refined columns stream: their two-phase
+// iteration has no resident counterpart, and another iteration ends some
+// systems a step earlier or later.)  Two steps of 16 refined cavities of 16^2
+// to 128^2: 55.5 ms streaming, 24.1 with the pressure solves resident; with
+// the velocity's resident too, in the single-reduction iteration, 20.4, but
+// the fields moved by up to 6e-4 (inside what solves to 1e-8 leave).
+bool batch_resident(Device &d, const std::vector<CgRequest> &reqs, BatchLaunch &l) {
+    constexpr int nc = 1, w = kResRowShort;
+    constexpr bool mixed = true;
+    if (!want_resident(nc, mixed)) return false;
+    std::vector<int> cap;
+    int tiles = 0, grid = 0;
+    size_t lds = 0;
+    for (size_t k = 0; k < l.which.size(); ++k) {
+        const Matrix &m = *reqs[l.which[k]].m;
+        ResidentPlan plan;
+        if (m.nnz <= 0 || m.max_row_nz > w || l.blocks[k] > kFlatMax ||
+            !res_fits(m, nc, mixed, w, kResWavesBatch, l.blocks[k], plan))
+            return false;
+        cap.push_back(plan.cap);
+        tiles = std::max(tiles, plan.tiles);
+        lds = std::max(lds, plan.lds);
+        grid += l.blocks[k];
+    }
+    const void *fn = res_kernel(nc, mixed, w, tiles, true, kResWavesBatch);
+    if (grid > res_max_grid(d, fn, kResWavesBatch, lds)) return false;
+    l.cap = cap;
+    l.resident = true;
+    l.width = w;
+    l.waves = kResWavesBatch;
+    l.tiles = tiles;
+    l.lds = lds;
+    return true;
 }
 
 }  // namespace
@@ -4681,8 +4713,8 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
     }
     bool idx16 = want_idx16();
     int wi = 4;
-    std::vector<BatchLaunch> launches =
-        resident_launches(d, reqs, nc, mixed, std::max(1, block_scale));
+    std::vector<BatchLaunch> launches;
+    if (!mixed) launches = resident_launches(d, reqs, nc, mixed, std::max(1, block_scale));
     if (launches.empty()) {
         // batched launches run 1024-thread blocks: one load per nonzero per
         // lane unless NSFEM_CG_PHASE says otherwise
@@ -4707,6 +4739,17 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
             l.blocks = split_blocks(rq, maxg, std::max(1, block_scale));
             l.cap.assign(rq.size(), 0);
             launches.push_back(std::move(l));
+        }
+        // Refined one-column solves: resident on the streaming form's split
+        // (its bits) where that fits.  A batch that wants more blocks than
+        // the device has gives its small systems more tiles a wave than the
+        // registers hold and takes the resident form's split (other bits, as
+        // any change of the batch's split): 64 cavities of 16^2 to 256^2,
+        // autotuned, 6.16 batch-steps/s streaming, 11.4 resident.
+        if (mixed && nc == 1 && !(launches.size() == 1 && batch_resident(d, reqs, launches[0]))) {
+            std::vector<BatchLaunch> own =
+                resident_launches(d, reqs, nc, mixed, std::max(1, block_scale));
+            if (!own.empty()) launches.swap(own);
         }
     }
     int worst = NSFEM_OK;
@@ -4768,6 +4811,12 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
             for (int k = 0; k < nb[i]; ++k) map.push_back(make_int2((int)i, k));
         }
         const int grid = (int)map.size();
+        if (std::getenv("NSFEM_CG_VERBOSE"))  // one line per launch, in launch order
+            std::fprintf(stderr,
+                         "[nsfem] cg batch launch instances=%zu cols=%d grid=%d mixed=%d "
+                         "resident=%d waves=%d tiles=%d\n",
+                         I, nc, grid, (int)mixed, launch.resident ? launch.width : 0,
+                         launch.waves, launch.tiles);
         d.batch_map.ensure(map.size());
         NSFEM_HIP(hipMemcpyAsync(d.batch_args.ptr, args.data(), sizeof(CgArgs) * I,
                                  hipMemcpyHostToDevice, d.stream));
@@ -4784,12 +4833,12 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
         const int2 *dmap = d.batch_map.ptr;
         if (launch.resident) {
             void *kargs[] = {(void *)&dargs, (void *)&dmap};
-            ResMaxGrid mg{d, launch.lds, true, 0};
-            res_dispatch(nc, mixed, launch.width, launch.tiles, mg);
-            NSFEM_REQUIRE(grid <= mg.out, NSFEM_ERROR,
+            const void *fn =
+                res_kernel(nc, mixed, launch.width, launch.tiles, true, launch.waves);
+            NSFEM_REQUIRE(grid <= res_max_grid(d, fn, launch.waves, launch.lds), NSFEM_ERROR,
                           "batched CG: block split exceeds co-residency");
-            res_dispatch(nc, mixed, launch.width, launch.tiles,
-                         ResLaunch{d, kargs, grid, launch.lds, true});
+            NSFEM_HIP(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(64 * launch.waves), kargs,
+                                                 (unsigned)launch.lds, d.stream));
         } else {
             CgBatchLaunch ln{d, dargs, dmap, grid};
             cg_dispatch(nc, mixed, idx16, wi, ln);

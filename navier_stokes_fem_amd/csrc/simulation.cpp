@@ -2025,8 +2025,8 @@ void simulation_step(Simulation &s, int steps, nsfem_step_stats *stats) {
 // Several simulations stepped together: the per-instance stages (advection,
 // right-hand sides, boundary values) are launched instance by instance, and
 // each of the three solve kinds (u/v diffusion as a 2-column solve, pressure,
-// u/v mass as a 2-column solve) runs for every instance in one persistent
-// launch (run_cg_batch).
+// u/v mass as a 2-column solve) runs for all instances in one persistent
+// launch, or a few where the device's blocks do not hold them (run_cg_batch).
 void simulation_step_batch(const std::vector<Simulation *> &S, int steps,
                            nsfem_step_stats *stats) {
     NSFEM_REQUIRE(!S.empty(), NSFEM_INVALID_ARGUMENT, "empty batch");
