@@ -2584,7 +2584,16 @@ struct CgCtl {
     double pend[NC], alpha[NC], beta[NC], g[NC];
     int iters[NC], status[NC], stall[NC], active[NC], dropped[NC];
     int k, last_ru, refines, ru, has_pend, out_of_iters, any;
+    int range;  // FP64: a sum past the recurrence's range
 };
+
+// Status of a resident FP64 solve that left the range of its recurrence (no
+// public status is positive): x is as it was, and the streaming form, which
+// sums (r, r) itself, runs the solve.
+constexpr int kCgOutOfRange = 1;
+// Least (r, r), (q, q) and alpha^2, 2^-963 or 1.3e-290 (high word), whose
+// terms' underflow below 1e-307 is lost in rounding.
+constexpr int kCgLeastSum = 60 << 20;
 
 // After the set-up residual: acc[c] = (r, r) in FP64, acc[NC + c] = (b, b),
 // acc[2 NC + c] = (r, r) of the stored r.
@@ -2616,7 +2625,7 @@ __device__ void ctl_start(CgCtl<NC> &C, const CgArgs &A, const double (&acc)[3 *
             A.res[c].tolerance = tol;
         }
     }
-    C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = 0;
+    C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = C.range = 0;
 }
 
 // After the phase reduction: alpha_k, gamma_{k+1} and the reliable-update
@@ -2625,12 +2634,15 @@ __device__ void ctl_start(CgCtl<NC> &C, const CgArgs &A, const double (&acc)[3 *
 // rounding must not pile up over a steep fall); ru_gap iterations and the
 // iteration limit force one.  sums[4 c ...] = (p, q), (r, r), (r, q), (q, q).
 // MIXED = false (FP64): no updates; a column is done when its recursive
-// residual meets the tolerance.
+// residual meets the tolerance, and C.range is raised where that residual
+// cannot be formed: (q, q) of a matrix near 1e-170 underflows and alpha^2
+// overflows, (q, q) of one near 1e150 overflows, while (r, r) and (p, q) are
+// in range.  (The test costs 0.4 to 0.8% of an FP64 solve.)
 template <int NC, bool MIXED = true>
 __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&sums)[4 * NC]) {
     const int k = ++C.k;
     const double d2 = A.rdelta * A.rdelta;
-    bool want = false, any = false;
+    bool want = false, any = false, out = false;
     for (int c = 0; c < NC; ++c) {
         double alpha = 0.0, g = 0.0;
         bool dropped = false;
@@ -2644,9 +2656,16 @@ __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&su
                 alpha = gk / delta;
                 // gk - 2 alpha (r, q) + alpha^2 (q, q), its roundings spelt out:
                 // the same bits in every kernel this is inlined into
-                g = fmax(__builtin_fma(alpha * alpha, sums[4 * c + 3],
-                                       __builtin_fma(-2.0 * alpha, sums[4 * c + 2], gk)),
-                         0.0);
+                g = __builtin_fma(alpha * alpha, sums[4 * c + 3],
+                                  __builtin_fma(-2.0 * alpha, sums[4 * c + 2], gk));
+                if (!MIXED) {
+                    // (non-negative doubles compare as their high words)
+                    const int least = min(min(__double2hiint(gk), __double2hiint(sums[4 * c + 3])),
+                                          __double2hiint(alpha * alpha));
+                    out = out || (least < kCgLeastSum && gk != 0.0) ||
+                          (__double2hiint(g) & 0x7ff00000) == 0x7ff00000;  // infinite or NaN
+                }
+                g = fmax(g, 0.0);
                 C.gamma[c] = gk;
                 C.iters[c] = k;
                 if (MIXED) {
@@ -2665,6 +2684,13 @@ __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&su
         C.alpha[c] = alpha;
         C.g[c] = g;
         C.dropped[c] = dropped;
+    }
+    if (!MIXED && out) {
+        C.range = 1;
+        for (int c = 0; c < NC; ++c) {
+            C.active[c] = 0;
+            C.status[c] = kCgOutOfRange;
+        }
     }
     C.has_pend = 1;
     C.out_of_iters = k >= A.max_iter;
@@ -3766,11 +3792,14 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             par ^= 1;
         }
     }
+    // (the same sums in every block, so the same C.range)
+    if (MIXED || !C.range) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-        if (row[j] < 0) continue;
+        for (int j = 0; j < R; ++j) {
+            if (row[j] < 0) continue;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) A.x[(size_t)c * A.n + row[j]] = x[j].v[c];
+            for (int c = 0; c < NC; ++c) A.x[(size_t)c * A.n + row[j]] = x[j].v[c];
+        }
     }
     if (writer) ctl_finish<NC>(C, A);
     return;
@@ -4298,7 +4327,7 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
                         : std::min(maxg, std::max(1, m.n_wtiles / (per_wave * (bs / 64))));
     grid = std::max(1, std::min(grid, std::max(1, m.n_wtiles)));
     ResidentPlan res;
-    if (want_resident(nc, mixed))
+    if (req.resident && want_resident(nc, mixed))
         res = want > 0 ? plan_resident(m, nc, mixed, want, d.cu_count)
                        : resident_plan(d, m, nc, mixed);
     const void *res_fn = nullptr;
@@ -4369,6 +4398,12 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
         float ms = 0.f;
         NSFEM_HIP(hipEventElapsedTime(&ms, d.ev_start, d.ev_stop));
         P.ms += ms;
+        if (P.res[0].status == kCgOutOfRange) {
+            CgRequest r2 = req;
+            r2.resident = false;
+            cg_pass(d, r2, mixed, P, fixed);
+            return;
+        }
         bool drift = false;
         if (!mixed) true_residuals(d, m, req.b, req.x, nc, (double *)a.q, ws, P.final_res);
         for (int c = 0; c < nc; ++c) {
@@ -4871,6 +4906,24 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
         for (size_t i = 0; i < I; ++i) {
             const CgRequest &r = *rq[i];
             bool redo = false;
+            if (res[2 * i].status == kCgOutOfRange) {
+                // from the x it came with, in the streaming form
+                nsfem_cg_stats *st = stats + 2 * launch.which[i];
+                int st2 = NSFEM_BREAKDOWN;
+                if (finish) {
+                    CgRequest r2 = r;
+                    r2.resident = false;
+                    st2 = run_cg(d, r2, st);
+                    if (batch_seconds) *batch_seconds += st[0].seconds;
+                } else {
+                    for (int c = 0; c < nc; ++c) {
+                        st[c] = nsfem_cg_stats{};
+                        st[c].status = st2;
+                    }
+                }
+                if (st2 != NSFEM_OK && worst == NSFEM_OK && finish) worst = st2;
+                continue;
+            }
             for (int c = 0; c < nc; ++c) {
                 const CgColumnResult &cr = res[2 * i + c];
                 if (cr.status == NSFEM_BARRIER_TIMEOUT)

@@ -328,6 +328,7 @@ struct CgRequest {
     double reliable_delta = 0.5;
     int ru_gap = 0;   // mixed: forced reliable update after this many iterations (0 = 20000)
     int grid = 0;     // 0 = automatic
+    bool resident = true;  // may take the resident form
     bool jacobi = false;  // mixed: CG on D^-1/2 A D^-1/2 (Jacobi-preconditioned CG)
 };
 // Runs the persistent CG; fills stats[ncol].  Returns the worst status.

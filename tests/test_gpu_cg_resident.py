@@ -147,3 +147,57 @@ def test_resident_ends_as_streaming(gpu, monkeypatch, capfd, columns, precision)
         # a few steps from the same start: only the sums' order differs
         np.testing.assert_allclose(got[fine], want[fine], rtol=1e-4 if i == 1 else 1e-6,
                                    atol=1e-9 * (1 + np.abs(want[fine]).max(initial=0.0)))
+
+
+# (scale of the matrix, scale of the solution): (q, q) underflows; alpha^2
+# overflows; (q, q) overflows while (r, r) and (p, q) do not; the residual's
+# own squares leave the range
+SCALES = [(1e-170, 1.0), (1e-170, 1e100), (1e150, 1e-75), (1e150, 1e-160), (1e-60, 1e-100),
+          (1e160, 1e-80), (2.0 ** 300, 2.0 ** -200)]
+
+
+@pytest.mark.parametrize("columns", [1, 2])
+@pytest.mark.parametrize("n", [700, 9000])
+@pytest.mark.parametrize("matrix,solution", SCALES)
+def test_scales_past_the_recurrence(gpu, oracle, monkeypatch, capfd, n, columns, matrix, solution):
+    """FP64 at scales where the next (r, r) cannot be formed from (r, q) and
+    (q, q): the solve ends as the streaming one, which adds (r, r) itself."""
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    A = banded(n, (1, 30, 31), n)
+    A = (A[0], A[1], A[2] * matrix)
+    x = np.random.default_rng(n).standard_normal(columns * n) * solution
+    zero = np.zeros(n)
+    b = np.concatenate([oracle.spmv_sub(A, zero, -x[c * n:(c + 1) * n]) for c in range(columns)])
+    got, st, _ = solve(gpu, A, b, np.zeros(columns * n), columns, "fp64", capfd)
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", "0")
+    want, ref, _ = solve(gpu, A, b, np.zeros(columns * n), columns, "fp64", capfd)
+    assert [s["status"] for s in st] == [s["status"] for s in ref]
+    assert [s["iterations"] for s in st] == pytest.approx([s["iterations"] for s in ref], abs=2)
+    np.testing.assert_allclose(got, want, rtol=0, atol=1e-8 * solution)
+
+
+def test_scales_past_the_recurrence_in_a_batch(gpu, monkeypatch, capfd):
+    """Two of a batch's systems leave the recurrence's range ((q, q) below
+    1e-290): they run alone in the streaming form, the third stays."""
+    from navier_stokes_fem_amd import mesh
+    from navier_stokes_fem_amd.simulation import Simulation, step_batch
+
+    out = []
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    for resident in ("1", "0"):
+        monkeypatch.setenv("NSFEM_CG_RESIDENT", resident)
+        sims = [Simulation(mesh.cavity(n, lid_speed=lid), 1e-3, 5e-3, device=gpu, rtol=1e-6,
+                           precision="fp64") for n, lid in ((12, 1e-144), (16, 1.0), (20, 1e-144))]
+        capfd.readouterr()
+        stats = step_batch(sims, 2)
+        alone = [line for line in capfd.readouterr().err.splitlines() if "cg launch" in line]
+        assert bool(alone) == (resident == "1")
+        assert all("resident=0" in line for line in alone)
+        out.append(([s.fields() for s in sims], [st["cg_iterations"] for st in stats]))
+        for s in sims:
+            s.close()
+    (got, its), (want, ref) = out
+    for a, b, i, j in zip(got, want, its, ref):
+        assert np.abs(np.subtract(i, j)).max() <= 4
+        for fa, fb in zip(a, b):
+            np.testing.assert_allclose(fa, fb, rtol=0, atol=1e-3 * np.abs(fb).max())
