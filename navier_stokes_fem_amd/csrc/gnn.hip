@@ -820,11 +820,13 @@ GnnNet *gnn_create(Device &d, uint64_t seed) {
     g->wt3.resize(H * K2);
     g->wr3.resize(H * K2);
     NSFEM_HIP(hipMemcpy(g->params.ptr, h.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice));
-    NSFEM_HIP(hipMemset(g->grads.ptr, 0, NPARAM * sizeof(float)));
-    NSFEM_HIP(hipMemset(g->m.ptr, 0, NPARAM * sizeof(float)));
-    NSFEM_HIP(hipMemset(g->v.ptr, 0, NPARAM * sizeof(float)));
-    NSFEM_HIP(hipMemset(g->clip.ptr, 0, 2 * sizeof(float)));
-    NSFEM_HIP(hipMemset(g->wt1.ptr, 0, H * K1 * sizeof(uint16_t)));  // the padding
+    // (cleared on the stream that packs and trains: it does not wait for the
+    // null stream, and a late clear of wt1 would wipe the packed weights)
+    NSFEM_HIP(hipMemsetAsync(g->grads.ptr, 0, NPARAM * sizeof(float), d.stream));
+    NSFEM_HIP(hipMemsetAsync(g->m.ptr, 0, NPARAM * sizeof(float), d.stream));
+    NSFEM_HIP(hipMemsetAsync(g->v.ptr, 0, NPARAM * sizeof(float), d.stream));
+    NSFEM_HIP(hipMemsetAsync(g->clip.ptr, 0, 2 * sizeof(float), d.stream));
+    NSFEM_HIP(hipMemsetAsync(g->wt1.ptr, 0, H * K1 * sizeof(uint16_t), d.stream));  // the padding
     gnn_pack(*g);
     NSFEM_HIP(hipStreamSynchronize(d.stream));
     return g;

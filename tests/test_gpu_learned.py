@@ -278,3 +278,22 @@ def test_learned_warm_start_gain(gpu):
     assert it["learned_projection"] <= 1.02 * it["projection"]
     for net in nets.values():
         net.close()
+
+
+def test_a_new_net_runs_on_its_weights(gpu):
+    """A network's packed weights are whole as soon as it exists: its
+    gradients (the readout's see every layer) are those of the same network
+    after its weights were set."""
+    from navier_stokes_fem_amd import learned as L
+
+    og, pg, b, p, bb, pb = _setup(gpu, _mesh("cavity"), seed=3)
+    for seed in range(10):
+        net = L.WarmStartNet(gpu, seed=seed)
+        loss, fresh = net.gradients(pg, bb, pb)
+        net.set_params(net.get_params())
+        again, want = net.gradients(pg, bb, pb)
+        assert loss == again
+        np.testing.assert_array_equal(fresh, want)
+        assert np.abs(L.WarmStartNet.unflatten(fresh)["w4"]).max() > 0
+        net.close()
+    pg.close()

@@ -6,7 +6,8 @@
   cpp/kd_tree_builder.cpp:81-148) and FEM assembly (include/assembly.h:
   1302-1475) are bit-identical to the oracle's;
 * the mesh generators produce the layouts the kernels assume;
-* bench.py refuses more than one GPU before touching a device.
+* bench.py refuses more than one GPU before touching a device;
+* no clear of device memory is left unordered with the device's stream.
 """
 import ctypes as C
 import json
@@ -247,3 +248,22 @@ def test_cpp_device_header_compiles(tmp_path):
                           "-I" + os.path.join(ROOT, "include"), str(src)],
                          capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stderr
+
+
+def test_clears_are_ordered_with_the_stream():
+    """The device's stream does not wait for the null stream, and hipMemset
+    returns before it has run: device memory is cleared on the device's
+    stream, or (where the null stream's kernels use it) a blocking copy on the
+    null stream follows before anything runs on the device's."""
+    csrc = os.path.join(ROOT, "navier_stokes_fem_amd", "csrc")
+    seen = 0
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".hip", ".cpp", ".hpp")):
+            continue
+        text = open(os.path.join(csrc, name)).read()
+        for m in re.finditer(r"\bhipMemset\(", text):
+            seen += 1
+            line = text.count("\n", 0, m.start()) + 1
+            nxt = re.search(r"\bhipMemcpy\(|\bd\.stream\b|^}", text[m.start():], re.M)
+            assert nxt and nxt.group().startswith("hipMemcpy"), (name, line)
+    assert seen > 0
