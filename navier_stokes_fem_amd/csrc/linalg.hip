@@ -4062,10 +4062,14 @@ const void *res_kernel(int nc, bool mixed, int w, int tiles, bool batch, int wav
                  : res_kernel_tiles<1, false, L>(batch, waves, tiles);
 }
 
-// Allows a kernel its dynamic LDS and returns the blocks a device holds.
+// Allows a kernel the most dynamic LDS of any solve and returns the blocks a
+// device holds with this solve's.  (The attribute belongs to the kernel, in
+// every thread and device handle: a solve's own amount would lower it between
+// another handle's call here and its launch.)
 int res_max_grid(Device &d, const void *kernel, int waves, size_t lds) {
     if (lds > 48 * 1024)
-        NSFEM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        NSFEM_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)kResLds));
     int per_cu = 0;
     NSFEM_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, lds));
     return std::min(per_cu * d.cu_count, kResMaxBlocks);

@@ -149,6 +149,26 @@ def test_resident_ends_as_streaming(gpu, monkeypatch, capfd, columns, precision)
                                    atol=1e-9 * (1 + np.abs(want[fine]).max(initial=0.0)))
 
 
+def test_windows_of_two_handles(gpu, monkeypatch, capfd):
+    """Two device handles solve by turns with the same kernel, one with a
+    window of some 100 KB of LDS, the other of some 50: what a kernel may take
+    is not one solve's."""
+    from navier_stokes_fem_amd.device import GPUSimulationDevice
+
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    other = GPUSimulationDevice(0)
+    systems = [(gpu, banded(12000, (1, 2500), 21)), (other, banded(12000, (1, 1200), 22))]
+    b = np.random.default_rng(23).standard_normal(12000)
+    first = [None, None]
+    for turn in range(3):
+        for k, (dev, A) in enumerate(systems):
+            x, st, resident = solve(dev, A, b, np.zeros(12000), 1, "fp64", capfd)
+            assert resident and st[0]["status"] == 0
+            if turn == 0:
+                first[k] = x
+            np.testing.assert_array_equal(x, first[k])
+
+
 # (scale of the matrix, scale of the solution): (q, q) underflows; alpha^2
 # overflows; (q, q) overflows while (r, r) and (p, q) do not; the residual's
 # own squares leave the range
