@@ -265,6 +265,8 @@ void build_wave_tiles(Matrix &m, int rows, int nnz) {
     m.n_wtiles = (int)w.size() - 1;
     m.host_wtiles = w;
     for (auto &plan : m.res_plan) plan = ResidentPlan{};
+    for (auto &plan : m.batch_least) plan = ResidentPlan{};
+    for (auto &plan : m.batch_plan) plan = ResidentPlan{};
     m.host_wtile_prefix.assign(w.size(), 0);
     for (int i = 0; i < m.n_wtiles; ++i)
         m.host_wtile_prefix[i + 1] =
@@ -4622,6 +4624,37 @@ struct BatchLaunch {
     size_t lds = 0;
 };
 
+// Plans of a system in a batch's resident launch, kept with the matrix's tiles
+// as a single solve's is: a step plans three or more launches of the same
+// matrices, and each plan walks a system's wave tiles.
+int batch_kind(int nc, bool mixed, int w, int waves) {
+    if (waves == kResWavesBatch) return 4;
+    return mixed ? 3 : nc == 2 ? 2 : w == kResRowLong ? 1 : 0;
+}
+const ResidentPlan &batch_plan(Matrix &m, int nc, bool mixed, int w, int waves, int blocks) {
+    ResidentPlan &plan = m.batch_plan[batch_kind(nc, mixed, w, waves)];
+    if (!plan.made || plan.asked != blocks) {
+        plan = ResidentPlan{};
+        res_fits(m, nc, mixed, w, waves, blocks, plan);
+        plan.made = true;
+        plan.asked = blocks;
+    }
+    return plan;
+}
+// On the fewest blocks, at most `most`.
+const ResidentPlan &batch_least(Matrix &m, int nc, bool mixed, int w, int waves, int most) {
+    ResidentPlan &plan = m.batch_least[batch_kind(nc, mixed, w, waves)];
+    if (!plan.made || plan.asked != most) {
+        plan = ResidentPlan{};
+        const int room = waves * res_tiles(mixed, w);
+        int g = (m.n_wtiles + room - 1) / room;
+        while (g <= std::min(most, m.n_wtiles) && !res_fits(m, nc, mixed, w, waves, g, plan)) ++g;
+        plan.made = true;
+        plan.asked = most;
+    }
+    return plan;
+}
+
 // The launches of a batch in the resident form, or none when a system does
 // not allow it (refined: two columns and long rows never do).  Systems go
 // largest first, so that those of like iteration counts share a launch, each
@@ -4638,7 +4671,6 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
         if (m.max_row_nz > kResRowShort) w = kResRowLong;
     }
     if (mixed && w == kResRowLong) return out;
-    const int room = kResWaves * res_tiles(mixed, w);
     const int maxg = res_max_grid(d, res_kernel(nc, mixed, w, res_tiles(mixed, w), true), kResWaves,
                                   kResLds);
     std::vector<size_t> order(reqs.size());
@@ -4651,11 +4683,9 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
     std::vector<int> least(reqs.size());
     int used = maxg + 1;
     for (size_t i : order) {
-        const Matrix &m = *reqs[i].m;
-        ResidentPlan plan;
-        int g = (m.n_wtiles + room - 1) / room;
-        while (g <= std::min(maxg, m.n_wtiles) && !res_fits(m, nc, mixed, w, kResWaves, g, plan)) ++g;
+        const ResidentPlan &plan = batch_least(*reqs[i].m, nc, mixed, w, kResWaves, maxg);
         if (!plan.ok) return std::vector<BatchLaunch>();
+        const int g = plan.grid;
         least[i] = g;
         if (used + g > maxg) {
             out.emplace_back();
@@ -4680,14 +4710,14 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
         l.width = w;
         l.waves = kResWaves;
         for (size_t k = 0; k < rq.size(); ++k) {
-            ResidentPlan plan;
-            if (!res_fits(*rq[k]->m, nc, mixed, w, kResWaves, l.blocks[k], plan)) {
-                l.blocks[k] = nb[k];
-                res_fits(*rq[k]->m, nc, mixed, w, kResWaves, nb[k], plan);
+            const ResidentPlan *plan = &batch_plan(*rq[k]->m, nc, mixed, w, kResWaves, l.blocks[k]);
+            if (!plan->ok) {
+                plan = &batch_least(*rq[k]->m, nc, mixed, w, kResWaves, maxg);
+                l.blocks[k] = plan->grid;
             }
-            l.cap.push_back(plan.cap);
-            l.tiles = std::max(l.tiles, plan.tiles);
-            l.lds = std::max(l.lds, plan.lds);
+            l.cap.push_back(plan->cap);
+            l.tiles = std::max(l.tiles, plan->tiles);
+            l.lds = std::max(l.lds, plan->lds);
         }
     }
     return out;
@@ -4712,11 +4742,10 @@ bool batch_resident(Device &d, const std::vector<CgRequest> &reqs, BatchLaunch &
     int tiles = 0, grid = 0;
     size_t lds = 0;
     for (size_t k = 0; k < l.which.size(); ++k) {
-        const Matrix &m = *reqs[l.which[k]].m;
-        ResidentPlan plan;
-        if (m.nnz <= 0 || m.max_row_nz > w || l.blocks[k] > kFlatMax ||
-            !res_fits(m, nc, mixed, w, kResWavesBatch, l.blocks[k], plan))
-            return false;
+        Matrix &m = *reqs[l.which[k]].m;
+        if (m.nnz <= 0 || m.max_row_nz > w || l.blocks[k] > kFlatMax) return false;
+        const ResidentPlan &plan = batch_plan(m, nc, mixed, w, kResWavesBatch, l.blocks[k]);
+        if (!plan.ok) return false;
         cap.push_back(plan.cap);
         tiles = std::max(tiles, plan.tiles);
         lds = std::max(lds, plan.lds);

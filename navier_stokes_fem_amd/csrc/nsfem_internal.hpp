@@ -118,6 +118,7 @@ struct ResidentPlan {
     int grid = 0;    // blocks
     int cap = 0;     // rows of the largest block window
     size_t lds = 0;  // bytes of dynamic LDS
+    int asked = 0;   // batches: the blocks (or the most of them) it was made for
 };
 
 struct Matrix {
@@ -140,6 +141,9 @@ struct Matrix {
     // the diagonal, and the resident solves' plans by columns and precision
     int max_row_nz = 0, band_lo = 0, band_hi = 0;
     ResidentPlan res_plan[4];
+    // the batched ones by kernel (batch_kind): the fewest blocks the system
+    // fits in, and the plan on the blocks of the last batch
+    ResidentPlan batch_least[5], batch_plan[5];
     // ownership of wave tiles by persistent blocks, cached per grid size:
     // both arrays hold kMaxGridBlocks + 1 entries from the tiling on, so a
     // change of grid size copies and never allocates
