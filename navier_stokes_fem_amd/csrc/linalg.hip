@@ -2586,7 +2586,6 @@ struct CgCtl {
     double pend[NC], alpha[NC], beta[NC], g[NC];
     int iters[NC], status[NC], stall[NC], active[NC], dropped[NC];
     int k, last_ru, refines, ru, has_pend, out_of_iters, any;
-    int range;  // FP64: a sum past the recurrence's range
 };
 
 // Status of a resident FP64 solve that left the range of its recurrence (no
@@ -2627,7 +2626,7 @@ __device__ void ctl_start(CgCtl<NC> &C, const CgArgs &A, const double (&acc)[3 *
             A.res[c].tolerance = tol;
         }
     }
-    C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = C.range = 0;
+    C.k = C.last_ru = C.refines = C.ru = C.has_pend = C.out_of_iters = 0;
 }
 
 // After the phase reduction: alpha_k, gamma_{k+1} and the reliable-update
@@ -2636,8 +2635,8 @@ __device__ void ctl_start(CgCtl<NC> &C, const CgArgs &A, const double (&acc)[3 *
 // rounding must not pile up over a steep fall); ru_gap iterations and the
 // iteration limit force one.  sums[4 c ...] = (p, q), (r, r), (r, q), (q, q).
 // MIXED = false (FP64): no updates; a column is done when its recursive
-// residual meets the tolerance, and C.range is raised where that residual
-// cannot be formed: (q, q) of a matrix near 1e-170 underflows and alpha^2
+// residual meets the tolerance, and all end as kCgOutOfRange where that
+// residual cannot be formed: (q, q) of a matrix near 1e-170 underflows and alpha^2
 // overflows, (q, q) of one near 1e150 overflows, while (r, r) and (p, q) are
 // in range.  (The test costs 0.4 to 0.8% of an FP64 solve.)
 template <int NC, bool MIXED = true>
@@ -2688,7 +2687,6 @@ __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&su
         C.dropped[c] = dropped;
     }
     if (!MIXED && out) {
-        C.range = 1;
         for (int c = 0; c < NC; ++c) {
             C.active[c] = 0;
             C.status[c] = kCgOutOfRange;
@@ -3794,8 +3792,8 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             par ^= 1;
         }
     }
-    // (the same sums in every block, so the same C.range)
-    if (MIXED || !C.range) {
+    // (the same sums in every block, so the same status)
+    if (MIXED || C.status[0] != kCgOutOfRange) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             if (row[j] < 0) continue;
@@ -4146,6 +4144,25 @@ const ResidentPlan &resident_plan(Device &d, Matrix &m, int nc, bool mixed) {
     return plan;
 }
 
+// Blocks of a streaming solve of `waves` waves each, before the device's
+// limit: two wave tiles a wave.  One-column mixed solves of matrices that fit
+// the resident form take its grid (a comparison run then has its bits); of
+// long rows that do not fit, one tile a wave up to 96 blocks and where two
+// need more than the flat reduction takes, as the reduction grows with the
+// blocks (microseconds a solve at one and two tiles a wave, mass matrices in
+// the reference's node order, 29 to 34 iterations: 16,597 rows 557 and 694,
+// 37,062 727 and 735, 65,657 865 and 846, 82,990 1,072 and 962, 102,372 1,170
+// and 1,064, 147,220 1,357 and 1,382).
+int streaming_blocks(Device &d, Matrix &m, int nc, bool mixed, int waves) {
+    const int two = m.n_wtiles / (2 * waves), one = m.n_wtiles / waves;
+    if (!(mixed && nc == 1)) return two;
+    if (waves == kResWaves) {
+        const ResidentPlan &res = resident_plan(d, m, nc, mixed);
+        if (res.ok) return res.grid;
+    }
+    return cg_tiles_per_wave(m) == 1 && (one <= 96 || two > kFlatMax) ? one : two;
+}
+
 // Whether a solve may take the resident form: not when a comparison run asks
 // for one of the streaming forms (NSFEM_CG_RESIDENT=0, or the form's own
 // switches; read at every solve).
@@ -4327,11 +4344,8 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
         const char *env = std::getenv("NSFEM_CG_GRID");
         if (env) want = std::atoi(env);
     }
-    // (the one-column mixed form shares its grid with its resident form)
-    const int per_wave = mixed && nc == 1 ? cg_tiles_per_wave(m) : 2;
-    int grid = want > 0 ? std::min(want, maxg)
-                        : std::min(maxg, std::max(1, m.n_wtiles / (per_wave * (bs / 64))));
-    grid = std::max(1, std::min(grid, std::max(1, m.n_wtiles)));
+    int grid = want > 0 ? want : streaming_blocks(d, m, nc, mixed, bs / 64);
+    grid = std::max(1, std::min(std::min(grid, maxg), std::max(1, m.n_wtiles)));
     ResidentPlan res;
     if (req.resident && want_resident(nc, mixed))
         res = want > 0 ? plan_resident(m, nc, mixed, want, d.cu_count)
