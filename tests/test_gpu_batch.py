@@ -21,10 +21,13 @@ def _batch(gpu, specs, precision, rtol):
 SPECS = [(8, 1.0, 0.01), (20, 0.7, 0.002), (12, 1.9, 0.005), (16, 1.2, 0.001), (10, 0.5, 0.008)]
 
 
+@pytest.mark.parametrize("resident", ["1", "0"])
 @pytest.mark.parametrize("precision", ["fp64", "fp32_refined"])
-def test_batch_matches_individual_steps(gpu, precision):
+def test_batch_matches_individual_steps(gpu, monkeypatch, capfd, precision, resident):
     from navier_stokes_fem_amd.simulation import step_batch
 
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", resident)
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
     # the FP32 form is run at 1e-9: on these tiny systems a tighter
     # tolerance exhausts the default iteration limit (the row count)
     rtol = 1e-11 if precision == "fp64" else 1e-9
@@ -33,7 +36,10 @@ def test_batch_matches_individual_steps(gpu, precision):
     many = _batch(gpu, SPECS, precision, rtol)
     for s in one:
         s.step(4)
+    capfd.readouterr()
     stats = step_batch(many, 4)
+    form = {cols: waves > 0 for _, cols, waves in _launches(capfd.readouterr().err)}
+    assert form == {1: resident == "1", 2: resident == "1" and precision == "fp64"}
     assert len(stats) == len(SPECS)
     for a, b, st in zip(one, many, stats):
         assert st["steps"] == 4
@@ -203,3 +209,77 @@ def test_refined_batch_past_the_device(gpu, monkeypatch, capfd):
     for a, b in zip(got, want):
         for fa, fb in zip(a, b):
             assert np.linalg.norm(fa - fb) <= 2e-3 * np.linalg.norm(fb)
+
+
+def _shuffled(n, seed):
+    """The n^2 cavity with its pressure nodes in random order: no window of
+    rows holds the columns of a block's."""
+    from navier_stokes_fem_amd import mesh
+
+    m = mesh.cavity(n)
+    old = np.arange(m.node_count)
+    old[:m.pressure_count] = np.random.default_rng(seed).permutation(m.pressure_count)
+    new = np.empty_like(old)
+    new[old] = np.arange(m.node_count)
+    return mesh.Mesh(nodes=m.nodes[old], elements=new[m.elements].astype(m.elements.dtype),
+                     pressure_count=m.pressure_count,
+                     vel_bc_nodes=new[m.vel_bc_nodes].astype(m.vel_bc_nodes.dtype),
+                     vel_bc_u=m.vel_bc_u, vel_bc_v=m.vel_bc_v,
+                     p_bc_nodes=new[m.p_bc_nodes].astype(m.p_bc_nodes.dtype),
+                     p_bc_values=m.p_bc_values, name=m.name, info=m.info, grid=None)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32_refined"])
+def test_batch_with_a_system_that_streams(gpu, monkeypatch, capfd, precision):
+    """A pressure system past the resident form's window sends its launch to
+    the streaming form; every solve meets its tolerance and the instances match
+    the same simulations stepped alone (solves to 1e-9, as in
+    test_batch_matches_individual_steps)."""
+    from navier_stokes_fem_amd import mesh
+    from navier_stokes_fem_amd.simulation import Simulation, step_batch
+
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    n = 126 if precision == "fp64" else 180  # 8 and 4 bytes a row of the window
+    meshes = [mesh.cavity(12), _shuffled(n, 1), mesh.cavity(20)]
+    one, many = ([Simulation(m, 0.01, 0.005, device=gpu, rtol=1e-9, precision=precision)
+                  for m in meshes] for _ in range(2))
+    for s in one:
+        s.step(1)
+    capfd.readouterr()
+    stats = step_batch(many, 1)
+    launches = _launches(capfd.readouterr().err)
+    assert (3, 1, 0) in launches and (3, 1, 12) not in launches and (3, 1, 16) not in launches
+    for a, b, st in zip(one, many, stats):
+        assert max(st["max_relative_residual"]) <= 1e-9 * 1.01
+        for fa, fb in zip(a.fields(), b.fields()):
+            assert np.linalg.norm(fa - fb) <= 1e-3 * np.linalg.norm(fa)
+    for s in one + many:
+        s.close()
+
+
+@pytest.mark.parametrize("resident", ["1", "0"])
+def test_batch_of_more_instances_than_blocks(gpu, monkeypatch, capfd, resident):
+    """270 instances: a second launch in either form, with the same fields as
+    alone."""
+    from navier_stokes_fem_amd import mesh
+    from navier_stokes_fem_amd.simulation import Simulation, step_batch
+
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", resident)
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    specs = [(2 + k % 4, 1.0 + k / 270.0, 0.01) for k in range(270)]
+    sims = _batch(gpu, specs, "fp64", 1e-10)
+    capfd.readouterr()
+    stats = step_batch(sims, 1)
+    launches = _launches(capfd.readouterr().err)
+    assert all((waves > 0) == (resident == "1") for _, _, waves in launches)
+    assert len(launches) == 6 and sum(i for i, _, _ in launches) == 3 * 270
+    for k in (0, 3, 255, 256, 269):
+        assert max(stats[k]["max_relative_residual"]) <= 1e-10 * 1.01
+        n, lid, nu = specs[k]
+        alone = Simulation(mesh.cavity(n, lid_speed=lid), nu, 0.005, device=gpu, rtol=1e-10)
+        alone.step(1)
+        for fa, fb in zip(alone.fields(), sims[k].fields()):
+            np.testing.assert_allclose(fb, fa, rtol=0, atol=1e-7 * max(1.0, np.abs(fa).max()))
+        alone.close()
+    for s in sims:
+        s.close()

@@ -5,7 +5,8 @@ residuals are bit-identical; the 768-thread block variant partitions the
 rows differently (other reduction order) and agrees to the solve's
 tolerance.  The form is chosen by NSFEM_CG_PHASE /
 NSFEM_CG_BLOCK, which the library reads at every solve; without them a
-single solve runs group loads in 768-thread blocks."""
+single solve that streams runs group loads in 768-thread blocks, and one that
+runs resident has their bits."""
 import os
 
 import numpy as np
@@ -79,7 +80,9 @@ def test_phase_forms_with_descriptors_beyond_lds(gpu):
             assert got[k][1:] == ref[k][1:], (phase, k, got[k][1:], ref[k][1:])
 
 
-def test_default_form_is_groups_in_wide_blocks(gpu):
+@pytest.mark.parametrize("resident", ["1", "0"])
+def test_default_form_is_groups_in_wide_blocks(gpu, monkeypatch, resident):
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", resident)
     ref = _solves(gpu, "groups", "768")
     got = _solves(gpu, None, None)
     for k in ref:

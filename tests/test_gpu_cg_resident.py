@@ -149,6 +149,29 @@ def test_resident_ends_as_streaming(gpu, monkeypatch, capfd, columns, precision)
                                    atol=1e-9 * (1 + np.abs(want[fine]).max(initial=0.0)))
 
 
+@pytest.mark.parametrize("n,rule", [(20000, "one"), (36000, "two"), (60000, "two"), (100000, "one")])
+def test_streaming_blocks_of_long_rows(gpu, oracle, monkeypatch, capfd, n, rule):
+    """One-column refined solves past the resident window: one wave tile a
+    wave up to 96 blocks and where two tiles need more than 128, else two
+    (tiles of some 28 rows of 19 nonzeros)."""
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+    A = banded(n, (1, 2, 3, 4, 5, 6, 7, 8, n // 2), 31)
+    b = np.random.default_rng(32).standard_normal(n)
+    gpu.upload_csr(6, *A)
+    x = gpu.buffer(np.zeros(n))
+    capfd.readouterr()
+    st = gpu.cg_solve(6, gpu.buffer(b), x, rtol=1e-10, precision="fp32_refined")[0]
+    line = [v for v in capfd.readouterr().err.splitlines() if "cg launch" in v][0]
+    f = dict(w.split("=") for w in line.split() if "=" in w)
+    tiles = int(line.split("wave tiles=")[1].split()[0])
+    one, two = tiles // 12, tiles // 24
+    assert rule == ("one" if one <= 96 or two > 128 else "two")
+    assert f["resident"] == "0"
+    assert int(f["grid"]) == min(int(f["maxgrid"]), one if rule == "one" else two)
+    assert st["status"] == 0
+    assert np.linalg.norm(oracle.spmv_sub(A, b, x.download())) <= 1e-10 * np.linalg.norm(b) * (1 + 1e-9)
+
+
 def test_windows_of_two_handles(gpu, monkeypatch, capfd):
     """Two device handles solve by turns with the same kernel, one with a
     window of some 100 KB of LDS, the other of some 50: what a kernel may take

@@ -188,15 +188,17 @@ def test_cg_matches_oracle(gpu, oracle, which, precision):
         assert st["refinements"] >= 1
 
 
-# two-column mixed forms: the single-reduction iteration (narrow-gather by
-# default, packed) in both block sizes, and the two-phase iteration
-PAIRED_FORMS = [("fp64", {}), ("fp32_refined", {}),
+# two-column forms: the resident one (the default at this size) and the
+# streaming ones, mixed: the single-reduction iteration (narrow-gather,
+# packed) in both block sizes, and the two-phase iteration
+PAIRED_FORMS = [("fp64", {}), ("fp32_refined", {}), ("fp64", {"NSFEM_CG_RESIDENT": "0"}),
+                ("fp32_refined", {"NSFEM_CG_PAIRED": "narrow"}),
                 ("fp32_refined", {"NSFEM_CG_P2_BLOCK": "768", "NSFEM_CG_P2_LOADS": "4"}),
                 ("fp32_refined", {"NSFEM_CG_PAIRED": "packed"}),
                 ("fp32_refined", {"NSFEM_CG_PAIRED": "twophase"})]
 
 
-def test_cg_two_columns(gpu, oracle, monkeypatch):
+def test_cg_two_columns(gpu, oracle, monkeypatch, capfd):
     m, A = _cavity_system(oracle, 20, "diffusion")
     rs, col, val = A
     n = len(rs) - 1
@@ -208,9 +210,12 @@ def test_cg_two_columns(gpu, oracle, monkeypatch):
         print(f"two columns {precision} {env}", flush=True)
         for k, v in env.items():
             monkeypatch.setenv(k, v)
+        monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
+        capfd.readouterr()
         bx = _buf(gpu, np.zeros(2 * n))
         st = gpu.cg_solve(11, _buf(gpu, b), bx, columns=2, rtol=1e-10, precision=precision)
         x = bx.download()
+        assert ("resident=0" in capfd.readouterr().err) == bool(env)
         for c in range(2):
             bc = b[c * n:(c + 1) * n]
             xc = x[c * n:(c + 1) * n]
@@ -231,10 +236,12 @@ def test_cg_two_columns(gpu, oracle, monkeypatch):
             monkeypatch.delenv(k)
 
 
-@pytest.mark.parametrize("env", [{}, {"NSFEM_CG_P2_BLOCK": "768"}, {"NSFEM_CG_PAIRED": "packed"},
+@pytest.mark.parametrize("env", [{}, {"NSFEM_CG_PAIRED": "narrow"}, {"NSFEM_CG_P2_BLOCK": "768"},
+                                 {"NSFEM_CG_PAIRED": "packed"},
                                  {"NSFEM_CG_PAIRED": "packed", "NSFEM_CG_P2_BLOCK": "768"},
                                  {"NSFEM_CG_PAIRED": "twophase"}],
-                         ids=["narrow1024", "narrow768", "packed1024", "packed768", "twophase"])
+                         ids=["resident", "narrow1024", "narrow768", "packed1024", "packed768",
+                              "twophase"])
 def test_cg_two_columns_one_converged(gpu, oracle, monkeypatch, env):
     """A pair whose second column starts at its solution (zero right-hand
     side, zero guess) and one whose second column converges in a handful of
@@ -312,8 +319,10 @@ def test_cg_zero_rhs_and_breakdown(gpu):
     assert ei.value.code == BREAKDOWN
 
 
-def test_cg_large_grid(gpu, oracle):
-    """A system big enough to run on many persistent blocks (grid barrier)."""
+@pytest.mark.parametrize("resident", ["1", "0"])
+def test_cg_large_grid(gpu, oracle, monkeypatch, capfd, resident):
+    """A system big enough to run on many persistent blocks (grid barrier),
+    in the resident and the streaming form."""
     from navier_stokes_fem_amd import device as D
     from navier_stokes_fem_amd import mesh
 
@@ -324,10 +333,14 @@ def test_cg_large_grid(gpu, oracle):
     gpu.upload_csr(15, rs, col, val)
     rng = np.random.default_rng(31)
     b = rng.standard_normal(n)
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", resident)
+    monkeypatch.setenv("NSFEM_CG_VERBOSE", "1")
     for precision in ("fp64", "fp32_refined"):
         bx = _buf(gpu, np.zeros(n))
+        capfd.readouterr()
         st = gpu.cg_solve(15, _buf(gpu, b), bx, rtol=1e-8, precision=precision)[0]
         x = bx.download()
+        assert ("resident=0" in capfd.readouterr().err) == (resident == "0")
         r = np.linalg.norm(oracle.spmv_sub((rs, col, val), b, x))
         assert st["status"] == 0 and r <= 1e-8 * np.linalg.norm(b) * (1 + 1e-9), (precision, st)
 

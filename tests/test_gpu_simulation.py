@@ -400,8 +400,11 @@ def test_export_fields(gpu, tmp_path):
     np.testing.assert_array_equal(sol["v"], v)
     np.testing.assert_array_equal(sol["p"], p)
 
-def test_velocity_jacobi(gpu):
-    """Jacobi-preconditioned velocity solves (CG on D^-1/2 A D^-1/2 in FP32,
+@pytest.mark.parametrize("pair", [False, True], ids=["apart", "paired"])
+@pytest.mark.parametrize("resident", ["1", "0"])
+def test_velocity_jacobi(gpu, monkeypatch, resident, pair):
+    """Jacobi-preconditioned velocity solves, resident and streaming, the
+    columns apart and paired (CG on D^-1/2 A D^-1/2 in FP32,
     x, b and the FP64 residual passes unscaled): every solve meets the same
     unscaled 1e-8 relative residual, the diffusion and mass solves take
     fewer iterations than unscaled, the pressure solve is untouched, and the
@@ -409,12 +412,13 @@ def test_velocity_jacobi(gpu):
     from navier_stokes_fem_amd import mesh
     from navier_stokes_fem_amd.simulation import Simulation
 
+    monkeypatch.setenv("NSFEM_CG_RESIDENT", resident)
     m = mesh.cavity(96)
     out = {}
     for form, prec, jac, rtol in (("tight", "fp64", False, 1e-12), ("plain", "fp32_refined", False, 1e-8),
                                   ("jacobi", "fp32_refined", True, 1e-8)):
         sim = Simulation(m, 1e-3, 1e-3, device=gpu, rtol=rtol, precision=prec, velocity_jacobi=jac,
-                         pair_velocity=False)
+                         pair_velocity=pair)
         st = sim.step(10)
         out[form] = (st, sim.fields())
         sim.close()
