@@ -181,7 +181,7 @@ int nsfem_cg_solve(nsfem_device *dev, int slot, const nsfem_buffer *b,
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, stopping rule, results and kernels as nsfem_cg_solve;
  * every work vector, the grid-reduction state and the results live in one
- * static device array of the library (about 48.4 MiB, held by each GPU the
+ * static device array of the library (about 48.5 MiB, held by each GPU the
  * library runs on until the process ends).  Limit: rows * columns <=
  * 1,048,576 (1 << 20) in either precision (an FP32 + refinement solve keeps
  * room for its FP64 continuation); larger systems return
@@ -536,7 +536,7 @@ int nsfem_simulation_set_velocity_coarse_space(nsfem_simulation *sim, int coarse
                                                const int32_t *col, const double *val);
 /* Adds a level below the deepest level of the velocity hierarchy: P has one
  * row per node of the level above and `count` columns; the new level's
- * matrix is P^T A_above P (a level of at most 600 nodes is solved by its
+ * matrix is P^T A_above P (a level of at most 1,100 nodes is solved by its
  * dense inverse, else by CG to 1e-10).  No counterpart in the reference. */
 int nsfem_simulation_add_velocity_coarse_level(nsfem_simulation *sim, int count, int64_t nnz,
                                                const int32_t *row_start, const int32_t *col,

@@ -2354,8 +2354,9 @@ __device__ __forceinline__ void cg_body(const CgArgs &A, const int bid, const in
 // beta_{k+1} without a second reduction (Meurant's single-synchronisation
 // form of Hestenes-Stiefel CG, equal to it in exact arithmetic).  The state
 // of step k goes to the other buffer, so no block overwrites rows that
-// another still gathers.  (The FP64 solve keeps the two-phase iteration: its
-// packed state would need two gathers per nonzero, and measured slower.)
+// another still gathers.  (The streaming FP64 solve keeps the two-phase
+// iteration: its packed state would need two gathers per nonzero, and
+// measured slower.)
 __device__ __forceinline__ float next_r(float alpha, float r, float q) {
     return __builtin_fmaf(-alpha, q, r);
 }
@@ -3333,15 +3334,19 @@ __global__ __launch_bounds__(BS, BS / 256) void k_cg_p2(const CgArgs A) {
 // One exchange an iteration (the single-reduction iteration of the one-column
 // mixed solves, in FP64 too).  In the one-column mixed form every product,
 // sum and reduction has phase_f1g's order (wave tiles to waves, lanes to rows,
-// the same grid), so its iterates are that form's, bit for bit.
+// the same grid; blocks as the flat reduction adds them), so up to kFlatMax
+// blocks its iterates are that form's, bit for bit; past them the streaming
+// form adds the blocks' sums as a tree.
 //
-// Measured per iteration, streaming -> resident: 1,089 pressure rows in one
-// block, FP64 11.1 -> 2.2 us; 65,656 rows on 42 blocks, FP64 18.1 -> 4.5,
-// refined 12.4 -> 4.9 with its residual passes; 261,247 rows on 170 blocks,
-// FP64 25.9 -> 6.3, refined 20.8 -> 6.6; 261,241 P2 rows on 256 blocks, FP64
-// 55.9 -> 16.2, both columns refined 121 -> 50 (23 residual passes in 47
-// iterations).  Systems past the registers or the window (a million P2 rows,
-// the vertices-first node order of larger meshes) keep the streaming forms.
+// Measured per iteration, streaming -> resident, refined with the residual
+// passes: 1,089 pressure rows in one block, FP64 11.5 -> 2.2 us, refined 10.9
+// -> 3.2; 65,656 rows on 42 blocks 18.3 -> 4.6 and 12.5 -> 5.0; 261,247 rows
+// on 170 blocks 26.9 -> 6.5 and 21.6 -> 6.7; P2 mass matrices in lattice
+// order, 4,225 rows on 8 blocks, two columns, FP64 22.9 -> 10.4, refined (22
+// passes in 27 iterations) 48.0 -> 19.8; 261,241 rows on 256 blocks, one
+// column FP64 33.7 -> 15.6, two refined (23 passes in 47) 108 -> 42.8.
+// Systems past the registers or the window (a million P2 rows, the
+// vertices-first node order of larger meshes) keep the streaming forms.
 
 constexpr int kResWaves = 12;  // 3 waves a SIMD: 168 VGPRs each
 // Waves of a block of the refined one-column batch: those of the streaming
@@ -4017,7 +4022,12 @@ struct CgLaunch {
 
 // ---- resident solves
 // Most nonzeros of a row and most wave tiles of a wave of the resident
-// kernels: what 168 registers hold beside the solve's state.
+// kernels.  168 registers hold short rows and one tile of long ones in one
+// column; the kernels of two and three tiles of long rows and of two columns
+// spill 14 (two refined columns, one tile) to 310 registers and are still
+// ahead of the streaming forms, which read the matrix anew each iteration
+// (times above; two FP64 columns of 261,241 P2 rows, 300 spilled: 26.6 us an
+// iteration against 50.9).
 constexpr int kResRowShort = 8, kResRowLong = 20;
 constexpr int res_tiles(bool mixed, int w) { return w == kResRowShort ? 4 : mixed ? 3 : 2; }
 // Most LDS of a resident block (160 KB a CU; one block a CU).
@@ -4075,15 +4085,19 @@ int res_max_grid(Device &d, const void *kernel, int waves, size_t lds) {
     return std::min(per_cu * d.cu_count, kResMaxBlocks);
 }
 
-// Window rows and LDS of a matrix split over `grid` blocks; false when a
-// block's tiles, window or LDS go past what the kernel holds.
-// Wave tiles a wave that a solve's grid aims at.  Short rows (P1): two, as the
-// grid reductions grow with the blocks (resident, 65,656 rows: 4.5 us an
-// iteration on 42 or 64 blocks, 5.2 on 128, 6.3 on 256).  Long rows (P2): one,
-// as a tile's work and the residual passes outweigh them (65,657 rows, two
-// columns: FP64 19.1 us on 63 blocks, 13.9 on 128; refined 38.9 and 25.3).
+// Wave tiles a wave that a resident solve's grid aims at (the quotient is
+// rounded down, so some blocks give their waves one more: 65,656 rows come to
+// 42 blocks where the first grid without a third tile is 47).  Short rows
+// (P1): two, as the grid reductions grow with the blocks (65,656 rows, FP64
+// and refined: 4.6 and 5.0 us an iteration on 42 blocks, 4.5 and 4.7 on 47,
+// 4.4 and 4.5 on 64, 5.3 and 5.4 on 128, 6.3 and 6.3 on 256).  Long rows
+// (P2): one, as a tile's work and the residual passes outweigh them (16,597
+// rows, two columns, FP64 and refined: 15.7 and 26.9 us on 16 blocks, 12.7
+// and 21.7 on this rule's 31, 9.6 and 15.1 on 64, 12.1 and 18.0 on 256).
 int cg_tiles_per_wave(const Matrix &m) { return m.max_row_nz > kResRowShort ? 1 : 2; }
 
+// Window rows and LDS of a matrix split over `grid` blocks; false when a
+// block's tiles, window or LDS go past what the kernel holds.
 bool res_fits(const Matrix &m, int nc, bool mixed, int w, int waves, int grid, ResidentPlan &plan) {
     std::vector<int32_t> bt;
     split_tiles(m, grid, bt);

@@ -36,7 +36,7 @@ void simulation_reset(Simulation &s);
 
 // A-orthonormal basis X of past solutions of one matrix, with A X, for the
 // projection guess (a pressure solve, and the coarse solves of the coarse
-// correction); w, dx, guess: vectors of the matrix's size; s: dot results.
+// correction); w, dx, guess: vectors of the matrix's size.
 struct ProjBasis {
     int n = 0, dim = 0, max = 0;
     DeviceArray<double> x, ax, w, dx, guess;
