@@ -2589,14 +2589,6 @@ struct CgCtl {
     int k, last_ru, refines, ru, has_pend, out_of_iters, any;
 };
 
-// Status of a resident FP64 solve that left the range of its recurrence (no
-// public status is positive): x is as it was, and the streaming form, which
-// sums (r, r) itself, runs the solve.
-constexpr int kCgOutOfRange = 1;
-// Least (r, r), (q, q) and alpha^2, 2^-963 or 1.3e-290 (high word), whose
-// terms' underflow below 1e-307 is lost in rounding.
-constexpr int kCgLeastSum = 60 << 20;
-
 // After the set-up residual: acc[c] = (r, r) in FP64, acc[NC + c] = (b, b),
 // acc[2 NC + c] = (r, r) of the stored r.
 template <int NC>
@@ -2636,15 +2628,12 @@ __device__ void ctl_start(CgCtl<NC> &C, const CgArgs &A, const double (&acc)[3 *
 // rounding must not pile up over a steep fall); ru_gap iterations and the
 // iteration limit force one.  sums[4 c ...] = (p, q), (r, r), (r, q), (q, q).
 // MIXED = false (FP64): no updates; a column is done when its recursive
-// residual meets the tolerance, and all end as kCgOutOfRange where that
-// residual cannot be formed: (q, q) of a matrix near 1e-170 underflows and alpha^2
-// overflows, (q, q) of one near 1e150 overflows, while (r, r) and (p, q) are
-// in range.  (The test costs 0.4 to 0.8% of an FP64 solve.)
+// residual meets the tolerance.
 template <int NC, bool MIXED = true>
 __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&sums)[4 * NC]) {
     const int k = ++C.k;
     const double d2 = A.rdelta * A.rdelta;
-    bool want = false, any = false, out = false;
+    bool want = false, any = false;
     for (int c = 0; c < NC; ++c) {
         double alpha = 0.0, g = 0.0;
         bool dropped = false;
@@ -2658,16 +2647,9 @@ __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&su
                 alpha = gk / delta;
                 // gk - 2 alpha (r, q) + alpha^2 (q, q), its roundings spelt out:
                 // the same bits in every kernel this is inlined into
-                g = __builtin_fma(alpha * alpha, sums[4 * c + 3],
-                                  __builtin_fma(-2.0 * alpha, sums[4 * c + 2], gk));
-                if (!MIXED) {
-                    // (non-negative doubles compare as their high words)
-                    const int least = min(min(__double2hiint(gk), __double2hiint(sums[4 * c + 3])),
-                                          __double2hiint(alpha * alpha));
-                    out = out || (least < kCgLeastSum && gk != 0.0) ||
-                          (__double2hiint(g) & 0x7ff00000) == 0x7ff00000;  // infinite or NaN
-                }
-                g = fmax(g, 0.0);
+                g = fmax(__builtin_fma(alpha * alpha, sums[4 * c + 3],
+                                       __builtin_fma(-2.0 * alpha, sums[4 * c + 2], gk)),
+                         0.0);
                 C.gamma[c] = gk;
                 C.iters[c] = k;
                 if (MIXED) {
@@ -2686,12 +2668,6 @@ __device__ void ctl_after_phase(CgCtl<NC> &C, const CgArgs &A, const double (&su
         C.alpha[c] = alpha;
         C.g[c] = g;
         C.dropped[c] = dropped;
-    }
-    if (!MIXED && out) {
-        for (int c = 0; c < NC; ++c) {
-            C.active[c] = 0;
-            C.status[c] = kCgOutOfRange;
-        }
     }
     C.has_pend = 1;
     C.out_of_iters = k >= A.max_iter;
@@ -3427,7 +3403,41 @@ struct ResShared {
     double part[2][kMaxRed][NW];  // by epoch parity
     double sum[kMaxRed];
     int fail;
+    int range;  // FP64: a sum was past the recurrence's range
 };
+
+// Status of a resident FP64 solve that left the range of its recurrence (no
+// public status is positive): x is as it was, and the streaming form, which
+// sums (r, r) itself, runs the solve.
+constexpr int kCgOutOfRange = 1;
+// Least (r, r), (q, q) and alpha^2, 2^-963 or 1.3e-290 (high word), whose
+// terms' underflow below 1e-307 is lost in rounding.
+constexpr int kCgLeastSum = 60 << 20;
+
+// Whether the next (r, r) of an FP64 column cannot be formed from an
+// iteration's sums: (q, q) of a matrix near 1e-170 underflows and alpha^2
+// overflows, (q, q) of one near 1e150 overflows, while (r, r) and (p, q) are in
+// range.  The mark stays: whatever the recurrence does from there (converge
+// on a clamped 0, break down on an infinity), x is written only at the end.
+// A thread of its own tests while thread 0 steps the control state (on thread
+// 0's chain the test took 0.7 to 1.6% of a solve).
+template <int NC>
+__device__ __forceinline__ bool past_range(const double *sums) {
+    bool out = false;
+    for (int c = 0; c < NC; ++c) {
+        const double delta = sums[4 * c], gk = sums[4 * c + 1], qq = sums[4 * c + 3];
+        if (!(delta > 0.0) || gk == 0.0) continue;  // a breakdown, or done
+        const double alpha = gk / delta;
+        const double g = __builtin_fma(alpha * alpha, qq,
+                                       __builtin_fma(-2.0 * alpha, sums[4 * c + 2], gk));
+        // (non-negative doubles compare as their high words)
+        const int least = min(min(__double2hiint(gk), __double2hiint(qq)),
+                              __double2hiint(alpha * alpha));
+        out = out || least < kCgLeastSum ||
+              (__double2hiint(g) & 0x7ff00000) == 0x7ff00000;  // infinite or NaN
+    }
+    return out;
+}
 
 // The grid's sums of K values a thread, into S.sum, and a barrier over the
 // solve's blocks: every block's agent-scope stores before it are visible to
@@ -3581,7 +3591,7 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
     unsigned idx[R][(W + 1) / 2];
     Row r[R], q[R];
     VecN<NC, double> x[R];
-    if (t0) S.fail = 0;
+    if (t0) S.fail = S.range = 0;
     {
         Row zero;
 #pragma unroll
@@ -3741,6 +3751,7 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
                 ctl_after_phase<NC, MIXED>(C, A, sums);
                 if (!C.ru) ctl_end<NC>(C);
             }
+            if (!MIXED && tid == 64 && past_range<NC>(S.sum)) S.range = 1;
             __syncthreads();
             fresh = false;
             if constexpr (MIXED) {
@@ -3797,8 +3808,8 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             par ^= 1;
         }
     }
-    // (the same sums in every block, so the same status)
-    if (MIXED || C.status[0] != kCgOutOfRange) {
+    // (the same sums in every block, so the same mark)
+    if (MIXED || S.range == 0) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             if (row[j] < 0) continue;
@@ -3806,7 +3817,11 @@ __device__ __forceinline__ void cg_resident(const CgArgs &A, const int b, const 
             for (int c = 0; c < NC; ++c) A.x[(size_t)c * A.n + row[j]] = x[j].v[c];
         }
     }
-    if (writer) ctl_finish<NC>(C, A);
+    if (writer) {
+        ctl_finish<NC>(C, A);
+        if (!MIXED && S.range != 0)
+            for (int c = 0; c < NC; ++c) A.res[c].status = kCgOutOfRange;
+    }
     return;
 timeout:
     if (writer) {
@@ -4053,8 +4068,9 @@ const void *res_kernel_tiles(bool batch, int waves, int tiles) {
     if (tiles <= 1) return res_kernel<NC, MIXED, W, 1>(batch, waves);
     if (tiles == 2) return res_kernel<NC, MIXED, W, 2>(batch, waves);
     if constexpr (MIXED && W == kResRowShort) {
-        // 128 registers hold three tiles, not four (58 spilled): what two
-        // tiles a wave come to where the blocks do not divide them evenly
+        // 128 registers: three tiles spill 16, the next kernel's four 58;
+        // three is what two tiles a wave come to where the blocks do not
+        // divide them evenly
         if (waves == kResWavesBatch && tiles == 3)
             return (const void *)k_cg_res_batch<NC, MIXED, W, 3, kResWavesBatch>;
     }
