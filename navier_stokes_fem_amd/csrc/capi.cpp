@@ -24,6 +24,7 @@ void upload_csr(Device &d, Matrix &m, int rows, int cols, int64_t nnz, const int
     NSFEM_REQUIRE(rs && (nnz == 0 || (col && val)), NSFEM_INVALID_ARGUMENT, "null CSR array");
     NSFEM_REQUIRE(rs[0] == 0 && rs[rows] == nnz, NSFEM_INVALID_ARGUMENT,
                   "row_start must start at 0 and end at nnz");
+    RowShape shape;
     for (int r = 0; r < rows; ++r) {
         NSFEM_REQUIRE(rs[r] <= rs[r + 1], NSFEM_INVALID_ARGUMENT, "row_start must not decrease");
         for (int32_t k = rs[r]; k < rs[r + 1]; ++k) {
@@ -31,6 +32,11 @@ void upload_csr(Device &d, Matrix &m, int rows, int cols, int64_t nnz, const int
                           "column index out of range");
             NSFEM_REQUIRE(k == rs[r] || col[k - 1] < col[k], NSFEM_INVALID_ARGUMENT,
                           "columns must ascend strictly within a row");
+        }
+        if (rows == cols && rs[r] < rs[r + 1]) {
+            shape.max_nz = std::max(shape.max_nz, rs[r + 1] - rs[r]);
+            shape.lo = std::max(shape.lo, r - col[rs[r]]);
+            shape.hi = std::max(shape.hi, col[rs[r + 1] - 1] - r);
         }
     }
     std::lock_guard<std::mutex> lk(m.mtx);
@@ -60,7 +66,7 @@ void upload_csr(Device &d, Matrix &m, int rows, int cols, int64_t nnz, const int
         NSFEM_HIP(hipMemcpy(m.val.ptr, &zv, sizeof(double), hipMemcpyHostToDevice));
     }
     std::vector<int32_t> hrs(rs, rs + rows + 1);
-    build_tiles(m, hrs);
+    build_tiles(m, hrs, &shape);
     // the FP32 copy the refined solver streams, made here so that no solve
     // has to allocate it (the no-allocation entry point relies on it)
     if (rows == cols && nnz > 0) ensure_val32(d, m);

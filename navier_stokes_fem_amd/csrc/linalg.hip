@@ -223,7 +223,7 @@ __global__ void k_row_shape(int rows, const int32_t *__restrict__ rs,
     }
 }
 
-void row_shape(Matrix &m) {
+RowShape row_shape(const Matrix &m) {
     int h[3] = {0, 0, 0};
     if (m.rows == m.cols && m.nnz > 0) {
         DeviceArray<int> out;
@@ -234,13 +234,11 @@ void row_shape(Matrix &m) {
         NSFEM_HIP(hipGetLastError());
         NSFEM_HIP(hipMemcpy(h, out.ptr, sizeof(h), hipMemcpyDeviceToHost));
     }
-    m.max_row_nz = h[0];
-    m.band_lo = h[1];
-    m.band_hi = h[2];
+    return {h[0], h[1], h[2]};
 }
 }  // namespace
 
-void build_tiles(Matrix &m, const std::vector<int32_t> &rs) {
+void build_tiles(Matrix &m, const std::vector<int32_t> &rs, const RowShape *shape) {
     std::vector<int32_t> t = cut_rows(rs, m.rows, kTileRows, kSpmvTileNnz);
     m.n_tiles = (int)t.size() - 1;
     m.host_rs = rs;
@@ -251,7 +249,7 @@ void build_tiles(Matrix &m, const std::vector<int32_t> &rs) {
     NSFEM_HIP(hipMemcpy(m.tiles.ptr, meta.data(), meta.size() * sizeof(int4),
                         hipMemcpyHostToDevice));
     m.bcol_ok = col_delta(m, m.n_tiles, m.tiles.ptr, m.bcol);
-    row_shape(m);
+    m.shape = shape ? *shape : row_shape(m);
     build_wave_tiles(m, kWaveRows, kStageNnz);
 }
 
@@ -4110,7 +4108,7 @@ int res_max_grid(Device &d, const void *kernel, int waves, size_t lds) {
 // (P2): one, as a tile's work and the residual passes outweigh them (16,597
 // rows, two columns, FP64 and refined: 15.7 and 26.9 us on 16 blocks, 12.7
 // and 21.7 on this rule's 31, 9.6 and 15.1 on 64, 12.1 and 18.0 on 256).
-int cg_tiles_per_wave(const Matrix &m) { return m.max_row_nz > kResRowShort ? 1 : 2; }
+int cg_tiles_per_wave(const Matrix &m) { return m.shape.max_nz > kResRowShort ? 1 : 2; }
 
 // Window rows and LDS of a matrix split over `grid` blocks; false when a
 // block's tiles, window or LDS go past what the kernel holds.
@@ -4123,8 +4121,8 @@ bool res_fits(const Matrix &m, int nc, bool mixed, int w, int waves, int grid, R
         tiles = std::max(tiles, (bt[b + 1] - bt[b] + waves - 1) / waves);
         if (bt[b + 1] <= bt[b] || tiles > res_tiles(mixed, w)) return false;
         const int64_t r0 = m.host_wtiles[bt[b]], r1 = m.host_wtiles[bt[b + 1]];
-        const int64_t w0 = std::max<int64_t>(0, r0 - m.band_lo);
-        const int64_t w1 = std::min<int64_t>(m.rows, r1 + m.band_hi);
+        const int64_t w0 = std::max<int64_t>(0, r0 - m.shape.lo);
+        const int64_t w1 = std::min<int64_t>(m.rows, r1 + m.shape.hi);
         cap = std::max(cap, w1 - w0);
         halo = std::max(halo, (w1 - w0) - (r1 - r0));
     }
@@ -4146,8 +4144,8 @@ bool res_fits(const Matrix &m, int nc, bool mixed, int w, int waves, int grid, R
 // than it holds.
 ResidentPlan plan_resident(const Matrix &m, int nc, bool mixed, int want, int max_blocks) {
     ResidentPlan plan;
-    if (m.rows != m.cols || m.nnz <= 0 || m.max_row_nz > kResRowLong) return plan;
-    const int w = nc == 1 && m.max_row_nz <= kResRowShort ? kResRowShort : kResRowLong;
+    if (m.rows != m.cols || m.nnz <= 0 || m.shape.max_nz > kResRowLong) return plan;
+    const int w = nc == 1 && m.shape.max_nz <= kResRowShort ? kResRowShort : kResRowLong;
     const int most = std::min(std::min(max_blocks, kResMaxBlocks), m.n_wtiles);
     if (most < 1) return plan;
     if (want > 0) {
@@ -4417,8 +4415,8 @@ void cg_pass(Device &d, const CgRequest &req, bool mixed, CgPass &P,
     set_cg_params(d, req, n, a);
     a.sync = ws.sync;
     a.res = ws.res;
-    a.band_lo = m.band_lo;
-    a.band_hi = m.band_hi;
+    a.band_lo = m.shape.lo;
+    a.band_hi = m.shape.hi;
     a.win_cap = res.cap;
     const int ngroups = (grid + kGroup - 1) / kGroup;
 
@@ -4711,8 +4709,8 @@ std::vector<BatchLaunch> resident_launches(Device &d, const std::vector<CgReques
     int w = nc == 1 ? kResRowShort : kResRowLong;
     for (const CgRequest &r : reqs) {
         const Matrix &m = *r.m;
-        if (m.nnz <= 0 || m.max_row_nz > kResRowLong || m.n_wtiles < 1) return out;
-        if (m.max_row_nz > kResRowShort) w = kResRowLong;
+        if (m.nnz <= 0 || m.shape.max_nz > kResRowLong || m.n_wtiles < 1) return out;
+        if (m.shape.max_nz > kResRowShort) w = kResRowLong;
     }
     if (mixed && w == kResRowLong) return out;
     const int maxg = res_max_grid(d, res_kernel(nc, mixed, w, res_tiles(mixed, w), true), kResWaves,
@@ -4787,7 +4785,7 @@ bool batch_resident(Device &d, const std::vector<CgRequest> &reqs, BatchLaunch &
     size_t lds = 0;
     for (size_t k = 0; k < l.which.size(); ++k) {
         Matrix &m = *reqs[l.which[k]].m;
-        if (m.nnz <= 0 || m.max_row_nz > w || l.blocks[k] > kFlatMax) return false;
+        if (m.nnz <= 0 || m.shape.max_nz > w || l.blocks[k] > kFlatMax) return false;
         const ResidentPlan &plan = batch_plan(m, nc, mixed, w, kResWavesBatch, l.blocks[k]);
         if (!plan.ok) return false;
         cap.push_back(plan.cap);
@@ -4917,8 +4915,8 @@ int run_cg_batch(Device &d, const std::vector<CgRequest> &reqs, nsfem_cg_stats *
             a.sync = reinterpret_cast<SyncState *>(sm + i * sync_bytes);
             a.res = d.batch_res.ptr + 2 * i;
             a.nblocks = nb[i];
-            a.band_lo = m.band_lo;
-            a.band_hi = m.band_hi;
+            a.band_lo = m.shape.lo;
+            a.band_hi = m.shape.hi;
             a.win_cap = launch.cap[i];
             for (int k = 0; k < nb[i]; ++k) map.push_back(make_int2((int)i, k));
         }

@@ -121,6 +121,12 @@ struct ResidentPlan {
     int asked = 0;   // batches: the blocks (or the most of them) it was made for
 };
 
+// Square matrices: most nonzeros of a row, most columns below and above the
+// diagonal.
+struct RowShape {
+    int max_nz = 0, lo = 0, hi = 0;
+};
+
 struct Matrix {
     int rows = 0, cols = 0;
     int64_t nnz = 0;
@@ -137,9 +143,8 @@ struct Matrix {
     int wave_rows = kWaveRows, wave_nnz = kWaveNnz;  // current wave-tile shape
     int max_multirow_nz = 0;  // most nonzeros of a wave tile with more than one row
     std::vector<int32_t> host_wtiles;  // [n_wtiles + 1] first row of each wave tile
-    // square matrices: most nonzeros of a row, most columns below and above
-    // the diagonal, and the resident solves' plans by columns and precision
-    int max_row_nz = 0, band_lo = 0, band_hi = 0;
+    RowShape shape;
+    // the resident solves' plans by columns and precision
     ResidentPlan res_plan[4];
     // the batched ones by kernel (batch_kind): the fewest blocks the system
     // fits in, and the plan on the blocks of the last batch
@@ -288,7 +293,7 @@ struct Buffer {
 
 // ------------------------------------------------------------ entry points
 // (implemented in the .hip translation units, called by the C ABI layer)
-void build_tiles(Matrix &m, const std::vector<int32_t> &row_start);
+void build_tiles(Matrix &m, const std::vector<int32_t> &row_start, const RowShape *shape = nullptr);
 // Re-cut the rows into wave tiles of <= rows (<= 64) rows and <= nnz (<= 512)
 // nonzeros (the persistent CG's unit of work).
 void build_wave_tiles(Matrix &m, int rows, int nnz);
